@@ -49,6 +49,7 @@ extern "C" int lumen_ctx_create(int device, lumen_ctx **out) {
     lumen_warm_attn_oproj(c->stream);
     lumen_warm_elementwise(c->stream);
     lumen_warm_gemm(c->stream);
+    lumen_warm_gemm_f16x2(c->stream);
     lumen_warm_gemv(c->stream);
     lumen_warm_mlp_chain(c->stream);
     lumen_warm_prefill_attention(c->stream);

@@ -3,6 +3,7 @@
 #include "internal.h"
 #include "mixers.h"
 #include "wave_reduce.h"
+#include "f16_split.h"
 
 #include <cmath>
 
@@ -34,11 +35,13 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(const float *__restrict__ 
 
 // The same for rows of up to 1024 * VPT floats that are 16-byte aligned: a thread requests all of its
 // pieces of the row and of the gains at once (the scalar loop above takes a trip to memory per element
-// and pass) and keeps the row in registers between the two passes.
-template <int VPT>
+// and pass) and keeps the row in registers between the two passes.  SPLIT: the rows are left as f16 pairs (f16_split.h),
+// which a third pass over the registers makes.
+template <int VPT, bool SPLIT>
 __global__ __launch_bounds__(256) void rmsnorm_vec_kernel(const float *__restrict__ x, const float *__restrict__ w,
-                                                          float *__restrict__ out, int dim, float eps) {
+                                                          float *__restrict__ out, int dim, float eps, int *__restrict__ exps) {
     __shared__ float red[4];
+    __shared__ unsigned top[4];
     const float *xr = x + (size_t)blockIdx.x * dim;
     float *o = out + (size_t)blockIdx.x * dim;
     const int tid = threadIdx.x;
@@ -67,31 +70,55 @@ __global__ __launch_bounds__(256) void rmsnorm_vec_kernel(const float *__restric
     const float tot = (red[0] + red[1]) + (red[2] + red[3]);
     const float rms = sqrtf(tot / (float)dim + eps);
     const float inv = 1.0f / rms;
+    unsigned m = 0;
 #pragma unroll
     for (int i = 0; i < VPT; ++i) {
         const int k = (tid + i * 256) * 4;
-        if (k < dim) {
-            v4f r;
-            r.x = v[i].x * inv * g[i].x;
-            r.y = v[i].y * inv * g[i].y;
-            r.z = v[i].z * inv * g[i].z;
-            r.w = v[i].w * inv * g[i].w;
+        v4f r;
+        r.x = v[i].x * inv * g[i].x;
+        r.y = v[i].y * inv * g[i].y;
+        r.z = v[i].z * inv * g[i].z;
+        r.w = v[i].w * inv * g[i].w;
+        if (SPLIT) {  // (past the end: zeros)
+            v[i] = r;
+            m = max(m, magnitude_bits(r));
+        } else if (k < dim) {
             *(v4f *)(o + k) = r;
         }
     }
+    if (!SPLIT) return;
+    m = wave_umax(m);
+    if ((tid & 63) == 0) top[tid >> 6] = m;
+    __syncthreads();
+    const int e = row_exponent(max(max(top[0], top[1]), max(top[2], top[3])));
+    const float s = exp2_int(e);
+    if (tid == 0) exps[blockIdx.x] = e;
+#pragma unroll
+    for (int i = 0; i < VPT; ++i) {
+        const int k = (tid + i * 256) * 4;
+        if (k < dim) store_split4((uint16_t *)o, k, v[i], s);
+    }
 }
 
-int launch_rmsnorm(lumen_ctx *ctx, const float *x, const float *w, float *out, int rows, int dim, float eps) {
+int launch_rmsnorm(lumen_ctx *ctx, const float *x, const float *w, float *out, int rows, int dim, float eps, int *exps) {
     if (rows <= 0 || dim <= 0) return LUMEN_OK;
     const bool vec = dim % 4 == 0 && ((((uintptr_t)x | (uintptr_t)w | (uintptr_t)out) & 15) == 0);
+    if (vec && exps && dim % 16 == 0 && dim <= 4096) {
+        if (dim <= 2048)
+            hipLaunchKernelGGL((rmsnorm_vec_kernel<2, true>), dim3(rows), dim3(256), 0, ctx->stream, x, w, out, dim, eps, exps);
+        else
+            hipLaunchKernelGGL((rmsnorm_vec_kernel<4, true>), dim3(rows), dim3(256), 0, ctx->stream, x, w, out, dim, eps, exps);
+        LUMEN_CHECK_LAUNCH();
+        return LUMEN_OK;
+    }
     if (vec && dim <= 2048)
-        hipLaunchKernelGGL(rmsnorm_vec_kernel<2>, dim3(rows), dim3(256), 0, ctx->stream, x, w, out, dim, eps);
+        hipLaunchKernelGGL((rmsnorm_vec_kernel<2, false>), dim3(rows), dim3(256), 0, ctx->stream, x, w, out, dim, eps, nullptr);
     else if (vec && dim <= 4096)
-        hipLaunchKernelGGL(rmsnorm_vec_kernel<4>, dim3(rows), dim3(256), 0, ctx->stream, x, w, out, dim, eps);
+        hipLaunchKernelGGL((rmsnorm_vec_kernel<4, false>), dim3(rows), dim3(256), 0, ctx->stream, x, w, out, dim, eps, nullptr);
     else
         hipLaunchKernelGGL(rmsnorm_kernel, dim3(rows), dim3(256), 0, ctx->stream, x, w, out, dim, eps);
     LUMEN_CHECK_LAUNCH();
-    return LUMEN_OK;
+    return exps ? launch_split_rows(ctx, out, rows, dim, out, exps) : LUMEN_OK;
 }
 
 // -------------------------------------------------------------- elementwise

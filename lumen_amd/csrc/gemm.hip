@@ -22,6 +22,9 @@
 #include "internal.h"
 #include "wave_reduce.h"
 #include "stage_times.h"
+#include "f16_split.h"
+
+#include <algorithm>
 
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef float v16f __attribute__((ext_vector_type(16)));
@@ -817,11 +820,13 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(GemmArgs a, int splits
 // The same for whole rows, with the RMSNorm of the finished row on top: one workgroup per row of C (N <= 4096, a
 // multiple of 4); a thread keeps its pieces of the row in registers between the sum of squares and the scaling.
 // Splits are added in index order, the sum of squares in the order of rmsnorm_vec_kernel: same bits as the two
-// launches it replaces.
+// launches it replaces.  SPLIT: the normalised rows are left as f16 pairs (f16_split.h).
 #define GEMM_ROW_VPT 4
+template <bool SPLIT>
 __global__ __launch_bounds__(256) void gemm_reduce_norm_kernel(GemmArgs a, int splits) {
     typedef float v4 __attribute__((ext_vector_type(4)));
     __shared__ float red[4];
+    __shared__ unsigned top[4];
     const int row = blockIdx.x, tid = threadIdx.x, N = a.N;
     const size_t MN = (size_t)a.M * N, base = (size_t)row * N;
     v4 v[GEMM_ROW_VPT], g[GEMM_ROW_VPT];
@@ -858,17 +863,33 @@ __global__ __launch_bounds__(256) void gemm_reduce_norm_kernel(GemmArgs a, int s
     __syncthreads();
     const float tot = (red[0] + red[1]) + (red[2] + red[3]);
     const float inv = 1.0f / sqrtf(tot / (float)N + a.norm_eps);
+    unsigned m = 0;
 #pragma unroll
     for (int i = 0; i < GEMM_ROW_VPT; ++i) {
         const int k = (tid + i * 256) * 4;
-        if (k < N) {
-            v4 r;
-            r.x = v[i].x * inv * g[i].x;
-            r.y = v[i].y * inv * g[i].y;
-            r.z = v[i].z * inv * g[i].z;
-            r.w = v[i].w * inv * g[i].w;
+        v4 r;
+        r.x = v[i].x * inv * g[i].x;
+        r.y = v[i].y * inv * g[i].y;
+        r.z = v[i].z * inv * g[i].z;
+        r.w = v[i].w * inv * g[i].w;
+        if (SPLIT) {  // (past the end: zeros)
+            v[i] = r;
+            m = max(m, magnitude_bits(r));
+        } else if (k < N) {
             *(v4 *)(a.norm_out + base + k) = r;
         }
+    }
+    if (!SPLIT) return;
+    m = wave_umax(m);
+    if ((tid & 63) == 0) top[tid >> 6] = m;
+    __syncthreads();
+    const int e = row_exponent(max(max(top[0], top[1]), max(top[2], top[3])));
+    const float s = exp2_int(e);
+    if (tid == 0) a.norm_exp[row] = e;
+#pragma unroll
+    for (int i = 0; i < GEMM_ROW_VPT; ++i) {
+        const int k = (tid + i * 256) * 4;
+        if (k < N) store_split4((uint16_t *)(a.norm_out + base), k, v[i], s);
     }
 }
 
@@ -1005,6 +1026,7 @@ static int gemm_stream_splits(const lumen_ctx *ctx, const GemmArgs &a) {
     while (s > 1 && (size_t)s * a.M * a.N * sizeof(float) > ((size_t)256 << 20)) --s;
     return s < 1 ? 1 : (int)s;
 }
+bool gemm_takes_split(int M, int K, int w_bf16) { return M > gemm_stream_max_rows(w_bf16) && K > 0 && K % 64 == 0; }
 int gemm_reserve_workspace(lumen_ctx *ctx, size_t need) {
     if (ctx->gemm_ws_bytes >= need) return LUMEN_OK;
     HIP_TRY(hipStreamSynchronize(ctx->stream));
@@ -1017,13 +1039,17 @@ int gemm_reserve_workspace(lumen_ctx *ctx, size_t need) {
 }
 
 // bytes of partial tiles launch_gemm would want for this product (0: no K split)
-size_t gemm_workspace_bytes(const lumen_ctx *ctx, int M, int N, int K, int w_bf16) {
+size_t gemm_workspace_bytes(const lumen_ctx *ctx, int M, int N, int K, int w_bf16, bool split) {
     GemmArgs a = {};
     a.M = M; a.N = N; a.K = K; a.w_bf16 = w_bf16;
     if (M <= 0 || N <= 0 || K <= 0 || K % (w_bf16 ? 8 : 4)) return 0;
     if (M > GEMM_SKINNY_MAX_M && M <= gemm_stream_max_rows(w_bf16)) {  // (alignment is the caller's: assume the streaming kernel)
         const int st = gemm_stream_splits(ctx, a);
         return st > 1 ? (size_t)st * M * N * sizeof(float) : 0;
+    }
+    if (split && gemm_takes_split(M, K, w_bf16)) {  // (the larger of what the two ways to add the splits take)
+        const int sp = std::max(gemm_split_plan(ctx->num_cus, M, N, K, w_bf16, false).splits, gemm_split_plan(ctx->num_cus, M, N, K, w_bf16, true).splits);
+        return sp > 1 ? (size_t)sp * M * N * sizeof(float) : 0;
     }
     int splits = gemm_big_splits(ctx, a);
     if (splits <= 0) splits = gemm_splits(ctx, a);
@@ -1123,9 +1149,13 @@ int launch_gemm(lumen_ctx *ctx, const GemmArgs &a) {
     if (a.epi == EPI_SWIGLU && (a.N & 1)) LUMEN_FAIL(LUMEN_ERR_SHAPE, "SwiGLU epilogue needs an even column count, got %d", a.N);
     GemmArgs g = a;
     const bool stream = gemm_stream_applies(a);
-    int splits = stream ? 0 : gemm_big_splits(ctx, a);
-    const bool big = splits > 0;
+    const bool split = a.a_split && !stream && gemm_takes_split(a.M, a.K, a.w_bf16);
+    SplitPlan plan = {};
+    if (split) plan = gemm_split_plan(ctx->num_cus, a.M, a.N, a.K, a.w_bf16, a.keep_splits && a.splits_used && a.epi == EPI_STORE);
+    int splits = stream ? 0 : split ? plan.splits : gemm_big_splits(ctx, a);
+    const bool big = !split && splits > 0;
     if (stream) splits = gemm_stream_splits(ctx, a);
+    else if (split) {}
     else if (!big) splits = gemm_splits(ctx, a);
     if (splits > 1) {
         LUMEN_TRY(gemm_reserve_workspace(ctx, (size_t)splits * a.M * a.N * sizeof(float)));
@@ -1142,6 +1172,8 @@ int launch_gemm(lumen_ctx *ctx, const GemmArgs &a) {
         stage_times_report(ctx, "weight-streaming prompt product", (a.N + 15) / 16 * splits,
                            "start, [1] requests out, [2] first block done, [3] eighth block done, [4] blocks done, [5] after the "
                            "barrier, [6] stores acknowledged");
+    } else if (split) {
+        launch_gemm_f16x2(g, plan, ctx->stream);
     } else if (big) {
         dim3 bgrid((a.N + GB_N - 1) / GB_N, (a.M + GB_M - 1) / GB_M, splits);
         if (a.w_bf16) launch_gemm_tile<true, 4>(g, bgrid, ctx->stream);
@@ -1166,8 +1198,15 @@ int launch_gemm(lumen_ctx *ctx, const GemmArgs &a) {
     if (splits > 1) {
         if (want_norm && splits <= GEMM_MAX_SPLITS && a.N % 4 == 0 && a.N <= 256 * 4 * GEMM_ROW_VPT &&
             ((((uintptr_t)a.C | (uintptr_t)a.residual | (uintptr_t)g.part | (uintptr_t)a.norm_w | (uintptr_t)a.norm_out) & 15) == 0)) {
-            hipLaunchKernelGGL(gemm_reduce_norm_kernel, dim3(a.M), dim3(256), 0, ctx->stream, g, splits);
+            if (a.norm_exp && a.N % 16 == 0) {
+                hipLaunchKernelGGL(gemm_reduce_norm_kernel<true>, dim3(a.M), dim3(256), 0, ctx->stream, g, splits);
+            } else {
+                hipLaunchKernelGGL(gemm_reduce_norm_kernel<false>, dim3(a.M), dim3(256), 0, ctx->stream, g, splits);
+                if (a.norm_exp) LUMEN_TRY(launch_split_rows(ctx, a.norm_out, a.M, a.N, a.norm_out, a.norm_exp));
+            }
             norm_done = true;
+        } else if (a.epi == EPI_SWIGLU && a.c_exp) {
+            return launch_reduce_swiglu_split(ctx, g, splits);
         } else {
             size_t blocks = ((size_t)a.M * a.N + 255) / 256;
             if (blocks > (size_t)ctx->num_cus * 8) blocks = (size_t)ctx->num_cus * 8;
@@ -1175,7 +1214,8 @@ int launch_gemm(lumen_ctx *ctx, const GemmArgs &a) {
         }
         LUMEN_CHECK_LAUNCH();
     }
-    if (want_norm && !norm_done) LUMEN_TRY(launch_rmsnorm(ctx, a.C, a.norm_w, a.norm_out, a.M, a.N, a.norm_eps));
+    if (want_norm && !norm_done) LUMEN_TRY(launch_rmsnorm(ctx, a.C, a.norm_w, a.norm_out, a.M, a.N, a.norm_eps, a.norm_exp));
+    if (a.epi == EPI_SWIGLU && a.c_exp) return launch_split_rows(ctx, a.C, a.M, a.N / 2, a.C, a.c_exp);
     return LUMEN_OK;
 }
 

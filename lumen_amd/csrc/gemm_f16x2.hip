@@ -1,0 +1,409 @@
+// C[M,N] = A[M,K] W[N,K]^T at f32 accuracy on the f16 matrix cores, for the prompt passes of the models.
+//
+// gemm.hip takes an f32 product as six bf16 products of three-part values.  f16 has three bits more per part, so two parts
+// (f16_split.h) and three products -- hi hi, hi lo, lo hi -- carry 2^-22 of every product, and a bf16-stored weight is one
+// f16 value: two products.  Half (two thirds) of the matrix instructions, a third less LDS and split arithmetic.  f16's
+// range is what it costs: a row of either operand carries an exponent (A's is found by the kernel that makes A, W's once when a
+// weight is set), so only callers that know them take this path; the others keep gemm.hip.
+//
+// A arrives as split rows (f16_split.h); W is split on its way into LDS.
+//
+// What bounds it: the matrix pipes, whose clock the chip lowers under them (a library bf16 product of 8192^3 runs at 1.16 PFLOP/s here; this
+// kernel's 256 x 256 tiles issue 0.9 to 1.0), and with few rows the start of a launch and the partial products of K splits.
+// Useful TFLOP/s, before (three bf16 parts) and after, with the error against a float64 product (relative, over all elements):
+//   3968 x 11264 x 2048 f32   195 -> 297   6.8e-7 -> 4.9e-7      2048 x 8192 x 2048 bf16   318 -> 510   4.6e-7 -> 4.1e-7
+//   3968 x  2048 x 5632 f32   183 -> 302   8.1e-7 -> 5.7e-7       509 x 4096 x 11008 bf16  251 -> 360   5.7e-7 -> 4.8e-7
+//    512 x 11264 x 2048 f32   148 -> 204   5.0e-7 -> 3.4e-7       128 x 11264 x 2048 f32   125 -> 151   3.2e-7 -> 2.4e-7
+//     64 x   512 x   64 f32   (1 piece)    1.3e-7 -> 1.1e-7       300 x 1024 x  256 f32    (4 pieces)   1.8e-7 -> 1.5e-7
+// The error is smaller because half as many sums are rounded.
+#include "f16_split.h"
+
+typedef float v4f __attribute__((ext_vector_type(4)));
+typedef float v16f __attribute__((ext_vector_type(16)));
+typedef unsigned int v2u __attribute__((ext_vector_type(2)));
+typedef unsigned int v4u __attribute__((ext_vector_type(4)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+
+
+
+// In LDS a slice of 32 k is four planes of 8 k, [k / 8][row][8 f16] with two rows of padding: an operand read of 32 rows is 512
+// contiguous bytes, and a staging write of two rows' pieces (the planes start 32 bytes apart, modulo the banks) covers all banks once.
+template <int EPI, bool PARTIAL, int FI, int FJ>
+__device__ __forceinline__ void store_scaled_tiles(const GemmArgs &a, const v16f (&acc)[FI][FJ], const int *ae_tile, const int *we_tile, int bm, int bn,
+                                                   int wrow, int wcol, int lane) {
+    const int M = a.M, N = a.N;
+    float *part = PARTIAL ? a.part + (size_t)blockIdx.z * M * N : nullptr;
+    int we[FJ];
+#pragma unroll
+    for (int j = 0; j < FJ; ++j) we[j] = we_tile[wcol + j * 32 + (lane & 31)];
+#pragma unroll
+    for (int i = 0; i < FI; ++i)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int trow = wrow + i * 32 + (r >> 2) * 8 + (lane >> 5) * 4 + (r & 3), row = bm + trow;
+            const int ae = ae_tile[trow];
+#pragma unroll
+            for (int j = 0; j < FJ; ++j) {
+                const int col = bn + wcol + j * 32 + (lane & 31);
+                const float v = ldexpf(acc[i][j][r], -(ae + we[j]));
+                if (PARTIAL) {
+                    if (row < M && col < N) part[(size_t)row * N + col] = v;
+                } else if (EPI == EPI_SWIGLU) {
+                    const float up = __shfl_xor(v, 1, 64);
+                    if (!(col & 1) && row < M && col < N) a.C[(size_t)row * (N >> 1) + (col >> 1)] = v / (1.0f + expf(-v)) * up;
+                } else if (row < M && col < N) {
+                    const size_t o = (size_t)row * N + col;
+                    a.C[o] = (EPI == EPI_RESIDUAL) ? fmaf(a.alpha, v, a.residual[o]) : v;
+                }
+            }
+        }
+}
+
+// WM x WN wavefronts, FI x FJ tiles of 32 x 32 each; slices of HK of K in a ring of RING in LDS, D slices in flight from memory.  All operands of a
+// slice are in registers before its first matrix instruction, so that the barrier and the LDS reads after it cost no time
+// on the matrix pipe (operands read after the barrier: 260 instead of 297 TFLOP/s at 3968 x 11264 x 2048); every LDS access is
+// conflict-free (the counter reads 0).  bf16 weights: slices of 32, because a 16-deep one would read 32 bytes of a row.
+template <bool WBF16, int EPI, bool PARTIAL, int FI, int FJ, int WM, int WN, int DEPTH>
+__global__ __launch_bounds__(64 * WM * WN, (FI * FJ > 8 ? 1 : 2)) void gemm_f16x2_kernel(GemmArgs a) {
+    constexpr int T = 64 * WM * WN;
+    constexpr int HK = WBF16 ? 32 : 16, KS = HK / 16, RING = WBF16 ? 3 : 4;
+    constexpr int D = DEPTH;                          // slices in flight from memory
+    constexpr int PW = WBF16 ? 1 : 2;                 // f16 parts of a weight
+    constexpr int TM = 32 * FI * WM, TN = 32 * FJ * WN;
+    constexpr int AST = TM * HK / 4 / T;              // 16-byte pieces of A (both parts) per thread and slice
+    constexpr int WST = TN * HK / (WBF16 ? 8 : 4) / T;  // ... of W
+    constexpr int NPROD = WBF16 ? 2 : 3;
+    constexpr int APAD = WBF16 ? 1 : 2, WPAD = WBF16 ? 2 : 4;
+    constexpr int GROUPS = KS * FJ;                   // groups of FI NPROD matrix instructions of a slice
+    __shared__ __align__(16) uint16_t As[RING][KS][2][2][TM + APAD][8];   // [slot][k / 16][part][k half][row]
+    __shared__ __align__(16) uint16_t Ws[RING][PW][KS][2][TN + WPAD][8];
+    __shared__ int ae_tile[TM], we_tile[TN];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int wrow = wave / WN * (32 * FI), wcol = wave % WN * (32 * FJ);
+    const int bm = blockIdx.y * TM, bn = blockIdx.x * TN;
+    const int M = a.M, N = a.N, K = a.K;
+    // this workgroup's slices: whole pieces of 64 of K (the launcher's condition on K)
+    const int pieces = K / 64, per = (pieces + (int)gridDim.z - 1) / (int)gridDim.z;
+    const int p0 = min((int)blockIdx.z * per, pieces), s0 = p0 * (64 / HK), n = min(per, pieces - p0) * (64 / HK);
+
+    v16f acc[FI][FJ];
+#pragma unroll
+    for (int i = 0; i < FI; ++i)
+#pragma unroll
+        for (int j = 0; j < FJ; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+
+    // A piece i of this thread: row (tid + T i) / (HK / 4), piece (tid + T i) % (HK / 4) of the row's 4 HK bytes; f32 weights: row (tid + T i) / 4,
+    // k 4 * (tid % 4); bf16 weights: row (tid + T i) / 4, k 8 * (tid % 4).  Rows past the end are clamped (their products are never stored).
+    const char *abase = (const char *)a.a_split + ((size_t)bm * K + (size_t)s0 * HK) * 4;
+    const char *wbase = (const char *)a.W + ((size_t)bn * K + (size_t)s0 * HK) * (WBF16 ? 2 : 4);
+    unsigned aoff[AST], woff[WST];
+    float ws[WST];
+#pragma unroll
+    for (int i = 0; i < AST; ++i) {
+        const int idx = tid + i * T;
+        aoff[i] = (unsigned)(min(bm + idx / (HK / 4), M - 1) - bm) * (unsigned)K * 4u + (unsigned)(idx % (HK / 4)) * 16u;
+    }
+#pragma unroll
+    for (int i = 0; i < WST; ++i) {
+        const int row = min(bn + ((tid + i * T) >> 2), N - 1);
+        woff[i] = (unsigned)(row - bn) * (unsigned)K * (WBF16 ? 2u : 4u) + (unsigned)(tid & 3) * 16u;
+        ws[i] = exp2_int(a.w_exp[row]);
+    }
+    v4u va[D][AST], vw[D][WST];
+    auto fetch_a = [&](int r, int i, int s) { va[r][i] = *(const v4u *)(abase + (size_t)s * (HK * 4) + aoff[i]); };
+    auto fetch_w = [&](int r, int i, int s) { vw[r][i] = *(const v4u *)(wbase + (size_t)s * 64 + woff[i]); };
+    auto stage_a = [&](int r, int slot, int i) {
+        const int idx = tid + i * T, rem = idx % (HK / 4);
+        *(v4u *)&As[slot][rem >> 2][(rem >> 1) & 1][rem & 1][idx / (HK / 4)][0] = va[r][i];
+    };
+    auto stage_w = [&](int r, int slot, int i) {
+        const int row = (tid + i * T) >> 2;
+        if (WBF16) {
+            const unsigned src[4] = {vw[r][i].x, vw[r][i].y, vw[r][i].z, vw[r][i].w};
+            unsigned dst[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const f16x2_t h = {(_Float16)fmaf(__uint_as_float(src[e] << 16), ws[i], 0.f), (_Float16)fmaf(__uint_as_float(src[e] & 0xffff0000u), ws[i], 0.f)};
+                dst[e] = __builtin_bit_cast(unsigned, h);
+            }
+            *(v4u *)&Ws[slot][0][(tid & 3) >> 1][tid & 1][row][0] = v4u{dst[0], dst[1], dst[2], dst[3]};
+        } else {
+            unsigned h0, l0, h1, l1;
+            split_pair(__uint_as_float(vw[r][i].x), __uint_as_float(vw[r][i].y), ws[i], h0, l0);
+            split_pair(__uint_as_float(vw[r][i].z), __uint_as_float(vw[r][i].w), ws[i], h1, l1);
+            *(v2u *)&Ws[slot][0][0][(tid & 3) >> 1][row][(tid & 1) * 4] = v2u{h0, h1};
+            *(v2u *)&Ws[slot][PW - 1][0][(tid & 3) >> 1][row][(tid & 1) * 4] = v2u{l0, l1};
+        }
+    };
+    const int c = lane & 31, gk = lane >> 5;
+    f16x8 af[2][FI][2], wf[2][FJ][PW];  // operands of 16 k, two sets
+    auto read_a = [&](int set, int slot, int ks, int i) {
+#pragma unroll
+        for (int p = 0; p < 2; ++p) af[set][i][p] = __builtin_bit_cast(f16x8, *(const v4u *)&As[slot][ks][p][gk][wrow + i * 32 + c][0]);
+    };
+    auto read_w = [&](int set, int slot, int ks, int j) {
+#pragma unroll
+        for (int p = 0; p < PW; ++p) wf[set][j][p] = __builtin_bit_cast(f16x8, *(const v4u *)&Ws[slot][p][ks][gk][wcol + j * 32 + c][0]);
+    };
+    // Slice s is multiplied from registers; meanwhile its later operands and the first ones of slice s + 1 are read from LDS, slice s + 2 is staged
+    // (slot and values free since the barrier before the last) and slice s + 2 + D requested.  Nothing in it is conditional: past the end
+    // the last slice is requested again, staged and not used.
+    auto slice = [&](int set0, int r, int s, int slot, int slot1, int slot2) {
+        const int next = min(s + 2 + D, n - 1);
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            const int set = (set0 + ks) & 1;
+            const bool over = ks + 1 == KS;
+#pragma unroll
+            for (int j = 0; j < FJ; ++j) {
+                constexpr int PA_[3] = {1, 0, 0}, PW_[3] = {0, 1, 0};  // products by ascending size: lo hi, hi lo, hi hi (bf16 weights: lo w, hi w)
+#pragma unroll
+                for (int q = 0; q < NPROD; ++q)
+#pragma unroll
+                    for (int i = 0; i < FI; ++i)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[set][i][WBF16 ? 1 - q : PA_[q]], wf[set][j][WBF16 ? 0 : PW_[q]], acc[i][j], 0, 0, 0);
+                if (j < FI) read_a(set ^ 1, over ? slot1 : slot, over ? 0 : ks + 1, j);
+                read_w(set ^ 1, over ? slot1 : slot, over ? 0 : ks + 1, j);
+                const int g = ks * FJ + j;
+#pragma unroll
+                for (int i = 0; i < AST; ++i)
+                    if (i * GROUPS / AST == g) {
+                        stage_a(r, slot2, i);
+                        fetch_a(r, i, next);
+                    }
+#pragma unroll
+                for (int i = 0; i < WST; ++i)
+                    if (i * GROUPS / WST == g) {
+                        stage_w(r, slot2, i);
+                        fetch_w(r, i, next);
+                    }
+                if (FI == 4) {  // the group's order: everything else one by one in the shadows of its matrix instructions
+                    constexpr int NM = FI * NPROD, VPM = 24 / NM, NR = 2 + PW;
+#pragma unroll
+                    for (int k = 0; k < NM; ++k) {
+                        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);    // a matrix instruction,
+                        __builtin_amdgcn_sched_group_barrier(0x002, VPM, 0);  // vector ALU,
+                        if (k < NR) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);           // an LDS read,
+                        else if (k < NR + 3) __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);  // an LDS write
+                        else if (k < NR + 5) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);  // or a load
+                    }
+                }
+            }
+        }
+        __syncthreads();
+    };
+    static_assert(D % 2 == 0 && (64 / HK) % D == 0, "a piece of K is a whole number of turns of the register sets");
+    static_assert(FI <= FJ, "a group of matrix instructions per row tile whose operands are read under it");
+    for (int i = tid; i < TM; i += T) ae_tile[i] = a.a_exp[min(bm + i, M - 1)];
+    for (int i = tid; i < TN; i += T) we_tile[i] = a.w_exp[min(bn + i, N - 1)];
+    auto fetch = [&](int r, int s) {
+#pragma unroll
+        for (int i = 0; i < AST; ++i) fetch_a(r, i, min(s, n - 1));
+#pragma unroll
+        for (int i = 0; i < WST; ++i) fetch_w(r, i, min(s, n - 1));
+    };
+    auto stage = [&](int r, int slot) {
+#pragma unroll
+        for (int i = 0; i < AST; ++i) stage_a(r, slot, i);
+#pragma unroll
+        for (int i = 0; i < WST; ++i) stage_w(r, slot, i);
+    };
+    if (n > 0) {
+        // slice 2 + r of the rest goes through register set r % D; the first two through sets 0 and 1
+        fetch(0, 0);
+        fetch(1, 1);
+#pragma unroll
+        for (int r = 2; r < D; ++r) fetch(r, 2 + r);
+        stage(0, 0);
+        fetch(0, 2);
+        stage(1, 1);
+        fetch(1, 3);
+    }
+    __syncthreads();
+    if (n > 0) {
+#pragma unroll
+        for (int i = 0; i < FI; ++i) read_a(0, 0, 0, i);
+#pragma unroll
+        for (int j = 0; j < FJ; ++j) read_w(0, 0, 0, j);
+        int slot = 0;
+        auto after = [](int x) { return x + 1 == RING ? 0 : x + 1; };
+        for (int s = 0; s < n; s += D) {
+#pragma unroll
+            for (int r = 0; r < D; ++r) {
+                const int s1 = after(slot);
+                slice(KS == 1 ? r & 1 : 0, r, s + r, slot, s1, after(s1));
+                slot = s1;
+            }
+        }
+    }
+    store_scaled_tiles<EPI, PARTIAL, FI, FJ>(a, acc, ae_tile, we_tile, bm, bn, wrow, wcol, lane);
+}
+
+// ------------------------------------------------------------------------------------------ exponents, split rows
+// One wavefront per row of W.
+template <bool BF16>
+__global__ __launch_bounds__(256) void row_exponents_kernel(const void *W, int rows, int cols, int row0, int step, int *exps) {
+    const int r = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (r >= rows) return;
+    const size_t row = (size_t)row0 + (size_t)r * step;
+    unsigned m = 0;
+    for (int k = lane; k < cols; k += 64)
+        m = max(m, BF16 ? (unsigned)(((const uint16_t *)W)[row * cols + k] & 0x7fffu) << 16 : magnitude_bits(((const float *)W)[row * cols + k]));
+    m = wave_umax(m);
+    if (lane == 0) exps[row] = row_exponent(m);
+}
+
+// One workgroup per row, which is in registers before the first of it is stored (x and out may be the same).
+template <int VPT>
+__global__ __launch_bounds__(256) void split_rows_kernel(const float *x, int dim, float *out, int *exps) {
+    __shared__ unsigned top[4];
+    const int tid = threadIdx.x;
+    const size_t base = (size_t)blockIdx.x * dim;
+    v4f v[VPT];
+    unsigned m = 0;
+#pragma unroll
+    for (int i = 0; i < VPT; ++i) {
+        const int k = (tid + i * 256) * 4;
+        v[i] = v4f{0.f, 0.f, 0.f, 0.f};
+        if (k < dim) v[i] = *(const v4f *)(x + base + k);
+    }
+#pragma unroll
+    for (int i = 0; i < VPT; ++i) m = max(m, magnitude_bits(v[i]));
+    m = wave_umax(m);
+    if ((tid & 63) == 0) top[tid >> 6] = m;
+    __syncthreads();
+    const int e = row_exponent(max(max(top[0], top[1]), max(top[2], top[3])));
+    const float s = exp2_int(e);
+    if (tid == 0) exps[blockIdx.x] = e;
+#pragma unroll
+    for (int i = 0; i < VPT; ++i) {
+        const int k = (tid + i * 256) * 4;
+        if (k < dim) store_split4((uint16_t *)(out + base), k, v[i], s);
+    }
+}
+
+// Adds the K splits of a gate|up product in split order, applies silu(gate) * up and leaves the row split: one workgroup of 1024 per row
+// (a few hundred rows: what counts is that a thread has at most VPT trips to memory).
+template <int VPT>
+__global__ __launch_bounds__(1024) void reduce_swiglu_split_kernel(GemmArgs a, int splits) {
+    __shared__ unsigned top[16];
+    const int tid = threadIdx.x, I = a.N >> 1;
+    const size_t MN = (size_t)a.M * a.N, base = (size_t)blockIdx.x * a.N;
+    v4f v[VPT];
+    unsigned m = 0;
+#pragma unroll
+    for (int i = 0; i < VPT; ++i) {
+        const int k = (tid + i * 1024) * 4;  // of the I results; gate and up alternate in the product's columns
+        v[i] = v4f{0.f, 0.f, 0.f, 0.f};
+        if (k < I) {
+            v4f p0 = {0.f, 0.f, 0.f, 0.f}, p1 = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 8
+            for (int s = 0; s < splits; ++s) {
+                const float *src = a.part + (size_t)s * MN + base + 2 * k;
+                p0 += *(const v4f *)src;
+                p1 += *(const v4f *)(src + 4);
+            }
+            v[i] = v4f{p0.x / (1.0f + expf(-p0.x)) * p0.y, p0.z / (1.0f + expf(-p0.z)) * p0.w, p1.x / (1.0f + expf(-p1.x)) * p1.y,
+                       p1.z / (1.0f + expf(-p1.z)) * p1.w};
+            m = max(m, magnitude_bits(v[i]));
+        }
+    }
+    m = wave_umax(m);
+    if ((tid & 63) == 0) top[tid >> 6] = m;
+    __syncthreads();
+    m = 0;
+#pragma unroll
+    for (int w = 0; w < 16; ++w) m = max(m, top[w]);
+    const int e = row_exponent(m);
+    const float s = exp2_int(e);
+    if (tid == 0) a.c_exp[blockIdx.x] = e;
+#pragma unroll
+    for (int i = 0; i < VPT; ++i) {
+        const int k = (tid + i * 1024) * 4;
+        if (k < I) store_split4((uint16_t *)(a.C + (size_t)blockIdx.x * I), k, v[i], s);
+    }
+}
+
+int launch_row_exponents(lumen_ctx *ctx, const void *W, int w_bf16, int rows, int cols, int row0, int step, int *exps) {
+    if (rows <= 0) return LUMEN_OK;
+    if (w_bf16) hipLaunchKernelGGL(row_exponents_kernel<true>, dim3((rows + 3) / 4), dim3(256), 0, ctx->stream, W, rows, cols, row0, step, exps);
+    else hipLaunchKernelGGL(row_exponents_kernel<false>, dim3((rows + 3) / 4), dim3(256), 0, ctx->stream, W, rows, cols, row0, step, exps);
+    LUMEN_CHECK_LAUNCH();
+    return LUMEN_OK;
+}
+
+int launch_split_rows(lumen_ctx *ctx, const float *x, int rows, int dim, float *out, int *exps) {
+    if (rows <= 0) return LUMEN_OK;
+    if (dim % 16 || dim > 16384) LUMEN_FAIL(LUMEN_ERR_UNSUPPORTED, "split rows of %d", dim);
+    if (dim <= 2048) hipLaunchKernelGGL(split_rows_kernel<2>, dim3(rows), dim3(256), 0, ctx->stream, x, dim, out, exps);
+    else if (dim <= 6144) hipLaunchKernelGGL(split_rows_kernel<6>, dim3(rows), dim3(256), 0, ctx->stream, x, dim, out, exps);
+    else hipLaunchKernelGGL(split_rows_kernel<16>, dim3(rows), dim3(256), 0, ctx->stream, x, dim, out, exps);
+    LUMEN_CHECK_LAUNCH();
+    return LUMEN_OK;
+}
+
+int launch_reduce_swiglu_split(lumen_ctx *ctx, const GemmArgs &a, int splits) {
+    const int I = a.N / 2;
+    if (I % 16 || I > 16384) LUMEN_FAIL(LUMEN_ERR_UNSUPPORTED, "split rows of %d", I);
+    if (I <= 4096) hipLaunchKernelGGL(reduce_swiglu_split_kernel<1>, dim3(a.M), dim3(1024), 0, ctx->stream, a, splits);
+    else if (I <= 8192) hipLaunchKernelGGL(reduce_swiglu_split_kernel<2>, dim3(a.M), dim3(1024), 0, ctx->stream, a, splits);
+    else hipLaunchKernelGGL(reduce_swiglu_split_kernel<4>, dim3(a.M), dim3(1024), 0, ctx->stream, a, splits);
+    LUMEN_CHECK_LAUNCH();
+    return LUMEN_OK;
+}
+
+// Tile and K splits by what the busiest compute unit has to do, in microseconds measured on one MI355X (f32 / bf16 weights): a
+// 128 x 128 tile takes 1.5 / 1.15 per piece of 64 of K alone on its compute unit and 1.45 / 0.9 each beside others, a 256 x 256 tile 5.2 /
+// 3.1; a launch 7 / 8 besides; a K split 4 for the pass that adds the partial products and their bytes, written and read, at 9 TB/s (they stay
+// in the memory-side cache).  At most 16 splits (the passes that add them), 256 MiB of partial products.
+SplitPlan gemm_split_plan(int num_cus, int M, int N, int K, int w_bf16, bool sum_later) {
+    SplitPlan best = {false, 1};
+    double least = 0.0;
+    const long pieces = K / 64, cus = num_cus;
+    for (int big = 0; big < 2; ++big) {
+        const long t = big ? 256 : 128, tiles = ((N + t - 1) / t) * ((M + t - 1) / t);
+        for (long s = 1; s <= 16 && s <= pieces; ++s) {
+            const double bytes = (double)s * M * N * 4.0;
+            if (s > 1 && bytes > (double)((size_t)256 << 20)) break;
+            const long per_cu = (tiles * s + cus - 1) / cus, each = (pieces + s - 1) / s;
+            double us = (double)each * (double)per_cu * (big ? (w_bf16 ? 3.1 : 5.2) : per_cu == 1 ? (w_bf16 ? 1.15 : 1.5) : (w_bf16 ? 0.9 : 1.45));
+            us += big ? 8.0 : 7.0;
+            if (s > 1) us += (sum_later ? 0.0 : 4.0) + 2.0 * bytes / 9.0e6;
+            if ((big == 0 && s == 1) || us < least) {
+                least = us;
+                best.big = big != 0;
+                best.splits = (int)s;
+            }
+        }
+    }
+    return best;
+}
+
+template <bool BF16, int FI, int FJ, int DEPTH>
+static void launch_f16x2(const GemmArgs &a, dim3 grid, hipStream_t s) {
+    if (grid.z > 1) {
+        hipLaunchKernelGGL((gemm_f16x2_kernel<BF16, EPI_STORE, true, FI, FJ, 2, 2, DEPTH>), grid, dim3(256), 0, s, a);
+        return;
+    }
+    switch (a.epi) {
+        case EPI_STORE: hipLaunchKernelGGL((gemm_f16x2_kernel<BF16, EPI_STORE, false, FI, FJ, 2, 2, DEPTH>), grid, dim3(256), 0, s, a); break;
+        case EPI_RESIDUAL: hipLaunchKernelGGL((gemm_f16x2_kernel<BF16, EPI_RESIDUAL, false, FI, FJ, 2, 2, DEPTH>), grid, dim3(256), 0, s, a); break;
+        default: hipLaunchKernelGGL((gemm_f16x2_kernel<BF16, EPI_SWIGLU, false, FI, FJ, 2, 2, DEPTH>), grid, dim3(256), 0, s, a); break;
+    }
+}
+
+void launch_gemm_f16x2(const GemmArgs &a, const SplitPlan &p, hipStream_t s) {
+    const int t = p.big ? 256 : 128;
+    const dim3 grid((a.N + t - 1) / t, (a.M + t - 1) / t, p.splits);
+    if (p.big) {
+        if (a.w_bf16) launch_f16x2<true, 4, 4, 2>(a, grid, s);
+        else launch_f16x2<false, 4, 4, 2>(a, grid, s);
+    } else {
+        if (a.w_bf16) launch_f16x2<true, 2, 2, 2>(a, grid, s);
+        else launch_f16x2<false, 2, 2, 4>(a, grid, s);
+    }
+}
+
+LUMEN_DEFINE_WARM(gemm_f16x2)

@@ -208,7 +208,26 @@ struct GemmArgs {
     // consumer that adds them itself (in split order) and report how many there are; 1 = C holds the product
     int keep_splits;
     int *splits_used;
+    // optional: A as split rows with their exponents (f16_split.h), and the exponents of W's rows; where gemm_takes_split says that the
+    // product runs on them A itself is not read
+    const uint16_t *a_split;
+    const int *a_exp, *w_exp;
+    int *norm_exp;  // with norm_out, not null: the normalised rows are left split, in norm_out, with their exponents here
+    int *c_exp;     // with EPI_SWIGLU, not null: likewise the rows of C [M, N / 2]
 };
+// rows [dim] -> split rows at out (may be x itself) and exponents; dim a multiple of 16
+int launch_split_rows(lumen_ctx *ctx, const float *x, int rows, int dim, float *out, int *exps);
+// exponents of rows row0, row0 + step, ... of W [.., cols]
+int launch_row_exponents(lumen_ctx *ctx, const void *W, int w_bf16, int rows, int cols, int row0, int step, int *exps);
+// Does a product of M rows run on split rows where its caller has them?  (gemm_f16x2.hip; the few-row kernels read f32 rows)
+bool gemm_takes_split(int M, int K, int w_bf16);
+struct SplitPlan {
+    bool big;    // tiles of 256 x 256, else 128 x 128
+    int splits;  // of K
+};
+SplitPlan gemm_split_plan(int num_cus, int M, int N, int K, int w_bf16, bool sum_later);
+void launch_gemm_f16x2(const GemmArgs &a, const SplitPlan &p, hipStream_t s);
+int launch_reduce_swiglu_split(lumen_ctx *ctx, const GemmArgs &a, int splits);
 int launch_gemm(lumen_ctx *ctx, const GemmArgs &a);
 int launch_gemm_grouped(lumen_ctx *ctx, const GemmArgs &a, int max_tiles);  // M: total rows
 // act(gate, up) of a clamped expert
@@ -218,7 +237,7 @@ __device__ __forceinline__ float expert_act(float g, float u, float limit) {
     return g / (1.0f + expf(-1.702f * g)) * (u + 1.0f);
 }
 int gemm_reserve_workspace(lumen_ctx *ctx, size_t bytes);  // grows the split-K workspace (synchronises the stream when it does)
-size_t gemm_workspace_bytes(const lumen_ctx *ctx, int M, int N, int K, int w_bf16);
+size_t gemm_workspace_bytes(const lumen_ctx *ctx, int M, int N, int K, int w_bf16, bool split = false);
 
 // One empty kernel per translation unit with kernels.  The runtime loads a translation unit's device code at the first
 // launch of one of its kernels (milliseconds for the larger ones); lumen_ctx_create launches these so that the first
@@ -230,12 +249,14 @@ void lumen_warm_attention(hipStream_t s);
 void lumen_warm_attn_oproj(hipStream_t s);
 void lumen_warm_elementwise(hipStream_t s);
 void lumen_warm_gemm(hipStream_t s);
+void lumen_warm_gemm_f16x2(hipStream_t s);
 void lumen_warm_gemv(hipStream_t s);
 void lumen_warm_mlp_chain(hipStream_t s);
 void lumen_warm_prefill_attention(hipStream_t s);
 
 
-int launch_rmsnorm(lumen_ctx *ctx, const float *x, const float *w, float *out, int rows, int dim, float eps);
+// exps not null: the rows are left split (f16_split.h) with their exponents there
+int launch_rmsnorm(lumen_ctx *ctx, const float *x, const float *w, float *out, int rows, int dim, float eps, int *exps = nullptr);
 int launch_silu(lumen_ctx *ctx, const float *x, float *out, size_t n);
 int launch_add(lumen_ctx *ctx, const float *a, const float *b, float *out, size_t n);
 int launch_mul(lumen_ctx *ctx, const float *a, const float *b, float *out, size_t n);

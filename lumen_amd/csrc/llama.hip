@@ -18,6 +18,7 @@
 
 struct LayerW {
     void *wqkv = nullptr, *wo = nullptr, *wgu = nullptr, *wdown = nullptr;  // weight dtype
+    int *e_wqkv = nullptr, *e_wo = nullptr, *e_wgu = nullptr, *e_wdown = nullptr;  // exponents of their rows (f16_split.h)
     float *in_norm = nullptr, *post_norm = nullptr, *q_norm = nullptr, *k_norm = nullptr;
 };
 
@@ -33,6 +34,7 @@ struct lumen_llama {
     float *embed = nullptr;    // [V,H] f32 (bf16 sources are widened: same values)
     void *lm_head = nullptr;   // [V,H] weight dtype; aliases embed when tied and f32
     bool lm_head_owned = false;
+    int *e_head = nullptr;     // exponents of its rows
     float *final_norm = nullptr;
     std::vector<LayerW> layers;
     float *cos_dev = nullptr, *sin_dev = nullptr;
@@ -79,7 +81,7 @@ struct lumen_llama {
     int pf_cap = 0, pf_logit_cap = 0;
     float *p_x = nullptr, *p_h = nullptr, *p_n = nullptr, *p_qkv = nullptr, *p_qrot = nullptr, *p_attn = nullptr,
           *p_act = nullptr, *p_logits = nullptr;
-    int *p_ids = nullptr;
+    int *p_ids = nullptr, *p_exp = nullptr;  // (p_exp: exponents of p_n's, p_attn's and p_act's rows)
     std::vector<void *> allocs;
 };
 
@@ -111,7 +113,7 @@ extern "C" int lumen_llama_destroy(lumen_llama *m) {
     if (m->graph) hipGraphDestroy(m->graph);
     for (void *p : m->allocs) hipFree(p);
     hipFree(m->p_x); hipFree(m->p_h); hipFree(m->p_n); hipFree(m->p_qkv); hipFree(m->p_qrot);
-    hipFree(m->p_attn); hipFree(m->p_act); hipFree(m->p_logits); hipFree(m->p_ids);
+    hipFree(m->p_attn); hipFree(m->p_act); hipFree(m->p_logits); hipFree(m->p_ids); hipFree(m->p_exp);
     delete m;
     return LUMEN_OK;
 }
@@ -162,6 +164,7 @@ static int llama_create_impl(lumen_ctx *ctx, const lumen_llama_config *cfg, bool
         M_TRY(dmalloc_weight(m, &m->lm_head, (size_t)V * H * m->esz));
         m->lm_head_owned = true;
     }
+    M_TRY(dmalloc_weight(m, (void **)&m->e_head, (size_t)V * sizeof(int)));
     M_TRY(dmalloc_t(m, &m->final_norm, (size_t)H));
     M_TRY(fill_ones(m, m->final_norm, H));  // RMSNorm::new, rms_norm.rs:14-20
     for (int l = 0; l < L; ++l) {
@@ -170,6 +173,10 @@ static int llama_create_impl(lumen_ctx *ctx, const lumen_llama_config *cfg, bool
         M_TRY(dmalloc_weight(m, &w.wo, (size_t)H * m->qd * m->esz));
         M_TRY(dmalloc_weight(m, &w.wgu, (size_t)2 * I * H * m->esz));
         M_TRY(dmalloc_weight(m, &w.wdown, (size_t)H * I * m->esz));
+        M_TRY(dmalloc_weight(m, (void **)&w.e_wqkv, (size_t)m->qkvd * sizeof(int)));
+        M_TRY(dmalloc_weight(m, (void **)&w.e_wo, (size_t)H * sizeof(int)));
+        M_TRY(dmalloc_weight(m, (void **)&w.e_wgu, (size_t)2 * I * sizeof(int)));
+        M_TRY(dmalloc_weight(m, (void **)&w.e_wdown, (size_t)H * sizeof(int)));
         M_TRY(dmalloc_t(m, &w.in_norm, (size_t)H));
         M_TRY(dmalloc_t(m, &w.post_norm, (size_t)H));
         M_TRY(fill_ones(m, w.in_norm, H));
@@ -322,8 +329,9 @@ void bf16_to_f32_host(const uint16_t *src, float *dst, size_t n) {
 
 // Copies a [rows, cols] host matrix (src dtype) into device memory of dst dtype
 // whose row r lands at dst + (row0 + r*row_step) * cols.
+// exps not null: the exponents of the rows go there, by the rows' places in dst.
 static int upload_matrix(lumen_llama *m, void *dst, bool dst_bf16, const void *src, int src_dtype, size_t rows,
-                         size_t cols, size_t row0, size_t row_step) {
+                         size_t cols, size_t row0, size_t row_step, int *exps = nullptr) {
     const size_t dsz = dst_bf16 ? 2 : 4;
     const bool src_bf16 = src_dtype == LUMEN_DTYPE_BF16;
     const size_t chunk_rows = std::max<size_t>(1, (size_t)(64u << 20) / (cols * 4));
@@ -344,7 +352,7 @@ static int upload_matrix(lumen_llama *m, void *dst, bool dst_bf16, const void *s
                                  m->ctx->stream));
         HIP_TRY(hipStreamSynchronize(m->ctx->stream));
     }
-    return LUMEN_OK;
+    return exps ? launch_row_exponents(m->ctx, dst, dst_bf16, (int)rows, (int)cols, (int)row0, (int)row_step, exps) : LUMEN_OK;
 }
 
 static int want_shape(const char *name, const int64_t *shape, int ndim, int64_t a, int64_t b) {
@@ -366,14 +374,14 @@ extern "C" int lumen_llama_set_param(lumen_llama *m, const char *name, const voi
     const std::string n(name);
     if (n == "model.embed_tokens.weight") {
         LUMEN_TRY(want_shape(name, shape, ndim, V, H));
-        LUMEN_TRY(upload_matrix(m, m->embed, false, data, dtype, V, H, 0, 1));
-        if (c.tie_embeddings && m->lm_head_owned) return upload_matrix(m, m->lm_head, m->bf16, data, dtype, V, H, 0, 1);
+        LUMEN_TRY(upload_matrix(m, m->embed, false, data, dtype, V, H, 0, 1, c.tie_embeddings && !m->lm_head_owned ? m->e_head : nullptr));
+        if (c.tie_embeddings && m->lm_head_owned) return upload_matrix(m, m->lm_head, m->bf16, data, dtype, V, H, 0, 1, m->e_head);
         return LUMEN_OK;
     }
     if (n == "lm_head.weight") {
         LUMEN_TRY(want_shape(name, shape, ndim, V, H));
         if (c.tie_embeddings) LUMEN_FAIL(LUMEN_ERR_INVALID, "lm_head.weight given but embeddings are tied");
-        return upload_matrix(m, m->lm_head, m->bf16, data, dtype, V, H, 0, 1);
+        return upload_matrix(m, m->lm_head, m->bf16, data, dtype, V, H, 0, 1, m->e_head);
     }
     if (n == "model.norm.weight") {
         LUMEN_TRY(want_shape(name, shape, ndim, H, -1));
@@ -387,31 +395,31 @@ extern "C" int lumen_llama_set_param(lumen_llama *m, const char *name, const voi
     LayerW &w = m->layers[layer];
     if (rest == "self_attn.q_proj.weight") {
         LUMEN_TRY(want_shape(name, shape, ndim, m->qd, H));
-        return upload_matrix(m, w.wqkv, m->bf16, data, dtype, m->qd, H, 0, 1);
+        return upload_matrix(m, w.wqkv, m->bf16, data, dtype, m->qd, H, 0, 1, w.e_wqkv);
     }
     if (rest == "self_attn.k_proj.weight") {
         LUMEN_TRY(want_shape(name, shape, ndim, m->kvd, H));
-        return upload_matrix(m, w.wqkv, m->bf16, data, dtype, m->kvd, H, m->qd, 1);
+        return upload_matrix(m, w.wqkv, m->bf16, data, dtype, m->kvd, H, m->qd, 1, w.e_wqkv);
     }
     if (rest == "self_attn.v_proj.weight") {
         LUMEN_TRY(want_shape(name, shape, ndim, m->kvd, H));
-        return upload_matrix(m, w.wqkv, m->bf16, data, dtype, m->kvd, H, m->qd + m->kvd, 1);
+        return upload_matrix(m, w.wqkv, m->bf16, data, dtype, m->kvd, H, m->qd + m->kvd, 1, w.e_wqkv);
     }
     if (rest == "self_attn.o_proj.weight") {
         LUMEN_TRY(want_shape(name, shape, ndim, H, m->qd));
-        return upload_matrix(m, w.wo, m->bf16, data, dtype, H, m->qd, 0, 1);
+        return upload_matrix(m, w.wo, m->bf16, data, dtype, H, m->qd, 0, 1, w.e_wo);
     }
     if (rest == "mlp.gate_proj.weight") {  // row i -> fused row 2i
         LUMEN_TRY(want_shape(name, shape, ndim, I, H));
-        return upload_matrix(m, w.wgu, m->bf16, data, dtype, I, H, 0, 2);
+        return upload_matrix(m, w.wgu, m->bf16, data, dtype, I, H, 0, 2, w.e_wgu);
     }
     if (rest == "mlp.up_proj.weight") {  // row i -> fused row 2i+1
         LUMEN_TRY(want_shape(name, shape, ndim, I, H));
-        return upload_matrix(m, w.wgu, m->bf16, data, dtype, I, H, 1, 2);
+        return upload_matrix(m, w.wgu, m->bf16, data, dtype, I, H, 1, 2, w.e_wgu);
     }
     if (rest == "mlp.down_proj.weight") {
         LUMEN_TRY(want_shape(name, shape, ndim, H, I));
-        return upload_matrix(m, w.wdown, m->bf16, data, dtype, H, I, 0, 1);
+        return upload_matrix(m, w.wdown, m->bf16, data, dtype, H, I, 0, 1, w.e_wdown);
     }
     if (rest == "input_layernorm.weight") {
         LUMEN_TRY(want_shape(name, shape, ndim, H, -1));
@@ -772,14 +780,21 @@ static int ids_to_int(const lumen_llama *m, const float *ids, int s, std::vector
 }
 
 // ------------------------------------------------------------------ prefill
+// Do the four products of a prompt pass of s rows run on split rows (f16_split.h)?  All or none: what makes a product's input
+// leaves it split or not.
+static bool takes_split_rows(const lumen_llama *m, int s) {
+    return gemm_takes_split(s, m->cfg.hidden_size, m->bf16) && gemm_takes_split(s, m->qd, m->bf16) &&
+           gemm_takes_split(s, m->cfg.intermediate_size, m->bf16);
+}
+
 static int ensure_prefill_buffers(lumen_llama *m, int s, bool all_rows) {
     const lumen_llama_config &c = m->cfg;
     if (s > m->pf_cap) {
         HIP_TRY(hipStreamSynchronize(m->ctx->stream));
         hipFree(m->p_x); hipFree(m->p_h); hipFree(m->p_n); hipFree(m->p_qkv); hipFree(m->p_qrot);
-        hipFree(m->p_attn); hipFree(m->p_act); hipFree(m->p_ids);
+        hipFree(m->p_attn); hipFree(m->p_act); hipFree(m->p_ids); hipFree(m->p_exp);
         m->p_x = m->p_h = m->p_n = m->p_qkv = m->p_qrot = m->p_attn = m->p_act = nullptr;
-        m->p_ids = nullptr;
+        m->p_ids = m->p_exp = nullptr;
         m->pf_cap = 0;
         const size_t S = (size_t)s;
         HIP_TRY(hipMalloc((void **)&m->p_x, S * c.hidden_size * 4));
@@ -790,13 +805,15 @@ static int ensure_prefill_buffers(lumen_llama *m, int s, bool all_rows) {
         HIP_TRY(hipMalloc((void **)&m->p_attn, S * m->qd * 4));
         HIP_TRY(hipMalloc((void **)&m->p_act, S * c.intermediate_size * 4));
         HIP_TRY(hipMalloc((void **)&m->p_ids, S * sizeof(int)));
+        HIP_TRY(hipMalloc((void **)&m->p_exp, 3 * S * sizeof(int)));
         m->pf_cap = s;
         // the split-K workspace of the four products at this many rows, so that no launch has to grow it
         const int H = c.hidden_size, I = c.intermediate_size;
-        size_t ws = gemm_workspace_bytes(m->ctx, s, m->qkvd, H, m->bf16);
-        ws = std::max(ws, gemm_workspace_bytes(m->ctx, s, H, m->qd, m->bf16));
-        ws = std::max(ws, gemm_workspace_bytes(m->ctx, s, 2 * I, H, m->bf16));
-        ws = std::max(ws, gemm_workspace_bytes(m->ctx, s, H, I, m->bf16));
+        const bool split = takes_split_rows(m, s);
+        size_t ws = gemm_workspace_bytes(m->ctx, s, m->qkvd, H, m->bf16, split);
+        ws = std::max(ws, gemm_workspace_bytes(m->ctx, s, H, m->qd, m->bf16, split));
+        ws = std::max(ws, gemm_workspace_bytes(m->ctx, s, 2 * I, H, m->bf16, split));
+        ws = std::max(ws, gemm_workspace_bytes(m->ctx, s, H, I, m->bf16, split));
         if (ws) LUMEN_TRY(gemm_reserve_workspace(m->ctx, ws));
     }
     if (all_rows && s > m->pf_logit_cap) {
@@ -818,16 +835,23 @@ static int run_prefill(lumen_llama *m, const std::vector<int> &ids, float *logit
     LUMEN_TRY(ensure_prefill_buffers(m, s, all_rows != 0));
     HIP_TRY(hipMemcpyAsync(m->p_ids, ids.data(), sizeof(int) * s, hipMemcpyHostToDevice, ctx->stream));
     LUMEN_TRY(launch_embedding(ctx, m->embed, m->p_ids, s, H, V, m->p_x));
+    // split rows: p_n, p_attn and p_act hold f16 pairs in place of the f32 values their products read, their exponents are in p_exp
+    const bool split = takes_split_rows(m, s);
+    int *e_n = split ? m->p_exp : nullptr, *e_attn = split ? m->p_exp + s : nullptr, *e_act = split ? m->p_exp + 2 * (size_t)s : nullptr;
+    auto split_input = [&](GemmArgs &g, const int *a_exp, const int *w_exp) {
+        if (split) { g.a_split = (const uint16_t *)g.A; g.a_exp = a_exp; g.w_exp = w_exp; }
+    };
     for (int l = 0; l < c.num_hidden_layers; ++l) {
         const LayerW &w = m->layers[l];
         // (from the second layer on the down product of the layer before has left the normalised rows in p_n)
-        if (l == 0) LUMEN_TRY(launch_rmsnorm(ctx, m->p_x, w.in_norm, m->p_n, s, H, c.rms_norm_eps));
+        if (l == 0) LUMEN_TRY(launch_rmsnorm(ctx, m->p_x, w.in_norm, m->p_n, s, H, c.rms_norm_eps, e_n));
         GemmArgs g = {};
         g.A = m->p_n; g.W = w.wqkv; g.C = m->p_qkv; g.M = s; g.N = m->qkvd; g.K = H; g.w_bf16 = m->bf16; g.epi = EPI_STORE;
         // the RoPE pass adds the K splits of this product itself (one launch and one pass less)
         int qkv_splits = 1;
         g.keep_splits = m->qkvd % 4 == 0;
         g.splits_used = &qkv_splits;
+        split_input(g, e_n, w.e_wqkv);
         LUMEN_TRY(launch_gemm(ctx, g));
         const float *qkv = qkv_splits > 1 ? ctx->gemm_ws : m->p_qkv;
         AttnPrefillArgs a = {};
@@ -841,13 +865,18 @@ static int run_prefill(lumen_llama *m, const std::vector<int> &ids, float *logit
         a.scale = m->scale; a.causal = 1; a.q_norm_w = w.q_norm; a.k_norm_w = w.k_norm; a.norm_eps = c.rms_norm_eps;
         a.q_rot = m->p_qrot;
         LUMEN_TRY(launch_attn_prefill(ctx, a));
+        if (split) LUMEN_TRY(launch_split_rows(ctx, m->p_attn, s, m->qd, m->p_attn, e_attn));
         g = {};
         g.A = m->p_attn; g.W = w.wo; g.C = m->p_h; g.M = s; g.N = H; g.K = m->qd; g.w_bf16 = m->bf16;
         g.epi = EPI_RESIDUAL; g.residual = m->p_x;
         g.norm_w = w.post_norm; g.norm_out = m->p_n; g.norm_eps = c.rms_norm_eps;  // post_attention_layernorm rides along
+        g.norm_exp = e_n;
+        split_input(g, e_attn, w.e_wo);
         LUMEN_TRY(launch_gemm(ctx, g));
         g = {};
         g.A = m->p_n; g.W = w.wgu; g.C = m->p_act; g.M = s; g.N = 2 * I; g.K = H; g.w_bf16 = m->bf16; g.epi = EPI_SWIGLU;
+        g.c_exp = e_act;
+        split_input(g, e_n, w.e_wgu);
         LUMEN_TRY(launch_gemm(ctx, g));
         g = {};
         g.A = m->p_act; g.W = w.wdown; g.C = m->p_x; g.M = s; g.N = H; g.K = I; g.w_bf16 = m->bf16;
@@ -855,13 +884,16 @@ static int run_prefill(lumen_llama *m, const std::vector<int> &ids, float *logit
         // the next layer's input_layernorm -- or, where every row's logits are wanted, the final norm -- rides along
         if (l + 1 < c.num_hidden_layers) { g.norm_w = m->layers[l + 1].in_norm; g.norm_out = m->p_n; g.norm_eps = c.rms_norm_eps; }
         else if (all_rows) { g.norm_w = m->final_norm; g.norm_out = m->p_n; g.norm_eps = c.rms_norm_eps; }
+        g.norm_exp = e_n;
+        split_input(g, e_act, w.e_wdown);
         LUMEN_TRY(launch_gemm(ctx, g));
     }
     const int head_bf16 = (m->lm_head == (void *)m->embed) ? 0 : (int)m->bf16;
     if (all_rows) {  // what the reference computes, llama.rs:202-205 (the final norm came with the last down product)
-        if (c.num_hidden_layers == 0) LUMEN_TRY(launch_rmsnorm(ctx, m->p_x, m->final_norm, m->p_n, s, H, c.rms_norm_eps));
+        if (c.num_hidden_layers == 0) LUMEN_TRY(launch_rmsnorm(ctx, m->p_x, m->final_norm, m->p_n, s, H, c.rms_norm_eps, e_n));
         GemmArgs g = {};
         g.A = m->p_n; g.W = m->lm_head; g.C = m->p_logits; g.M = s; g.N = V; g.K = H; g.w_bf16 = head_bf16; g.epi = EPI_STORE;
+        split_input(g, e_n, m->e_head);
         LUMEN_TRY(launch_gemm(ctx, g));
         m->len += s;
         if (logits_host) LUMEN_TRY(lumen_download(ctx, logits_host, m->p_logits, sizeof(float) * (size_t)s * V));

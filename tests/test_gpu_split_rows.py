@@ -1,0 +1,94 @@
+"""GPU parity of the prompt products that run on f16 pairs (prompts of more than 32 rows, 16 with bf16-stored weights, inner sizes that
+are multiples of 64): row and column counts around the tiles' edges, one piece of K and many, rows of very different
+magnitudes, rows of zeros and rows that are not finite, against the CPU oracle.
+
+Tolerance: the suite's 1e-4 of the largest logit for f32 weights, and the same for bf16-stored ones, whose values the oracle
+holds too (the pairs carry 2^-22 of a product; sums of up to 3000 f32 terms 3e-7)."""
+import numpy as np
+import pytest
+
+from lumen_amd import synth
+from lumen_amd.models import LlamaModel
+from oracle import lumen_oracle as lo
+from tests.gpu_util import max_rel
+
+pytestmark = pytest.mark.gpu
+
+
+def config(hidden, inter, heads, kv_heads, layers=2, vocab=301, max_seq=320):
+    return dict(vocab_size=vocab, hidden_size=hidden, intermediate_size=inter, num_hidden_layers=layers, num_attention_heads=heads,
+                num_key_value_heads=kv_heads, rms_norm_eps=1e-5, max_seq_len=max_seq, rope_theta=10000.0)
+
+
+def build(cfg, bf16, change=None):
+    params = synth.make_params(cfg, seed=3, std=0.1, gains_one=False)
+    if change:
+        change(params, np.random.default_rng(7))
+    gcfg, bits = dict(cfg), {}
+    if bf16:
+        gcfg["weight_dtype"] = "bf16"
+        bits = {n: synth.bf16_round(a).reshape(a.shape) for n, a in params.items() if a.ndim == 2}
+        params = {n: synth.bf16_widen(bits[n]) if n in bits else a for n, a in params.items()}
+    gpu = LlamaModel(gcfg)
+    for n, a in params.items():
+        gpu.set_param(n, bits.get(n, a))
+    return gpu, lo.Llama(cfg, params)
+
+
+def magnitudes(params, rng):
+    """Tokens, and rows of the matrices that write the residual stream, spread over many powers of two; a row of zeros."""
+    for n, a in params.items():
+        if "embed" in n:
+            a *= np.exp2(rng.integers(-20, 20, (len(a), 1))).astype(np.float32)
+        elif "o_proj" in n or "down_proj" in n:
+            a *= np.exp2(rng.integers(-30, 6, (len(a), 1))).astype(np.float32)
+            a[5] = 0
+
+
+@pytest.mark.parametrize("bf16", [False, True], ids=["f32", "bf16"])
+@pytest.mark.parametrize("cfg,rows", [
+    (config(64, 64, 4, 2), (33, 64)),                  # one piece of K
+    (config(128, 192, 4, 1, vocab=257), (127, 128, 129)),
+    (config(320, 704, 5, 5), (255, 257, 300)),         # columns that fill no tile, several pieces, K splits
+    (config(1024, 2816, 16, 4, layers=1, max_seq=1152), (1101,)),  # large tiles
+], ids=["64", "128", "320", "1024"])
+def test_prompts_at_the_edges_of_tiles(cfg, rows, bf16):
+    gpu, ora = build(cfg, bf16)
+    for s in rows:
+        ids = synth.make_tokens(s, cfg["vocab_size"], seed=s)
+        gpu.reset_kv_caches()
+        ora.reset()
+        got = gpu.forward(ids, all_rows=True)
+        rc, ref = ora.forward(ids)
+        assert rc == lo.LO_OK
+        assert max_rel(got, ref) <= 1e-4
+        gpu.reset_kv_caches()
+        last = gpu.forward(ids, all_rows=False)
+        assert max_rel(last, ref[-1]) <= 1e-4
+
+
+@pytest.mark.parametrize("bf16", [False, True], ids=["f32", "bf16"])
+def test_rows_of_very_different_magnitudes(bf16):
+    cfg = config(192, 320, 6, 3)
+    gpu, ora = build(cfg, bf16, magnitudes)
+    ids = synth.make_tokens(150, cfg["vocab_size"], seed=1)
+    got = gpu.forward(ids, all_rows=True)
+    rc, ref = ora.forward(ids)
+    assert rc == lo.LO_OK
+    for t in range(len(ids)):  # every row by itself: rows of small logits have to be right too
+        assert max_rel(got[t], ref[t]) <= 1e-4, t
+
+
+def test_a_token_that_is_not_finite_stays_in_its_row():
+    cfg = config(128, 192, 4, 2)
+    for bad in (np.inf, np.nan):
+        def change(params, rng):
+            params["model.embed_tokens.weight"][7, 3] = bad
+        gpu, ora = build(cfg, False, change)
+        ids = synth.make_tokens(90, cfg["vocab_size"], seed=2)
+        ids[ids == 7] = 8
+        ids[-1] = 7  # (the last: no other token sees it)
+        got = gpu.forward(ids, all_rows=True)
+        _, ref = ora.forward(ids[:-1])
+        assert not np.isfinite(got[-1]).any()
+        assert max_rel(got[:-1], ref) <= 1e-4
