@@ -864,8 +864,9 @@ static int run_prefill(lumen_llama *m, const std::vector<int> &ids, float *logit
         a.q_stride = a.k_stride = a.v_stride = m->qkvd;
         a.scale = m->scale; a.causal = 1; a.q_norm_w = w.q_norm; a.k_norm_w = w.k_norm; a.norm_eps = c.rms_norm_eps;
         a.q_rot = m->p_qrot;
+        a.out_exp = attn_prefill_mfma_supported(a) ? e_attn : nullptr;
         LUMEN_TRY(launch_attn_prefill(ctx, a));
-        if (split) LUMEN_TRY(launch_split_rows(ctx, m->p_attn, s, m->qd, m->p_attn, e_attn));
+        if (split && !a.out_exp) LUMEN_TRY(launch_split_rows(ctx, m->p_attn, s, m->qd, m->p_attn, e_attn));
         g = {};
         g.A = m->p_attn; g.W = w.wo; g.C = m->p_h; g.M = s; g.N = H; g.K = m->qd; g.w_bf16 = m->bf16;
         g.epi = EPI_RESIDUAL; g.residual = m->p_x;

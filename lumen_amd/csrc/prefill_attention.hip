@@ -9,16 +9,17 @@
 // so scores never leave the compute unit and every K/V tile read from the
 // cache serves all n_rep heads of the group and 128 / n_rep positions at once.
 //
-// The products run on the bf16 matrix cores at f32 accuracy, as in the prompt-pass GEMM: an f32
-// value is the exact sum of three bf16 values, a product the sum of the six part products whose
-// orders add up to at most four, accumulated in f32 by v_mfma_f32_32x32x16_bf16 (for head_dim 64:
-// 24 + 24 instructions of 8 passes per key tile and wavefront; the f32 instruction would take
-// 32 + 32 of 16 passes).
+// The products run on the f16 matrix cores at f32 accuracy, as the prompt products of gemm_f16x2.hip do: every operand is the sum of two f16
+// values (f16_split.h), a product the three part products down to 2^-22, accumulated in f32 by v_mfma_f32_32x32x16_f16.  One
+// exponent serves the keys of a head and one its values (kv_range_kernel finds their largest magnitudes), every query has its own, a
+// softmax weight takes 2^14.  No output exceeds the largest value, so its exponent also serves the output rows where
+// the next product reads them split.
+// Bound by the matrix instructions and the softmax between them, which wait for each other within a wavefront; two per SIMD overlap.
+// With three bf16 parts: 420 us for 3968 positions of 32 heads of 64 (4 KV heads), with f16 pairs 286; 509 of 32 heads of 128: 61 -> 47.
 //
 // Per wavefront (32 rows) and key tile, everything transposed so that a lane owns one query row:
 //   S^T = K Q^T       K from LDS ([part][key][element], split on its way in) is the A operand, Q
-//                     (split once, in registers) the B operand; two accumulators take turns so
-//                     that consecutive instructions do not wait.  A lane then holds 16 of the
+//                     (split once, in registers) the B operand.  A lane then holds 16 of the
 //                     tile's 32 scores of ITS row, lane ^ 32 the other 16
 //   softmax           row max and sum in the lane (one exchange with lane ^ 32 for the max, one at
 //                     the very end for the sum); scores in log2 units (Q pre-multiplied by
@@ -28,6 +29,7 @@
 //                     trip through LDS; the rescale by alpha is a per-lane scalar
 #include "internal.h"
 #include "attn_device.h"
+#include "f16_split.h"
 
 typedef float v16f __attribute__((ext_vector_type(16)));
 
@@ -35,44 +37,72 @@ typedef float v16f __attribute__((ext_vector_type(16)));
 #define FA_KEYS 32   // keys per tile
 #define FA_THREADS 256
 
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+#define FA_CHUNKS 32  // parts a head's keys and values are searched in for their largest magnitude
+#define FA_P_EXP 14   // softmax weights are split as p 2^14
+
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef unsigned int v4u __attribute__((ext_vector_type(4)));
 typedef unsigned int v2u __attribute__((ext_vector_type(2)));
 
-__device__ __forceinline__ unsigned fa_pack_hi(float odd, float even) {
-    return __builtin_amdgcn_perm(__float_as_uint(odd), __float_as_uint(even), 0x07060302u);
+// x[0..3] s -> two parts of 4 f16 (2 dwords each)
+__device__ __forceinline__ void fa_split4(const v4f x, float s, v2u (&part)[2]) {
+    unsigned h0, l0, h1, l1;
+    split_pair(x.x, x.y, s, h0, l0);
+    split_pair(x.z, x.w, s, h1, l1);
+    part[0] = v2u{h0, h1};
+    part[1] = v2u{l0, l1};
 }
-// x[0..3] -> three parts of 4 bf16 (2 dwords each)
-__device__ __forceinline__ void fa_split4(const v4f x, v2u (&part)[3]) {
-    float r[4] = {x.x, x.y, x.z, x.w};
+
+// Largest finite magnitude (bits) of each part of the L cached keys, and values, of a KV head: range [2][b hkv][FA_CHUNKS]
+__global__ __launch_bounds__(256) void kv_range_kernel(const float *k, const float *v, int max_seq, int d, int L, unsigned *range) {
+    __shared__ unsigned top[2][4];
+    const int tid = threadIdx.x, head = blockIdx.y;
+    const size_t base = (size_t)head * max_seq * d;
+    const int per = (L + FA_CHUNKS - 1) / FA_CHUNKS;
+    const size_t at = (size_t)min((int)blockIdx.x * per, L) * d, end = (size_t)min(((int)blockIdx.x + 1) * per, L) * d;
+    unsigned m[2] = {0u, 0u};
+    for (size_t i = at + tid * 4; i < end; i += 1024) {
+        const v4f x[2] = {*(const v4f *)(k + base + i), *(const v4f *)(v + base + i)};
 #pragma unroll
-    for (int p = 0; p < 3; ++p) {
-        part[p].x = fa_pack_hi(r[1], r[0]);
-        part[p].y = fa_pack_hi(r[3], r[2]);
-        if (p < 2) {
+        for (int w = 0; w < 2; ++w)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) r[e] -= __uint_as_float(__float_as_uint(r[e]) & 0xffff0000u);
-        }
+            for (int e = 0; e < 4; ++e) {
+                const unsigned u = magnitude_bits(x[w][e]);
+                m[w] = max(m[w], u < 0x7f800000u ? u : 0u);
+            }
     }
+#pragma unroll
+    for (int w = 0; w < 2; ++w) {
+        m[w] = wave_umax(m[w]);
+        if ((tid & 63) == 0) top[w][tid >> 6] = m[w];
+    }
+    __syncthreads();
+    if (tid < 2) range[((size_t)tid * gridDim.y + head) * FA_CHUNKS + blockIdx.x] = max(max(top[tid][0], top[tid][1]), max(top[tid][2], top[tid][3]));
 }
+
 // KT: key tiles of 32 per trip of the loop (2 for head_dim 64: one barrier pair, one row maximum and one rescale of
 // O per 64 keys; 1 for head_dim 128, whose K and V tiles fill LDS twice as fast).
 template <int D, int NREP, int KT>
-__global__ __launch_bounds__(FA_THREADS, (D == 64 ? 2 : 1)) void attn_prefill_bf16x3_kernel(AttnPrefillArgs a) {
+__global__ __launch_bounds__(FA_THREADS, 2) void attn_prefill_f16x2_kernel(AttnPrefillArgs a) {
     constexpr int BQ = FA_ROWS / NREP;  // positions per workgroup
     constexpr int KEYS = FA_KEYS * KT;   // keys per trip
     constexpr int DT = D / 32;          // 32-wide tiles of the head dimension
     constexpr int PIECES = D * KEYS / 4 / FA_THREADS;  // 16-byte pieces of a K (or V) tile per thread
     // rows of 4 words more than a multiple of 32: the 16-byte reads of 8 neighbouring rows hit distinct banks
     constexpr int LDK = D + 8, LDV = KEYS + 8;
-    __shared__ __align__(16) uint16_t Ks[3][KEYS][LDK];  // [part][key][element]
-    __shared__ __align__(16) uint16_t Vt[3][D][LDV];        // [part][element][key position]
+    __shared__ __align__(16) uint16_t Ks[2][KEYS][LDK];  // [part][key][element]
+    __shared__ __align__(16) uint16_t Vt[2][D][LDV];        // [part][element][key position]
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int c = lane & 31, half = lane >> 5;
     // workgroups are dealt in index order: the blocks of late positions (most keys) go first
     const int q0 = (int)(gridDim.x - 1 - blockIdx.x) * BQ, hk = blockIdx.y, bb = blockIdx.z;
     const int L = a.past_len + a.s;
+    // exponents of this head's keys and values; of all heads' values, which no output exceeds
+    const unsigned *kr = a.kv_range + ((size_t)bb * a.hkv + hk / a.kv_div) * FA_CHUNKS, *vr = kr + (size_t)gridDim.z * a.hkv * FA_CHUNKS;
+    const unsigned k_top = wave_umax(kr[c]), v_top = wave_umax(vr[c]);
+    const int ek = row_exponent(k_top), ev = row_exponent(v_top);
+    const float k_scale = exp2_int(ek), v_scale = exp2_int(ev);
     const size_t head_base = ((size_t)bb * a.hkv + hk / a.kv_div) * a.max_seq * D;  // kv_div > 1: grid row = query head
     const float *Kc = a.k_cache + head_base, *Vc = a.v_cache + head_base;
 
@@ -83,18 +113,31 @@ __global__ __launch_bounds__(FA_THREADS, (D == 64 ? 2 : 1)) void attn_prefill_bf
     const float *qrow = a.q_rot + (((size_t)bb * a.s + my_i) * a.hq + (size_t)hk * NREP + my_row % NREP) * D;
     const float qf_scale = a.scale * LUMEN_LOG2E;
     // Q as the B operand of S^T = K Q^T: lane (column c, half g) holds elements ks * 16 + g * 8 .. + 7 of its row
-    v4u qp[D / 16][3];
+    v4u qp[D / 16][2];
+    float s_unit;  // what an accumulated score is to be multiplied by
+    {
+        v4f x[D / 16][2];
+        unsigned m = 0;
 #pragma unroll
-    for (int ks = 0; ks < D / 16; ++ks) {
-        v2u lo[3], hi[3];
-        v4f x = *(const v4f *)(qrow + ks * 16 + half * 8);
-        x.x *= qf_scale; x.y *= qf_scale; x.z *= qf_scale; x.w *= qf_scale;
-        fa_split4(x, lo);
-        x = *(const v4f *)(qrow + ks * 16 + half * 8 + 4);
-        x.x *= qf_scale; x.y *= qf_scale; x.z *= qf_scale; x.w *= qf_scale;
-        fa_split4(x, hi);
+        for (int ks = 0; ks < D / 16; ++ks)
 #pragma unroll
-        for (int p = 0; p < 3; ++p) qp[ks][p] = (v4u){lo[p].x, lo[p].y, hi[p].x, hi[p].y};
+            for (int h = 0; h < 2; ++h) {
+                x[ks][h] = *(const v4f *)(qrow + ks * 16 + half * 8 + h * 4);
+                x[ks][h].x *= qf_scale; x[ks][h].y *= qf_scale; x[ks][h].z *= qf_scale; x[ks][h].w *= qf_scale;
+                m = max(m, magnitude_bits(x[ks][h]));
+            }
+        m = max(m, (unsigned)__shfl_xor((int)m, 32, 64));
+        const int eq = row_exponent(m);
+        const float q_scale = exp2_int(eq);
+        s_unit = ldexpf(1.0f, -(ek + eq));
+#pragma unroll
+        for (int ks = 0; ks < D / 16; ++ks) {
+            v2u lo[2], hi[2];
+            fa_split4(x[ks][0], q_scale, lo);
+            fa_split4(x[ks][1], q_scale, hi);
+#pragma unroll
+            for (int p = 0; p < 2; ++p) qp[ks][p] = (v4u){lo[p].x, lo[p].y, hi[p].x, hi[p].y};
+        }
     }
 
     const int q_last = min(q0 + BQ, a.s) - 1;
@@ -110,7 +153,7 @@ __global__ __launch_bounds__(FA_THREADS, (D == 64 ? 2 : 1)) void attn_prefill_bf
     for (int t = 0; t < DT; ++t)
 #pragma unroll
         for (int r = 0; r < 16; ++r) O[t][r] = 0.f;
-    float m_run = -INFINITY, l_run = 0.f;  // of this lane's row; l over this lane's half of the keys
+    float m_run = -INFINITY, l_run = 0.f;  // of this lane's row; l, times 2^14, over this lane's half of the keys
 
     // V^T is staged with bits 2 and 3 of the key index exchanged: the 8 keys a lane holds of S^T (4 + 4,
     // eight apart) then sit next to each other for the 16-byte operand read.  A thread takes 4 elements
@@ -132,52 +175,48 @@ __global__ __launch_bounds__(FA_THREADS, (D == 64 ? 2 : 1)) void attn_prefill_bf
         }
     };
 
-    constexpr int PA_[6] = {2, 0, 1, 1, 0, 0}, PB_[6] = {0, 2, 1, 0, 1, 0};  // part products by ascending size
+    constexpr int PA_[3] = {1, 0, 0}, PB_[3] = {0, 1, 0};  // part products by ascending size: lo hi, hi lo, hi hi
     if (kmax > 0) fetch(0);
     for (int j0 = 0; j0 < kmax; j0 += KEYS) {
 #pragma unroll
         for (int p = 0; p < PIECES; ++p) {
             const int idx = tid + p * FA_THREADS;
             const int key = idx / (D / 4), k4 = (idx % (D / 4)) * 4;
-            v2u kp[3];
-            fa_split4(kreg[p], kp);
+            v2u kp[2];
+            fa_split4(kreg[p], k_scale, kp);
 #pragma unroll
-            for (int q = 0; q < 3; ++q) *(v2u *)&Ks[q][key][k4] = kp[q];
+            for (int q = 0; q < 2; ++q) *(v2u *)&Ks[q][key][k4] = kp[q];
         }
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            v2u vp[3];
-            fa_split4((v4f){vreg[0][e], vreg[1][e], vreg[2][e], vreg[3][e]}, vp);
+            v2u vp[2];
+            fa_split4((v4f){vreg[0][e], vreg[1][e], vreg[2][e], vreg[3][e]}, v_scale, vp);
 #pragma unroll
-            for (int q = 0; q < 3; ++q) *(v2u *)&Vt[q][v_k4 + e][4 * v_g] = vp[q];
+            for (int q = 0; q < 2; ++q) *(v2u *)&Vt[q][v_k4 + e][4 * v_g] = vp[q];
         }
         __syncthreads();
         if (j0 + KEYS < kmax) fetch(j0 + KEYS);  // in flight during the matrix instructions below
 
         if (j0 < wave_kmax) {  // uniform per wavefront: tiles wholly above the causal diagonal are skipped
             // S^T = K Q^T: register r of tile kt holds key 32 kt + 8 (r / 4) + 4 half + r % 4 against this lane's row
-            v16f Sa[KT], Sb[KT];
+            v16f S[KT];
 #pragma unroll
             for (int kt = 0; kt < KT; ++kt)
 #pragma unroll
-                for (int r = 0; r < 16; ++r) Sa[kt][r] = Sb[kt][r] = 0.f;
+                for (int r = 0; r < 16; ++r) S[kt][r] = 0.f;
 #pragma unroll
             for (int ks = 0; ks < D / 16; ++ks) {
-                bf16x8 qf[3];
+                f16x8 kf[KT][2];
 #pragma unroll
-                for (int p = 0; p < 3; ++p) qf[p] = __builtin_bit_cast(bf16x8, qp[ks][p]);
+                for (int kt = 0; kt < KT; ++kt)
 #pragma unroll
-                for (int kt = 0; kt < KT; ++kt) {
-                    bf16x8 kf[3];
+                    for (int p = 0; p < 2; ++p)
+                        kf[kt][p] = __builtin_bit_cast(f16x8, *(const v4u *)&Ks[p][32 * kt + c][ks * 16 + half * 8]);
 #pragma unroll
-                    for (int p = 0; p < 3; ++p)
-                        kf[p] = __builtin_bit_cast(bf16x8, *(const v4u *)&Ks[p][32 * kt + c][ks * 16 + half * 8]);
+                for (int q = 0; q < 3; ++q)
 #pragma unroll
-                    for (int q = 0; q < 6; q += 2) {
-                        Sa[kt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[PA_[q]], qf[PB_[q]], Sa[kt], 0, 0, 0);
-                        Sb[kt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[PA_[q + 1]], qf[PB_[q + 1]], Sb[kt], 0, 0, 0);
-                    }
-                }
+                    for (int kt = 0; kt < KT; ++kt)
+                        S[kt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[kt][PA_[q]], __builtin_bit_cast(f16x8, qp[ks][PB_[q]]), S[kt], 0, 0, 0);
             }
 
             // softmax of this lane's row, in the lane: half of the trip's keys here, half in lane ^ 32
@@ -188,7 +227,7 @@ __global__ __launch_bounds__(FA_THREADS, (D == 64 ? 2 : 1)) void attn_prefill_bf
                 for (int kt = 0; kt < KT; ++kt)
 #pragma unroll
                     for (int r = 0; r < 16; ++r) {
-                        sc[16 * kt + r] = Sa[kt][r] + Sb[kt][r];
+                        sc[16 * kt + r] = S[kt][r] * s_unit;
                         m_tile = fmaxf(m_tile, sc[16 * kt + r]);
                     }
             } else {
@@ -198,7 +237,7 @@ __global__ __launch_bounds__(FA_THREADS, (D == 64 ? 2 : 1)) void attn_prefill_bf
                     for (int r = 0; r < 16; ++r) {
                         const int j = j0 + 32 * kt + 8 * (r >> 2) + 4 * half + (r & 3);
                         const bool valid = j < L && (!a.causal || j <= my_pos);
-                        sc[16 * kt + r] = valid ? Sa[kt][r] + Sb[kt][r] : -INFINITY;
+                        sc[16 * kt + r] = valid ? S[kt][r] * s_unit : -INFINITY;
                         m_tile = fmaxf(m_tile, sc[16 * kt + r]);
                     }
             }
@@ -210,7 +249,7 @@ __global__ __launch_bounds__(FA_THREADS, (D == 64 ? 2 : 1)) void attn_prefill_bf
             float psum = 0.f;
 #pragma unroll
             for (int r = 0; r < 16 * KT; ++r) {
-                sc[r] = fast_exp2(sc[r] - m_ref);
+                sc[r] = fast_exp2(sc[r] - (m_ref - FA_P_EXP));
                 psum += sc[r];
             }
             l_run = fmaf(l_run, alpha, psum);
@@ -223,51 +262,77 @@ __global__ __launch_bounds__(FA_THREADS, (D == 64 ? 2 : 1)) void attn_prefill_bf
             // (registers 8 ks .. 8 ks + 7 are the keys at positions 16 ks + 8 half .. + 7 of V^T)
 #pragma unroll
             for (int ks = 0; ks < KEYS / 16; ++ks) {
-                bf16x8 pf[3];
+                f16x8 pf[2];
                 {
-                    v2u lo[3], hi[3];
-                    fa_split4((v4f){sc[8 * ks], sc[8 * ks + 1], sc[8 * ks + 2], sc[8 * ks + 3]}, lo);
-                    fa_split4((v4f){sc[8 * ks + 4], sc[8 * ks + 5], sc[8 * ks + 6], sc[8 * ks + 7]}, hi);
+                    v2u lo[2], hi[2];
+                    fa_split4((v4f){sc[8 * ks], sc[8 * ks + 1], sc[8 * ks + 2], sc[8 * ks + 3]}, 1.0f, lo);
+                    fa_split4((v4f){sc[8 * ks + 4], sc[8 * ks + 5], sc[8 * ks + 6], sc[8 * ks + 7]}, 1.0f, hi);
 #pragma unroll
-                    for (int p = 0; p < 3; ++p) pf[p] = __builtin_bit_cast(bf16x8, (v4u){lo[p].x, lo[p].y, hi[p].x, hi[p].y});
+                    for (int p = 0; p < 2; ++p) pf[p] = __builtin_bit_cast(f16x8, (v4u){lo[p].x, lo[p].y, hi[p].x, hi[p].y});
                 }
-                bf16x8 vf[DT][3];
+                f16x8 vf[DT][2];
 #pragma unroll
                 for (int t = 0; t < DT; ++t)
 #pragma unroll
-                    for (int p = 0; p < 3; ++p)
-                        vf[t][p] = __builtin_bit_cast(bf16x8, *(const v4u *)&Vt[p][32 * t + c][ks * 16 + half * 8]);
+                    for (int p = 0; p < 2; ++p)
+                        vf[t][p] = __builtin_bit_cast(f16x8, *(const v4u *)&Vt[p][32 * t + c][ks * 16 + half * 8]);
 #pragma unroll
-                for (int q = 0; q < 6; ++q)
+                for (int q = 0; q < 3; ++q)
 #pragma unroll
                     for (int t = 0; t < DT; ++t)
-                        O[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[t][PA_[q]], pf[PB_[q]], O[t], 0, 0, 0);
+                        O[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[t][PA_[q]], pf[PB_[q]], O[t], 0, 0, 0);
             }
         }
         __syncthreads();
     }
 
     // out = ctx / (sum + 1e-9), self_attention.rs:670-676; [B,S,Hq,D]
-    const float inv = 1.0f / ((l_run + __shfl_xor(l_run, 32, 64)) + 1e-9f);
+    const float inv = 1.0f / fmaf(l_run + __shfl_xor(l_run, 32, 64), exp2_int(-FA_P_EXP), 1e-9f);
+    const float v_unit = ldexpf(1.0f, -(ev + FA_P_EXP));
     const int i = q0 + my_row / NREP;
+    float o_scale = 0.f;
+    if (a.out_exp) {  // (uniform) the rows go out split, all with the exponent of the largest value there is
+        const unsigned *all = a.kv_range + ((size_t)gridDim.z + bb) * a.hkv * FA_CHUNKS;
+        unsigned m = 0;
+        for (int n = lane; n < a.hkv * FA_CHUNKS; n += 64) m = max(m, all[n]);
+        const int eo = row_exponent(wave_umax(m));
+        o_scale = exp2_int(eo);
+        if (hk == 0 && my_row % NREP == 0 && half == 0 && i < a.s) a.out_exp[(size_t)bb * a.s + i] = eo;
+    }
     if (i < a.s) {
-        float *o = a.out + (((size_t)bb * a.s + i) * a.hq + (size_t)hk * NREP + my_row % NREP) * D;
+        const size_t head = (size_t)hk * NREP + my_row % NREP;
+        float *row = a.out + ((size_t)bb * a.s + i) * a.hq * D;
 #pragma unroll
         for (int t = 0; t < DT; ++t)
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
-                v4f v = {O[t][4 * g] * inv, O[t][4 * g + 1] * inv, O[t][4 * g + 2] * inv, O[t][4 * g + 3] * inv};
-                *(v4f *)(o + 32 * t + 8 * g + 4 * half) = v;
+                const v4f v = {O[t][4 * g] * inv * v_unit, O[t][4 * g + 1] * inv * v_unit, O[t][4 * g + 2] * inv * v_unit, O[t][4 * g + 3] * inv * v_unit};
+                const int at = (int)head * D + 32 * t + 8 * g + 4 * half;
+                if (a.out_exp) store_split4((uint16_t *)row, at, v, o_scale);
+                else *(v4f *)(row + at) = v;
             }
     }
 }
 
 template <int D>
-static int launch_fa_d(lumen_ctx *ctx, const AttnPrefillArgs &a) {
+static int launch_fa_d(lumen_ctx *ctx, const AttnPrefillArgs &a_in) {
+    AttnPrefillArgs a = a_in;
     const int nrep = a.hq / a.hkv;
+    const size_t need = 2 * (size_t)a.b * a.hkv * FA_CHUNKS * sizeof(unsigned);
+    if (need > ctx->kv_range_bytes) {
+        HIP_TRY(hipStreamSynchronize(ctx->stream));
+        hipFree(ctx->kv_range);
+        ctx->kv_range = nullptr;
+        ctx->kv_range_bytes = 0;
+        HIP_TRY(hipMalloc((void **)&ctx->kv_range, need));
+        ctx->kv_range_bytes = need;
+    }
+    a.kv_range = ctx->kv_range;
+    hipLaunchKernelGGL(kv_range_kernel, dim3(FA_CHUNKS, a.b * a.hkv), dim3(256), 0, ctx->stream, a.k_cache, a.v_cache, a.max_seq, D, a.past_len + a.s,
+                       ctx->kv_range);
     dim3 block(FA_THREADS);
 #define LAUNCH_FA(NR)                                                                                    \
-    hipLaunchKernelGGL((attn_prefill_bf16x3_kernel<D, NR, (D == 64 ? 2 : 1)>), dim3((a.s + FA_ROWS / NR - 1) / (FA_ROWS / NR), a.hkv, a.b), \
+    hipLaunchKernelGGL((attn_prefill_f16x2_kernel<D, NR, (D == 64 ? 2 : 1)>), dim3((a.s + FA_ROWS / NR - 1) / (FA_ROWS / NR), a.hkv, a.b), \
                        block, 0, ctx->stream, a)
     switch (nrep) {
         case 1: LAUNCH_FA(1); break;
@@ -277,7 +342,7 @@ static int launch_fa_d(lumen_ctx *ctx, const AttnPrefillArgs &a) {
         default: {  // any other group size: one query head per grid row, its KV head = head / n_rep
             AttnPrefillArgs b = a;
             b.kv_div = nrep;
-            hipLaunchKernelGGL((attn_prefill_bf16x3_kernel<D, 1, (D == 64 ? 2 : 1)>), dim3((a.s + FA_ROWS - 1) / FA_ROWS, a.hq, a.b), block, 0,
+            hipLaunchKernelGGL((attn_prefill_f16x2_kernel<D, 1, (D == 64 ? 2 : 1)>), dim3((a.s + FA_ROWS - 1) / FA_ROWS, a.hq, a.b), block, 0,
                                ctx->stream, b);
         }
     }

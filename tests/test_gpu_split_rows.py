@@ -8,9 +8,11 @@ import numpy as np
 import pytest
 
 from lumen_amd import synth
+from lumen_amd.layers import KVCacheInner, RotaryEmbedding
 from lumen_amd.models import LlamaModel
 from oracle import lumen_oracle as lo
 from tests.gpu_util import max_rel
+from tests.test_gpu_attention import gpu_prefill
 
 pytestmark = pytest.mark.gpu
 
@@ -50,8 +52,9 @@ def magnitudes(params, rng):
     (config(64, 64, 4, 2), (33, 64)),                  # one piece of K
     (config(128, 192, 4, 1, vocab=257), (127, 128, 129)),
     (config(320, 704, 5, 5), (255, 257, 300)),         # columns that fill no tile, several pieces, K splits
+    (config(256, 320, 2, 1), (96, 161)),               # heads of 128
     (config(1024, 2816, 16, 4, layers=1, max_seq=1152), (1101,)),  # large tiles
-], ids=["64", "128", "320", "1024"])
+], ids=["64", "128", "320", "256", "1024"])
 def test_prompts_at_the_edges_of_tiles(cfg, rows, bf16):
     gpu, ora = build(cfg, bf16)
     for s in rows:
@@ -92,3 +95,26 @@ def test_a_token_that_is_not_finite_stays_in_its_row():
         _, ref = ora.forward(ids[:-1])
         assert not np.isfinite(got[-1]).any()
         assert max_rel(got[:-1], ref) <= 1e-4
+
+
+@pytest.mark.parametrize("d,h,h_kv,s,past", [(64, 8, 1, 96, 0), (64, 6, 2, 129, 70), (128, 4, 4, 97, 0), (128, 4, 2, 200, 33), (64, 2, 2, 127, 1)])
+@pytest.mark.parametrize("q_exp,k_exp,v_exp", [(0, 0, 0), (-90, 88, -100), (60, -61, 90)])
+def test_prompt_attention_over_magnitudes(d, h, h_kv, s, past, q_exp, k_exp, v_exp):
+    """Queries, keys and values far from 1, and keys and values spread over 2^8 within a head (2e-5 of the largest output, the suite's bound for
+    attention: scores of a few units, so that a relative error of 2^-22 of the terms of a score moves a weight by 1e-6)."""
+    rng = np.random.default_rng(s + d)
+
+    def draw(n, heads, e):
+        spread = np.exp2(rng.uniform(-8, 0, (1, n, heads, 1)))
+        return (rng.normal(0, 1, (1, n, heads, d)) * spread * 2.0 ** e).astype(np.float32)
+    rope, scale = RotaryEmbedding(d, 512, 10000.0), d ** -0.5 * 4.0
+    cos, sin = lo.rope_table(d, 512, 10000.0)
+    gpu, ora = KVCacheInner(1, h_kv, 512, d), lo.KVCache(1, h_kv, 512, d)
+    for n in (past, s):
+        if not n:
+            continue
+        q, k, v = draw(n, h, q_exp), draw(n, h_kv, k_exp), draw(n, h_kv, v_exp)
+        got = gpu_prefill(gpu, rope, q, k, v, scale)
+        rc, ref = lo.attn_prefill(ora, q, k, v, cos, sin, scale)
+        assert rc == lo.LO_OK
+    assert max_rel(got * 2.0 ** -v_exp, ref * 2.0 ** -v_exp) <= 2e-5
