@@ -327,10 +327,12 @@ __global__ __launch_bounds__(256) void polynorm_kernel(const float *z, const flo
 }
 
 // The same for 16-byte aligned rows of up to 4096 VPT elements: read once, kept in registers between the two passes.
-template <int VPT>
+// SPLIT: the rows are left as f16 pairs (f16_split.h), which saves the product a pass over them.
+template <int VPT, bool SPLIT>
 __global__ __launch_bounds__(1024) void polynorm_vec_kernel(const float *z, const float *__restrict__ coef, float *out, int dim,
-                                                            int stride, float eps) {
+                                                            int stride, float eps, int *__restrict__ exps) {
     __shared__ float red[3][16];
+    __shared__ unsigned top[16];
     const float *zr = z + (size_t)blockIdx.x * stride;
     float *o = out + (size_t)blockIdx.x * stride;
     const int tid = threadIdx.x, nt = blockDim.x, nw = nt >> 6;
@@ -371,33 +373,59 @@ __global__ __launch_bounds__(1024) void polynorm_vec_kernel(const float *z, cons
     }
     const float n = (float)dim;
     const float a1 = coef[0] / sqrtf(s1 / n + eps), a2 = coef[1] / sqrtf(s2 / n + eps), a3 = coef[2] / sqrtf(s3 / n + eps), c3 = coef[3];
+    unsigned m = 0;
 #pragma unroll
     for (int i = 0; i < VPT; ++i) {
         const int k = (tid + i * nt) * 4;
-        if (k < stride) {
-            v4f r;
+        v4f r;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) r[e] = k + e < dim ? fmaf(fmaf(fmaf(a3, v[i][e], a2), v[i][e], a1), v[i][e], c3) : 0.f;
+        for (int e = 0; e < 4; ++e) r[e] = k + e < dim ? fmaf(fmaf(fmaf(a3, v[i][e], a2), v[i][e], a1), v[i][e], c3) : 0.f;
+        if (SPLIT) {
+            v[i] = r;
+            m = max(m, magnitude_bits(r));
+        } else if (k < stride) {
             *(v4f *)(o + k) = r;
         }
     }
+    if (!SPLIT) return;
+    m = wave_umax(m);
+    if ((tid & 63) == 0) top[tid >> 6] = m;
+    __syncthreads();
+    m = 0;
+    for (int w = 0; w < nw; ++w) m = max(m, top[w]);
+    const int e = row_exponent(m);
+    const float s = exp2_int(e);
+    if (tid == 0) exps[blockIdx.x] = e;
+#pragma unroll
+    for (int i = 0; i < VPT; ++i) {
+        const int k = (tid + i * nt) * 4;
+        if (k < stride) store_split4((uint16_t *)o, k, v[i], s);
+    }
 }
 
-int launch_polynorm(lumen_ctx *ctx, const float *z, const float *coef, float *out, int rows, int dim, int stride, float eps) {
+template <bool SPLIT>
+static void launch_polynorm_vec(lumen_ctx *ctx, const float *z, const float *coef, float *out, int rows, int dim, int stride, float eps, int *exps) {
+    const int pieces = stride / 4, threads = pieces <= 256 ? 256 : pieces <= 512 ? 512 : 1024;
+    if (pieces <= threads)
+        hipLaunchKernelGGL((polynorm_vec_kernel<1, SPLIT>), dim3(rows), dim3(threads), 0, ctx->stream, z, coef, out, dim, stride, eps, exps);
+    else if (pieces <= 2 * threads)
+        hipLaunchKernelGGL((polynorm_vec_kernel<2, SPLIT>), dim3(rows), dim3(threads), 0, ctx->stream, z, coef, out, dim, stride, eps, exps);
+    else
+        hipLaunchKernelGGL((polynorm_vec_kernel<4, SPLIT>), dim3(rows), dim3(threads), 0, ctx->stream, z, coef, out, dim, stride, eps, exps);
+}
+
+int launch_polynorm(lumen_ctx *ctx, const float *z, const float *coef, float *out, int rows, int dim, int stride, float eps, int *exps) {
     if (rows <= 0 || dim <= 0) return LUMEN_OK;
-    if (stride % 4 == 0 && stride <= 16384 && (((uintptr_t)z | (uintptr_t)out) & 15) == 0) {
-        const int pieces = stride / 4, threads = pieces <= 256 ? 256 : pieces <= 512 ? 512 : 1024;
-        if (pieces <= threads)
-            hipLaunchKernelGGL(polynorm_vec_kernel<1>, dim3(rows), dim3(threads), 0, ctx->stream, z, coef, out, dim, stride, eps);
-        else if (pieces <= 2 * threads)
-            hipLaunchKernelGGL(polynorm_vec_kernel<2>, dim3(rows), dim3(threads), 0, ctx->stream, z, coef, out, dim, stride, eps);
-        else
-            hipLaunchKernelGGL(polynorm_vec_kernel<4>, dim3(rows), dim3(threads), 0, ctx->stream, z, coef, out, dim, stride, eps);
-    } else {
-        hipLaunchKernelGGL(polynorm_kernel, dim3(rows), dim3(256), 0, ctx->stream, z, coef, out, dim, stride, eps);
+    const bool vec = stride % 4 == 0 && stride <= 16384 && (((uintptr_t)z | (uintptr_t)out) & 15) == 0;
+    if (vec && exps && stride % 16 == 0) {
+        launch_polynorm_vec<true>(ctx, z, coef, out, rows, dim, stride, eps, exps);
+        LUMEN_CHECK_LAUNCH();
+        return LUMEN_OK;
     }
+    if (vec) launch_polynorm_vec<false>(ctx, z, coef, out, rows, dim, stride, eps, nullptr);
+    else hipLaunchKernelGGL(polynorm_kernel, dim3(rows), dim3(256), 0, ctx->stream, z, coef, out, dim, stride, eps);
     LUMEN_CHECK_LAUNCH();
-    return LUMEN_OK;
+    return exps ? launch_split_rows(ctx, out, rows, stride, out, exps) : LUMEN_OK;
 }
 
 __global__ __launch_bounds__(256) void token_shift_kernel(const float *__restrict__ h, const float *__restrict__ mu,
@@ -431,16 +459,58 @@ __global__ __launch_bounds__(256) void token_shift_vec_kernel(const float *__res
     if (t == s - 1) *(v4f *)(next + i) = c;
 }
 
+// The same with the mixes left as f16 pairs (f16_split.h): workgroup (token, mix).
+template <int VPT>
+__global__ __launch_bounds__(256) void token_shift_split_kernel(const float *__restrict__ h, const float *__restrict__ mu,
+                                                                const float *__restrict__ prev, float *__restrict__ next,
+                                                                float *__restrict__ mixes, int s, int dim, int *__restrict__ exps) {
+    __shared__ unsigned top[4];
+    const int t = blockIdx.x, mix = blockIdx.y, tid = threadIdx.x;
+    const float *cur = h + (size_t)t * dim, *bef = t ? cur - dim : prev;
+    v4f r[VPT];
+    unsigned m = 0;
+#pragma unroll
+    for (int i = 0; i < VPT; ++i) {
+        const int k = (tid + i * 256) * 4;
+        r[i] = v4f{0.f, 0.f, 0.f, 0.f};
+        if (k < dim) {
+            const v4f c = *(const v4f *)(cur + k), d = *(const v4f *)(bef + k) - c, f = *(const v4f *)(mu + (size_t)mix * dim + k);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) r[i][e] = fmaf(d[e], f[e], c[e]);
+            m = max(m, magnitude_bits(r[i]));
+            if (mix == 0 && t == s - 1) *(v4f *)(next + k) = c;
+        }
+    }
+    m = wave_umax(m);
+    if ((tid & 63) == 0) top[tid >> 6] = m;
+    __syncthreads();
+    const int e = row_exponent(max(max(top[0], top[1]), max(top[2], top[3])));
+    const float sc = exp2_int(e);
+    const size_t row = (size_t)mix * s + t;
+    if (tid == 0) exps[row] = e;
+#pragma unroll
+    for (int i = 0; i < VPT; ++i) {
+        const int k = (tid + i * 256) * 4;
+        if (k < dim) store_split4((uint16_t *)(mixes + row * dim), k, r[i], sc);
+    }
+}
+
 int launch_token_shift(lumen_ctx *ctx, const float *h, const float *mu, const float *prev, float *next, float *mixes, int n,
-                       int s, int dim) {
+                       int s, int dim, int *exps) {
     if (s <= 0 || dim <= 0) return LUMEN_OK;
     const bool vec = dim % 4 == 0 && (((uintptr_t)h | (uintptr_t)mu | (uintptr_t)prev | (uintptr_t)next | (uintptr_t)mixes) & 15) == 0;
+    if (vec && exps && dim % 16 == 0 && dim <= 4096) {
+        if (dim <= 2048) hipLaunchKernelGGL(token_shift_split_kernel<2>, dim3(s, n), dim3(256), 0, ctx->stream, h, mu, prev, next, mixes, s, dim, exps);
+        else hipLaunchKernelGGL(token_shift_split_kernel<4>, dim3(s, n), dim3(256), 0, ctx->stream, h, mu, prev, next, mixes, s, dim, exps);
+        LUMEN_CHECK_LAUNCH();
+        return LUMEN_OK;
+    }
     if (vec)
         hipLaunchKernelGGL(token_shift_vec_kernel, dim3(s, (dim + 1023) / 1024), dim3(256), 0, ctx->stream, h, mu, prev, next, mixes, n, s, dim);
     else
         hipLaunchKernelGGL(token_shift_kernel, dim3(s), dim3(256), 0, ctx->stream, h, mu, prev, next, mixes, n, s, dim);
     LUMEN_CHECK_LAUNCH();
-    return LUMEN_OK;
+    return exps ? launch_split_rows(ctx, mixes, n * s, dim, mixes, exps) : LUMEN_OK;
 }
 
 __global__ __launch_bounds__(256) void add_steps_kernel(const float *__restrict__ base, const float *__restrict__ step,

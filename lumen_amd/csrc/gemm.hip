@@ -1026,7 +1026,10 @@ static int gemm_stream_splits(const lumen_ctx *ctx, const GemmArgs &a) {
     while (s > 1 && (size_t)s * a.M * a.N * sizeof(float) > ((size_t)256 << 20)) --s;
     return s < 1 ? 1 : (int)s;
 }
-bool gemm_takes_split(int M, int K, int w_bf16) { return M > gemm_stream_max_rows(w_bf16) && K > 0 && K % 64 == 0; }
+// Split rows: more rows than the few-row kernels take (those read f32 rows), with bf16-stored weights from 48 on -- below, three bf16 products cost
+// the weights' stream nothing and the passes that split rows do (Llama-2-7B shape, 8 layers, before and after: 17 rows 1.56 -> 1.63
+// ms, 33 rows 1.65 -> 1.69, 64 rows 1.81 -> 1.78) --, whole pieces of 64 of K.
+bool gemm_takes_split(int M, int K, int w_bf16) { return M > (w_bf16 ? 47 : GEMM_STREAM_MAX_M) && K > 0 && K % 64 == 0; }
 int gemm_reserve_workspace(lumen_ctx *ctx, size_t need) {
     if (ctx->gemm_ws_bytes >= need) return LUMEN_OK;
     HIP_TRY(hipStreamSynchronize(ctx->stream));

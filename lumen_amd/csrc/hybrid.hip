@@ -38,6 +38,7 @@ struct Param {  // where a named tensor goes
     std::function<std::vector<float>(const std::vector<float> &)> expand;  // ... or what this makes of the whole tensor, [n] f32
     void *dst2 = nullptr;  // columns from col_split on go to a second matrix
     size_t col_split = 0;
+    int *exps = nullptr, *exps2 = nullptr;  // exponents of the rows of dst / dst2 (f16_split.h), or null
 };
 
 struct Layer {
@@ -52,6 +53,7 @@ struct Layer {
     int seg = 0, seg_last = 0;           // WKV: rows of a token-shift product
     int od = 0;                          // channels of the mixer's output (rounded)
     void *w_proj = nullptr, *w_o = nullptr, *w_lo = nullptr, *w_hi = nullptr, *w_up = nullptr, *w_down = nullptr;
+    int *e_proj = nullptr, *e_o = nullptr, *e_o2 = nullptr, *e_up = nullptr, *e_down = nullptr;  // exponents of their rows
     float *norm1 = nullptr, *norm2 = nullptr, *act = nullptr;
     float *norm1_b = nullptr, *norm1_a = nullptr, *norm2_b = nullptr, *norm2_a = nullptr;  // Dynamic Tanh: shift, alpha
     float *rg1_b = nullptr, *rg2_b = nullptr, *a_bias = nullptr;
@@ -84,6 +86,7 @@ struct lumen_hybrid {
     std::vector<Param> params;
     float *embed = nullptr, *final_norm = nullptr, *final_b = nullptr, *final_a = nullptr, *loop_step = nullptr, *positions = nullptr;
     void *head = nullptr, *loop_x = nullptr, *loop_x0 = nullptr;
+    int *e_loop_x = nullptr, *e_loop_x0 = nullptr;
     std::unique_ptr<SeqState> state;
     int len = 0;
     unsigned step = 0;  // forward passes since the reset: which slot of a two-slot state block is current (mirror of *d_step)
@@ -107,6 +110,11 @@ struct lumen_hybrid {
           *p_z = nullptr, *p_gate = nullptr, *p_logits = nullptr, *p_rows = nullptr, *p_raw = nullptr, *p_scan = nullptr, *p_mixed2 = nullptr,
           *p_y = nullptr, *p_y2 = nullptr, *p_rg = nullptr, *p_route = nullptr, *p_selw = nullptr, *p_act = nullptr, *p_eout = nullptr;
     int *p_ids = nullptr, *p_idx = nullptr, *p_plan = nullptr;
+    // split rows (f16_split.h) of a prompt's products: p_n, p_mixes, p_mixed, p_mixed2 and p_ff in place, rows that are read as f32 too in p_split
+    float *p_split = nullptr;
+    int *e_n = nullptr, *e_mixes = nullptr, *e_mixed = nullptr, *e_mixed2 = nullptr, *e_ff = nullptr, *e_split = nullptr;
+    const float *p_in = nullptr;  // what a mixer's projections read, with its exponents (null: f32 rows)
+    int *p_in_exp = nullptr;
     std::vector<void *> allocs;
     // per-class event times of a profiled step
     struct Probe *probe = nullptr;
@@ -145,8 +153,9 @@ static void add_param(lumen_hybrid *m, const std::string &name, std::vector<int6
 }
 
 // rows [row0, row0 + rows) of a weight matrix with rows of `cols` values
-static void add_matrix(lumen_hybrid *m, const std::string &name, void *base, int row0, int rows, int cols) {
+static void add_matrix(lumen_hybrid *m, const std::string &name, void *base, int row0, int rows, int cols, int *exps = nullptr) {
     add_param(m, name, {rows, cols}, (char *)base + (size_t)row0 * pad8(cols) * m->esz, false, rows, cols, pad8(cols));
+    m->params.back().exps = exps ? exps + row0 : nullptr;
 }
 static void add_vector(lumen_hybrid *m, const std::string &name, float *dst, int n) {
     add_param(m, name, {n}, dst, true, 1, n, n);
@@ -246,6 +255,7 @@ static int create_layer(lumen_hybrid *m, Layer &L, int i) {
     L.hi_rank = pad8(c.rank_hi);
     LUMEN_TRY(create_norm(m, p + "norm1", &L.norm1, &L.norm1_b, &L.norm1_a));
     LUMEN_TRY(weight(&L.w_o, W, H * Dv));
+    LUMEN_TRY(alloc_t(m, &L.e_o, pad8(W)));
     auto block = [&](int n) {  // the next block of the projection matrix
         const int off = L.n_proj;
         L.n_proj += pad8(n);
@@ -254,10 +264,11 @@ static int create_layer(lumen_hybrid *m, Layer &L, int i) {
     if (c.mixer == LUMEN_MIXER_WINDOW_ATTENTION) {
         L.off_q = block(H * D); L.off_k = block(G * D); L.off_v = block(G * Dv); L.off_g = block(H * Dv);
         LUMEN_TRY(weight(&L.w_proj, L.n_proj, W));
-        add_matrix(m, mp + "q", L.w_proj, L.off_q, H * D, W);
-        add_matrix(m, mp + "k", L.w_proj, L.off_k, G * D, W);
-        add_matrix(m, mp + "v", L.w_proj, L.off_v, G * Dv, W);
-        add_matrix(m, mp + "g", L.w_proj, L.off_g, H * Dv, W);
+        LUMEN_TRY(alloc_t(m, &L.e_proj, L.n_proj));
+        add_matrix(m, mp + "q", L.w_proj, L.off_q, H * D, W, L.e_proj);
+        add_matrix(m, mp + "k", L.w_proj, L.off_k, G * D, W, L.e_proj);
+        add_matrix(m, mp + "v", L.w_proj, L.off_v, G * Dv, W, L.e_proj);
+        add_matrix(m, mp + "g", L.w_proj, L.off_g, H * Dv, W, L.e_proj);
         LUMEN_TRY(alloc_t(m, &L.q_norm, H * D));
         LUMEN_TRY(alloc_t(m, &L.k_norm, G * D));
         LUMEN_TRY(alloc_t(m, &L.r1, H));
@@ -279,13 +290,14 @@ static int create_layer(lumen_hybrid *m, Layer &L, int i) {
         L.seg_last = L.lo_rank;
         L.off_q = block(H * D); L.off_k = block(H * D); L.off_v = block(H * D); L.off_g = block(H * D); L.off_lo = block(c.rank_lo);
         LUMEN_TRY(weight(&L.w_proj, L.n_proj, W));
+        LUMEN_TRY(alloc_t(m, &L.e_proj, L.n_proj));
         LUMEN_TRY(alloc_t(m, &L.mu, (size_t)5 * m->W));
         const char *names[5] = {"r", "k", "v", "g", "w"};
         for (int s = 0; s < 5; ++s) {
             add_vector(m, mp + "mu." + names[s], L.mu + (size_t)s * m->W, W);
-            if (s < 4) add_matrix(m, mp + names[s], L.w_proj, s * L.seg, H * D, W);
+            if (s < 4) add_matrix(m, mp + names[s], L.w_proj, s * L.seg, H * D, W, L.e_proj);
         }
-        add_matrix(m, mp + "w1", L.w_proj, L.off_lo, c.rank_lo, W);
+        add_matrix(m, mp + "w1", L.w_proj, L.off_lo, c.rank_lo, W, L.e_proj);
         LUMEN_TRY(weight(&L.w_lo, H * D, c.rank_lo));
         add_matrix(m, mp + "w2", L.w_lo, 0, H * D, c.rank_lo);
         LUMEN_TRY(alloc_t(m, &L.bias, H * D));
@@ -298,12 +310,13 @@ static int create_layer(lumen_hybrid *m, Layer &L, int i) {
         L.off_q = block(H * D); L.off_k = block(H * D); L.off_v = block(H * D); L.off_g = block(H * D); L.off_a = block(H * D);
         L.off_lo = block(c.rank_lo); L.off_rg = block(W);
         LUMEN_TRY(weight(&L.w_proj, L.n_proj, W));
-        add_matrix(m, mp + "r", L.w_proj, L.off_q, H * D, W);
-        add_matrix(m, mp + "k", L.w_proj, L.off_k, H * D, W);
-        add_matrix(m, mp + "v", L.w_proj, L.off_v, H * D, W);
-        add_matrix(m, mp + "g", L.w_proj, L.off_g, H * D, W);
-        add_matrix(m, mp + "a", L.w_proj, L.off_a, H * D, W);
-        add_matrix(m, mp + "w1", L.w_proj, L.off_lo, c.rank_lo, W);
+        LUMEN_TRY(alloc_t(m, &L.e_proj, L.n_proj));
+        add_matrix(m, mp + "r", L.w_proj, L.off_q, H * D, W, L.e_proj);
+        add_matrix(m, mp + "k", L.w_proj, L.off_k, H * D, W, L.e_proj);
+        add_matrix(m, mp + "v", L.w_proj, L.off_v, H * D, W, L.e_proj);
+        add_matrix(m, mp + "g", L.w_proj, L.off_g, H * D, W, L.e_proj);
+        add_matrix(m, mp + "a", L.w_proj, L.off_a, H * D, W, L.e_proj);
+        add_matrix(m, mp + "w1", L.w_proj, L.off_lo, c.rank_lo, W, L.e_proj);
         LUMEN_TRY(weight(&L.w_lo, H * D, c.rank_lo));
         add_matrix(m, mp + "w2", L.w_lo, 0, H * D, c.rank_lo);
         LUMEN_TRY(alloc_t(m, &L.bias, H * D));
@@ -319,16 +332,17 @@ static int create_layer(lumen_hybrid *m, Layer &L, int i) {
         L.off_mq = block(Hm * Dm); L.off_mk = block(Hm * Dm); L.off_mv = block(Hm * Vm); L.off_mg = block(Hm * Vm);
         L.off_mi = block(Hm); L.off_mf = block(Hm); L.off_rg = block(W);
         LUMEN_TRY(weight(&L.w_proj, L.n_proj, W));
-        add_matrix(m, lp + "q", L.w_proj, L.off_q, H * D, W);
-        add_matrix(m, lp + "k", L.w_proj, L.off_k, G * D, W);
-        add_matrix(m, lp + "v", L.w_proj, L.off_v, G * Dv, W);
-        add_matrix(m, lp + "g", L.w_proj, L.off_g, H, W);
-        add_matrix(m, rp + "q", L.w_proj, L.off_mq, Hm * Dm, W);
-        add_matrix(m, rp + "k", L.w_proj, L.off_mk, Hm * Dm, W);
-        add_matrix(m, rp + "v", L.w_proj, L.off_mv, Hm * Vm, W);
-        add_matrix(m, rp + "g", L.w_proj, L.off_mg, Hm * Vm, W);
-        add_matrix(m, rp + "i", L.w_proj, L.off_mi, Hm, W);
-        add_matrix(m, rp + "f", L.w_proj, L.off_mf, Hm, W);
+        LUMEN_TRY(alloc_t(m, &L.e_proj, L.n_proj));
+        add_matrix(m, lp + "q", L.w_proj, L.off_q, H * D, W, L.e_proj);
+        add_matrix(m, lp + "k", L.w_proj, L.off_k, G * D, W, L.e_proj);
+        add_matrix(m, lp + "v", L.w_proj, L.off_v, G * Dv, W, L.e_proj);
+        add_matrix(m, lp + "g", L.w_proj, L.off_g, H, W, L.e_proj);
+        add_matrix(m, rp + "q", L.w_proj, L.off_mq, Hm * Dm, W, L.e_proj);
+        add_matrix(m, rp + "k", L.w_proj, L.off_mk, Hm * Dm, W, L.e_proj);
+        add_matrix(m, rp + "v", L.w_proj, L.off_mv, Hm * Vm, W, L.e_proj);
+        add_matrix(m, rp + "g", L.w_proj, L.off_mg, Hm * Vm, W, L.e_proj);
+        add_matrix(m, rp + "i", L.w_proj, L.off_mi, Hm, W, L.e_proj);
+        add_matrix(m, rp + "f", L.w_proj, L.off_mf, Hm, W, L.e_proj);
         // attention
         const int B = c.bias_rows, most = c.bias_max;
         L.bias_n = 1;  // distances up to the first whose row is the last one, and to all further ones
@@ -351,7 +365,8 @@ static int create_layer(lumen_hybrid *m, Layer &L, int i) {
         // matrix memory
         L.od2 = pad8(Hm * Vm);
         LUMEN_TRY(weight(&L.w_o2, W, Hm * Vm));
-        add_matrix(m, rp + "o", L.w_o2, 0, W, Hm * Vm);
+        LUMEN_TRY(alloc_t(m, &L.e_o2, pad8(W)));
+        add_matrix(m, rp + "o", L.w_o2, 0, W, Hm * Vm, L.e_o2);
         LUMEN_TRY(alloc_t(m, &L.i_bias, Hm));
         LUMEN_TRY(alloc_t(m, &L.f_bias, Hm));
         LUMEN_TRY(alloc_t(m, &L.gain, Hm * Vm));
@@ -369,12 +384,13 @@ static int create_layer(lumen_hybrid *m, Layer &L, int i) {
         L.off_q = block(G * D); L.off_k = block(G * D); L.off_v = block(H * Dv); L.off_b = block(H);
         L.off_lo = block(c.rank_lo); L.off_hi = block(c.rank_hi);
         LUMEN_TRY(weight(&L.w_proj, L.n_proj, W));
-        add_matrix(m, mp + "q", L.w_proj, L.off_q, G * D, W);
-        add_matrix(m, mp + "k", L.w_proj, L.off_k, G * D, W);
-        add_matrix(m, mp + "v", L.w_proj, L.off_v, H * Dv, W);
-        add_matrix(m, mp + "b", L.w_proj, L.off_b, H, W);
-        add_matrix(m, mp + "a1", L.w_proj, L.off_lo, c.rank_lo, W);
-        add_matrix(m, mp + "g1", L.w_proj, L.off_hi, c.rank_hi, W);
+        LUMEN_TRY(alloc_t(m, &L.e_proj, L.n_proj));
+        add_matrix(m, mp + "q", L.w_proj, L.off_q, G * D, W, L.e_proj);
+        add_matrix(m, mp + "k", L.w_proj, L.off_k, G * D, W, L.e_proj);
+        add_matrix(m, mp + "v", L.w_proj, L.off_v, H * Dv, W, L.e_proj);
+        add_matrix(m, mp + "b", L.w_proj, L.off_b, H, W, L.e_proj);
+        add_matrix(m, mp + "a1", L.w_proj, L.off_lo, c.rank_lo, W, L.e_proj);
+        add_matrix(m, mp + "g1", L.w_proj, L.off_hi, c.rank_hi, W, L.e_proj);
         LUMEN_TRY(weight(&L.w_lo, H * D, c.rank_lo));
         LUMEN_TRY(weight(&L.w_hi, H * Dv, c.rank_hi));
         add_matrix(m, mp + "a2", L.w_lo, 0, H * D, c.rank_lo);
@@ -394,10 +410,10 @@ static int create_layer(lumen_hybrid *m, Layer &L, int i) {
         add_vector(m, mp + "A_log", L.a_log, H);
         add_vector(m, mp + "norm", L.gain, Dv);
     }
-    add_matrix(m, mp + (c.mixer == LUMEN_MIXER_PARALLEL ? "left.o" : "o"), L.w_o, 0, W, H * Dv);
+    add_matrix(m, mp + (c.mixer == LUMEN_MIXER_PARALLEL ? "left.o" : "o"), L.w_o, 0, W, H * Dv, L.e_o);
     if (m->cfg.residual_gate) {
         LUMEN_TRY(alloc_t(m, &L.rg1_b, m->W));
-        add_matrix(m, p + "rg1", L.w_proj, L.off_rg, W, W);
+        add_matrix(m, p + "rg1", L.w_proj, L.off_rg, W, W, L.e_proj);
         add_vector(m, p + "rg1.b", L.rg1_b, W);
     }
     if (c.ff > 0) {
@@ -407,14 +423,15 @@ static int create_layer(lumen_hybrid *m, Layer &L, int i) {
         L.up_at = m->cfg.residual_gate ? m->W : 0;
         L.n_up = L.up_at + pad8(experts ? c.experts : c.ff);
         LUMEN_TRY(weight(&L.w_up, L.n_up, W));
+        LUMEN_TRY(alloc_t(m, &L.e_up, L.n_up));
         if (m->cfg.residual_gate) {
             LUMEN_TRY(alloc_t(m, &L.rg2_b, m->W));
-            add_matrix(m, p + "rg2", L.w_up, 0, W, W);
+            add_matrix(m, p + "rg2", L.w_up, 0, W, W, L.e_up);
             add_vector(m, p + "rg2.b", L.rg2_b, W);
         }
         if (experts) {
             const size_t F = pad8(c.ff), K = m->W, E = c.experts;
-            add_matrix(m, p + "mlp.router", L.w_up, L.up_at, c.experts, W);
+            add_matrix(m, p + "mlp.router", L.w_up, L.up_at, c.experts, W, L.e_up);
             LUMEN_TRY(alloc_zero(m, &L.w_eup, E * 2 * F * K * m->esz));
             LUMEN_TRY(alloc_zero(m, &L.w_edown, E * K * F * m->esz));
             for (size_t e = 0; e < E; ++e) {  // gate and up rows in turn
@@ -429,8 +446,9 @@ static int create_layer(lumen_hybrid *m, Layer &L, int i) {
             m->max_experts = std::max(m->max_experts, pad8(c.experts));
         } else {
             LUMEN_TRY(weight(&L.w_down, W, c.ff));
-            add_matrix(m, p + "mlp.up", L.w_up, L.up_at, c.ff, W);
-            add_matrix(m, p + "mlp.down", L.w_down, 0, W, c.ff);
+            LUMEN_TRY(alloc_t(m, &L.e_down, pad8(W)));
+            add_matrix(m, p + "mlp.up", L.w_up, L.up_at, c.ff, W, L.e_up);
+            add_matrix(m, p + "mlp.down", L.w_down, 0, W, c.ff, L.e_down);
             if (c.ff_kind == LUMEN_FF_POLYNORM) {
                 LUMEN_TRY(alloc_t(m, &L.act, 4));
                 add_vector(m, p + "mlp.act", L.act, 4);
@@ -465,6 +483,9 @@ static int create_impl(lumen_hybrid *m, const lumen_hybrid_layer *layers) {
             Param p;
             p.name = "loop.in"; p.shape = {c.width, 2 * c.width}; p.dst = m->loop_x; p.dst2 = m->loop_x0; p.col_split = c.width;
             p.rows = c.width; p.cols = 2 * (size_t)c.width; p.ld = W;
+            LUMEN_TRY(alloc_t(m, &m->e_loop_x, W));
+            LUMEN_TRY(alloc_t(m, &m->e_loop_x0, W));
+            p.exps = m->e_loop_x; p.exps2 = m->e_loop_x0;
             m->params.push_back(p);
         }
         add_param(m, "loop.step", {c.loop_times, c.width}, m->loop_step, true, c.loop_times, c.width, W);
@@ -637,6 +658,8 @@ extern "C" int lumen_hybrid_set_param(lumen_hybrid *m, const char *name, const v
                                          (p.cols - first) * esz, nr, hipMemcpyHostToDevice, m->ctx->stream));
             HIP_TRY(hipStreamSynchronize(m->ctx->stream));
         }
+        if (p.exps) LUMEN_TRY(launch_row_exponents(m->ctx, p.dst, !to_f32, (int)p.rows, (int)p.ld, 0, 1, p.exps));
+        if (p.exps2) LUMEN_TRY(launch_row_exponents(m->ctx, p.dst2, !to_f32, (int)p.rows, (int)p.ld, 0, 1, p.exps2));
         return LUMEN_OK;
     }
     LUMEN_FAIL(LUMEN_ERR_INVALID, "Parameter %s not found in model", name);
@@ -939,6 +962,11 @@ static int ensure_prompt_buffers(lumen_hybrid *m, int s) {
     LUMEN_TRY(get(&m->p_xb, S * W));
     LUMEN_TRY(get(&m->p_n, S * W));
     LUMEN_TRY(get(&m->p_rows, S * W));
+    LUMEN_TRY(get(&m->p_split, S * W));
+    {
+        int **e[] = {&m->e_n, &m->e_mixed, &m->e_mixed2, &m->e_ff, &m->e_split, &m->e_mixes};
+        for (int **q : e) LUMEN_TRY(alloc_t(m, q, q == &m->e_mixes ? 5 * S : S, &m->pf_allocs));
+    }
     LUMEN_TRY(get(&m->p_proj, S * m->max_proj));
     if (wkv) LUMEN_TRY(get(&m->p_mixes, 5 * S * W));
     LUMEN_TRY(get(&m->p_mixed, S * m->max_od));
@@ -985,9 +1013,28 @@ static GemmArgs gemm_args(const lumen_hybrid *m, const float *A, const void *w, 
     return g;
 }
 
+// Do a prompt's products with K inner values run on split rows?  Rows that nothing leaves split by the way take a pass of their own (the
+// mixers' outputs; with gated residuals the norms too, whose rows the experts read as f32), which pays from some size on.  Prompt passes
+// before and after, ms: Pinavik 2048 wide, bf16, 96 tokens 2.66 -> 2.55, 1024 wide, f32, 128 tokens 2.21 -> 2.25 and 200 tokens 2.53 -> 2.49;
+// Nufapel 2048 wide 128 tokens 4.49 -> 4.59 and 200 tokens 5.18 -> 5.12, 1024 wide 200 tokens 3.95 -> 4.06 and 512 tokens level.
+static bool split_rows(const lumen_hybrid *m, int s, int K) {
+    const long least = m->cfg.residual_gate ? 7L << 16 : 3L << 16;
+    return (long)s * m->W >= least && K <= 16384 && gemm_takes_split(s, K, m->bf16);
+}
+static GemmArgs gemm_args(const lumen_hybrid *m, const float *A, const int *a_exp, const void *w, const int *w_exp, float *C, int M, int N, int K) {
+    GemmArgs g = gemm_args(m, A, w, C, M, N, K);
+    if (a_exp) { g.a_split = (const uint16_t *)A; g.a_exp = a_exp; g.w_exp = w_exp; }
+    return g;
+}
+// rows that only a product reads, split in place: their exponents, or null where the product takes f32 rows
+static int split_in_place(const lumen_hybrid *m, float *x, int s, int K, int *exps, int **used) {
+    *used = split_rows(m, s, K) ? exps : nullptr;
+    return *used ? launch_split_rows(m->ctx, x, s, K, x, exps) : LUMEN_OK;
+}
+
 static int prompt_attention(lumen_hybrid *m, const Layer &L, const Run &r, int s) {
     WindowAttnArgs a = attn_args(m, L, r, m->p_proj, L.n_proj);
-    LUMEN_TRY(launch_gemm(m->ctx, gemm_args(m, m->p_n, L.w_proj, m->p_proj, s, L.n_proj, m->W)));
+    LUMEN_TRY(launch_gemm(m->ctx, gemm_args(m, m->p_in, m->p_in_exp, L.w_proj, L.e_proj, m->p_proj, s, L.n_proj, m->W)));
     a.out = m->p_mixed; a.out_stride = L.od; a.pos = m->len; a.s = s; a.qn = m->p_q;
     return launch_window_attn_prefill(m->ctx, a);
 }
@@ -997,13 +1044,15 @@ static int prompt_wkv(lumen_hybrid *m, const Layer &L, const Run &r, int s) {
     const int W = m->W, H = L.c.heads, D = L.c.dim;
     float *shift = m->state->ptr(r.st_aux);
     const unsigned slot = m->step & 1u;
-    LUMEN_TRY(launch_token_shift(ctx, m->p_n, L.mu, shift + (size_t)slot * W, shift + (size_t)(slot ^ 1u) * W, m->p_mixes, 5, s, W));
+    LUMEN_TRY(launch_token_shift(ctx, m->p_n, L.mu, shift + (size_t)slot * W, shift + (size_t)(slot ^ 1u) * W, m->p_mixes, 5, s, W,
+                                 split_rows(m, s, W) ? m->e_mixes : nullptr));
     // r, k, v, gate and the decay's inner vector: a matrix each, one after the other
     float *part[5];
     for (int i = 0; i < 5; ++i) {
         part[i] = m->p_proj + (size_t)i * s * L.seg;
-        LUMEN_TRY(launch_gemm(ctx, gemm_args(m, m->p_mixes + (size_t)i * s * W, (const char *)L.w_proj + (size_t)i * L.seg * W * m->esz, part[i],
-                                             s, i < 4 ? L.seg : L.seg_last, W)));
+        LUMEN_TRY(launch_gemm(ctx, gemm_args(m, m->p_mixes + (size_t)i * s * W, split_rows(m, s, W) ? m->e_mixes + (size_t)i * s : nullptr,
+                                             (const char *)L.w_proj + (size_t)i * L.seg * W * m->esz, L.e_proj + (size_t)i * L.seg, part[i], s,
+                                             i < 4 ? L.seg : L.seg_last, W)));
     }
     LUMEN_TRY(launch_tanh(ctx, part[4], m->p_lo, (size_t)s * L.seg_last));
     LUMEN_TRY(launch_gemm(ctx, gemm_args(m, m->p_lo, L.w_lo, m->p_z, s, L.seg, L.lo_rank)));
@@ -1019,7 +1068,7 @@ static int prompt_wkv(lumen_hybrid *m, const Layer &L, const Run &r, int s) {
 static int prompt_delta(lumen_hybrid *m, const Layer &L, const Run &r, int s) {
     lumen_ctx *ctx = m->ctx;
     const int H = L.c.heads, G = L.c.kv_heads, D = L.c.dim, Dv = L.c.vdim, keep = L.c.conv - 1;
-    LUMEN_TRY(launch_gemm(ctx, gemm_args(m, m->p_n, L.w_proj, m->p_proj, s, L.n_proj, m->W)));
+    LUMEN_TRY(launch_gemm(ctx, gemm_args(m, m->p_in, m->p_in_exp, L.w_proj, L.e_proj, m->p_proj, s, L.n_proj, m->W)));
     float *conv = m->state->ptr(r.st_aux);
     const unsigned slot = m->step & 1u;
     DeltaPrepArgs p = {};
@@ -1045,7 +1094,7 @@ static int prompt_delta(lumen_hybrid *m, const Layer &L, const Run &r, int s) {
 static int prompt_general(lumen_hybrid *m, const Layer &L, const Run &r, int s) {
     lumen_ctx *ctx = m->ctx;
     const int H = L.c.heads, D = L.c.dim, n = L.n_proj;
-    LUMEN_TRY(launch_gemm(ctx, gemm_args(m, m->p_n, L.w_proj, m->p_proj, s, n, m->W)));
+    LUMEN_TRY(launch_gemm(ctx, gemm_args(m, m->p_in, m->p_in_exp, L.w_proj, L.e_proj, m->p_proj, s, n, m->W)));
     LUMEN_TRY(launch_tanh_rows(ctx, m->p_proj + L.off_lo, n, m->p_lo, s, L.lo_rank));
     LUMEN_TRY(launch_gemm(ctx, gemm_args(m, m->p_lo, L.w_lo, m->p_z, s, pad8(H * D), L.lo_rank)));
     RecurrenceArgs a = {};
@@ -1088,19 +1137,30 @@ static int prompt_gated_layer(lumen_hybrid *m, const Layer &L, const Run &r, int
         return launch_gated_residual(ctx, p);
     };
     const NormRef norm2 = {L.norm2, L.norm2_b, L.norm2_a};
+    // (p_n is read as f32 rows too, by the experts)
+    auto split_norm = [&]() {
+        m->p_in_exp = split_rows(m, s, W) ? m->e_split : nullptr;
+        m->p_in = m->p_in_exp ? m->p_split : m->p_n;
+        return m->p_in_exp ? launch_split_rows(ctx, m->p_n, s, W, m->p_split, m->e_split) : LUMEN_OK;
+    };
+    int *exps = nullptr;
+    LUMEN_TRY(split_norm());
     if (L.c.mixer == LUMEN_MIXER_PARALLEL) {
         LUMEN_TRY(prompt_attention(m, L, r, s));
         LUMEN_TRY(prompt_memory(m, L, r, s));
-        LUMEN_TRY(launch_gemm(ctx, gemm_args(m, m->p_mixed2, L.w_o2, m->p_y2, s, W, L.od2)));
+        LUMEN_TRY(split_in_place(m, m->p_mixed2, s, L.od2, m->e_mixed2, &exps));
+        LUMEN_TRY(launch_gemm(ctx, gemm_args(m, m->p_mixed2, exps, L.w_o2, L.e_o2, m->p_y2, s, W, L.od2)));
         p.y2 = m->p_y2; p.w1 = L.out1; p.w2 = L.out2; p.pair_scale = 0.5f;
     } else {
         LUMEN_TRY(prompt_general(m, L, r, s));
     }
-    LUMEN_TRY(launch_gemm(ctx, gemm_args(m, m->p_mixed, L.w_o, m->p_y, s, W, L.od)));
+    LUMEN_TRY(split_in_place(m, m->p_mixed, s, L.od, m->e_mixed, &exps));
+    LUMEN_TRY(launch_gemm(ctx, gemm_args(m, m->p_mixed, exps, L.w_o, L.e_o, m->p_y, s, W, L.od)));
     p.y = m->p_y;
     LUMEN_TRY(sum(cur, m->p_proj + L.off_rg, L.n_proj, L.rg1_b, L.c.ff > 0 ? norm2 : next));
     if (L.c.ff <= 0) return LUMEN_OK;
-    LUMEN_TRY(launch_gemm(ctx, gemm_args(m, m->p_n, L.w_up, m->p_rg, s, W, W)));
+    LUMEN_TRY(split_norm());
+    LUMEN_TRY(launch_gemm(ctx, gemm_args(m, m->p_in, m->p_in_exp, L.w_up, L.e_up, m->p_rg, s, W, W)));
     const void *up = (const char *)L.w_up + (size_t)L.up_at * W * m->esz;
     p.y2 = nullptr;
     if (L.c.ff_kind == LUMEN_FF_EXPERTS) {
@@ -1112,9 +1172,10 @@ static int prompt_gated_layer(lumen_hybrid *m, const Layer &L, const Run &r, int
         p.y = m->p_eout; p.top = L.c.top; p.sel_w = m->p_selw;
     } else {
         const int F = pad8(L.c.ff);
-        LUMEN_TRY(launch_gemm(ctx, gemm_args(m, m->p_n, up, m->p_ff, s, F, W)));
+        LUMEN_TRY(launch_gemm(ctx, gemm_args(m, m->p_in, m->p_in_exp, up, L.e_up + L.up_at, m->p_ff, s, F, W)));
         LUMEN_TRY(launch_gelu(ctx, m->p_ff, m->p_ff, (size_t)s * F));
-        LUMEN_TRY(launch_gemm(ctx, gemm_args(m, m->p_ff, L.w_down, m->p_y, s, W, F)));
+        LUMEN_TRY(split_in_place(m, m->p_ff, s, F, m->e_ff, &exps));
+        LUMEN_TRY(launch_gemm(ctx, gemm_args(m, m->p_ff, exps, L.w_down, L.e_down, m->p_y, s, W, F)));
     }
     return sum(x, m->p_rg, W, L.rg2_b, next);
 }
@@ -1128,16 +1189,19 @@ static int run_prompt(lumen_hybrid *m, const int32_t *ids, int s, const int *wan
     HIP_TRY(hipMemcpyAsync(m->p_ids, ids, sizeof(int) * (size_t)s, hipMemcpyHostToDevice, ctx->stream));
     LUMEN_TRY(embed_rows(m, m->p_ids, s, nullptr, m->len, m->p_x0));
     const bool mix = c.loop_times > 0 && c.loop_kind == LUMEN_LOOP_MIX, dyt = c.norm_kind == LUMEN_NORM_DYT;
+    const bool split_w = split_rows(m, s, W);
     if (mix) {
-        LUMEN_TRY(launch_gemm(ctx, gemm_args(m, m->p_x0, m->loop_x0, m->p_n, s, W, W)));
+        if (split_w) LUMEN_TRY(launch_split_rows(ctx, m->p_x0, s, W, m->p_split, m->e_split));
+        LUMEN_TRY(launch_gemm(ctx, gemm_args(m, split_w ? m->p_split : m->p_x0, split_w ? m->e_split : nullptr, m->loop_x0, m->e_loop_x0, m->p_n, s, W, W)));
         LUMEN_TRY(launch_add_steps(ctx, m->p_n, m->loop_step, m->p_steps, c.loop_times, s, W));
     }
     const float *cur = m->p_x0;
     bool normed = false;  // p_n holds norm1 of the next layer: it came with the product that finished cur
     auto out = [&]() { return cur == m->p_x0 ? m->p_xa : const_cast<float *>(cur); };
-    auto residual_gemm = [&](GemmArgs g, const float *residual, float alpha, const float *norm) {
+    // norm_exp: p_n is to hold split rows, its reader being a product (the token shift reads f32 rows)
+    auto residual_gemm = [&](GemmArgs g, const float *residual, float alpha, const float *norm, int *norm_exp) {
         g.epi = EPI_RESIDUAL; g.residual = residual; g.alpha = alpha;
-        if (norm) { g.norm_w = norm; g.norm_out = m->p_n; g.norm_eps = m->eps_w; }
+        if (norm) { g.norm_w = norm; g.norm_out = m->p_n; g.norm_eps = m->eps_w; g.norm_exp = norm_exp; }
         normed = norm != nullptr;
         cur = g.C;
         return launch_gemm(ctx, g);
@@ -1148,16 +1212,23 @@ static int run_prompt(lumen_hybrid *m, const int32_t *ids, int s, const int *wan
         const Run *next = ri + 1 < m->runs.size() ? &m->runs[ri + 1] : nullptr;
         const Layer *next_layer = next && next->pass < 0 ? &m->layers[next->layer] : nullptr;
         const float *next_norm = next_layer ? next_layer->norm1 : nullptr;
+        auto norm1_exp = [&](const Layer &y) { return split_w && !dyt && y.c.mixer != LUMEN_MIXER_WKV ? m->e_n : nullptr; };
+        int *next_exp = next_layer ? norm1_exp(*next_layer) : nullptr, *exps = nullptr;
         if (r.pass >= 0 && !mix) {
             float *y = cur == m->p_xa ? m->p_xb : m->p_xa;
             LUMEN_TRY(launch_add_steps(ctx, cur, m->loop_step + (size_t)r.pass * W, y, 1, s, W));
             cur = y;
             normed = false;
-        } else if (r.pass >= 0)
-            LUMEN_TRY(residual_gemm(gemm_args(m, cur, m->loop_x, cur == m->p_xa ? m->p_xb : m->p_xa, s, W, W),
-                                    m->p_steps + (size_t)r.pass * s * W, 1.0f, L.norm1));
+        } else if (r.pass >= 0) {
+            if (split_w) LUMEN_TRY(launch_split_rows(ctx, cur, s, W, m->p_split, m->e_split));
+            LUMEN_TRY(residual_gemm(gemm_args(m, split_w ? m->p_split : cur, split_w ? m->e_split : nullptr, m->loop_x, m->e_loop_x,
+                                              cur == m->p_xa ? m->p_xb : m->p_xa, s, W, W),
+                                    m->p_steps + (size_t)r.pass * s * W, 1.0f, L.norm1, norm1_exp(L)));
+        }
         if (!normed && dyt) LUMEN_TRY(launch_dyt(ctx, cur, L.norm1_a, L.norm1, L.norm1_b, m->p_n, s, W));
-        else if (!normed) LUMEN_TRY(launch_rmsnorm(ctx, cur, L.norm1, m->p_n, s, W, m->eps_w));
+        else if (!normed) LUMEN_TRY(launch_rmsnorm(ctx, cur, L.norm1, m->p_n, s, W, m->eps_w, norm1_exp(L)));
+        m->p_in = m->p_n;
+        m->p_in_exp = norm1_exp(L);
         if (c.residual_gate) {
             float *x = out();
             LUMEN_TRY(prompt_gated_layer(m, L, r, s, cur, x, next_layer ? NormRef{next_layer->norm1, next_layer->norm1_b, next_layer->norm1_a} : NormRef{}));
@@ -1169,12 +1240,16 @@ static int run_prompt(lumen_hybrid *m, const int32_t *ids, int s, const int *wan
         if (L.c.mixer == LUMEN_MIXER_WINDOW_ATTENTION) LUMEN_TRY(prompt_attention(m, L, r, s));
         else if (L.c.mixer == LUMEN_MIXER_WKV) LUMEN_TRY(prompt_wkv(m, L, r, s));
         else LUMEN_TRY(prompt_delta(m, L, r, s));
-        LUMEN_TRY(residual_gemm(gemm_args(m, m->p_mixed, L.w_o, out(), s, W, L.od), cur, c.residual_mult, L.c.ff > 0 ? L.norm2 : next_norm));
+        int *norm2_exp = split_w ? m->e_n : nullptr;
+        LUMEN_TRY(split_in_place(m, m->p_mixed, s, L.od, m->e_mixed, &exps));
+        LUMEN_TRY(residual_gemm(gemm_args(m, m->p_mixed, exps, L.w_o, L.e_o, out(), s, W, L.od), cur, c.residual_mult, L.c.ff > 0 ? L.norm2 : next_norm,
+                                L.c.ff > 0 ? norm2_exp : next_exp));
         if (L.c.ff > 0) {
             const int F = pad8(L.c.ff);
-            LUMEN_TRY(launch_gemm(ctx, gemm_args(m, m->p_n, L.w_up, m->p_ff, s, F, W)));
-            LUMEN_TRY(launch_polynorm(ctx, m->p_ff, L.act, m->p_ff, s, L.c.ff, F, c.norm_eps));
-            LUMEN_TRY(residual_gemm(gemm_args(m, m->p_ff, L.w_down, out(), s, W, F), cur, c.residual_mult, next_norm));
+            int *ff_exp = split_rows(m, s, F) ? m->e_ff : nullptr;
+            LUMEN_TRY(launch_gemm(ctx, gemm_args(m, m->p_n, norm2_exp, L.w_up, L.e_up, m->p_ff, s, F, W)));
+            LUMEN_TRY(launch_polynorm(ctx, m->p_ff, L.act, m->p_ff, s, L.c.ff, F, c.norm_eps, ff_exp));
+            LUMEN_TRY(residual_gemm(gemm_args(m, m->p_ff, ff_exp, L.w_down, L.e_down, out(), s, W, F), cur, c.residual_mult, next_norm, next_exp));
         }
         LUMEN_TRY(tap_rows(m, tap, ri, cur, s));
     }

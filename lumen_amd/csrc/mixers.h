@@ -13,10 +13,11 @@ enum GateAct { GATE_NONE = 0, GATE_SIGMOID = 1, GATE_SILU = 2 };
 // ------------------------------------------------------------- row operations (elementwise.hip)
 // out = a N(z) + b N(z^2) + c N(z^3) + e over the first dim of each row's `stride` elements (out may be z);
 // coef = {a, b, c, e}
-int launch_polynorm(lumen_ctx *ctx, const float *z, const float *coef, float *out, int rows, int dim, int stride, float eps);
+// (here and below: exps not null -- rows left split with their exponents there, f16_split.h)
+int launch_polynorm(lumen_ctx *ctx, const float *z, const float *coef, float *out, int rows, int dim, int stride, float eps, int *exps = nullptr);
 // mixes [n][s][dim]: h_t + (h_{t-1} - h_t) mu_i; h_{-1} is prev [dim], the last h goes to next [dim] (not prev)
 int launch_token_shift(lumen_ctx *ctx, const float *h, const float *mu, const float *prev, float *next, float *mixes, int n,
-                       int s, int dim);
+                       int s, int dim, int *exps = nullptr);
 // out [times][rows][dim] = base [rows][dim] + step [times][dim]
 int launch_add_steps(lumen_ctx *ctx, const float *base, const float *step, float *out, int times, int rows, int dim);
 // out row i = x row idx[i]

@@ -1,4 +1,4 @@
-"""GPU parity of the prompt products that run on f16 pairs (prompts of more than 32 rows, 16 with bf16-stored weights, inner sizes that
+"""GPU parity of the prompt products that run on f16 pairs (prompts of more than 32 rows, 47 with bf16-stored weights, inner sizes that
 are multiples of 64): row and column counts around the tiles' edges, one piece of K and many, rows of very different
 magnitudes, rows of zeros and rows that are not finite, against the CPU oracle.
 
@@ -11,6 +11,7 @@ from lumen_amd import synth
 from lumen_amd.layers import KVCacheInner, RotaryEmbedding
 from lumen_amd.models import LlamaModel
 from oracle import lumen_oracle as lo
+from tests import hybrid_util, nufapel_util
 from tests.gpu_util import max_rel
 from tests.test_gpu_attention import gpu_prefill
 
@@ -118,3 +119,25 @@ def test_prompt_attention_over_magnitudes(d, h, h_kv, s, past, q_exp, k_exp, v_e
         rc, ref = lo.attn_prefill(ora, q, k, v, cos, sin, scale)
         assert rc == lo.LO_OK
     assert max_rel(got * 2.0 ** -v_exp, ref * 2.0 ** -v_exp) <= 2e-5
+
+
+HYBRIDS = {
+    "pinavik": lambda: (hybrid_util, hybrid_util.config(1024, 307, [
+        hybrid_util.attention(4, 2, 32, 32, 50, ff=320), hybrid_util.wkv(4, 32, ff=100), hybrid_util.delta(2, 1, 64, 32, ff=192),
+        hybrid_util.wkv(2, 64)], loop=(1, 3, 2))),
+    "nufapel": lambda: (nufapel_util, nufapel_util.config(1024, 307, [
+        nufapel_util.parallel((4, 2, 32, 32), (2, 64, 64), nufapel_util.dense(320)), nufapel_util.general(4, 32, nufapel_util.dense(100))], loop=(0, 2, 2))),
+}
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("name,tokens", [("pinavik", 193), ("pinavik", 320), ("nufapel", 449)])
+def test_hybrid_prompt_at_once_and_in_portions(tmp_path, name, tokens, dtype):
+    """Portions of 60 tokens run on f32 rows (their rows times the width are below what split rows are taken for), the prompt at once on split
+    ones; sums of up to 1024 terms in another order, over a few layers: 2e-5 of the largest logit, as for other cuts of a prompt."""
+    util, cfg = HYBRIDS[name]()
+    model = hybrid_util.load(tmp_path, cfg, util.make_params(cfg, seed=4), dtype)
+    ids = synth.make_tokens(tokens, 307, seed=tokens)
+    at_once, portions = (hybrid_util.run(model, ids, cuts) for cuts in ([tokens], [60]))
+    assert max_rel(at_once, portions) <= 2e-5
+    assert not np.array_equal(at_once, portions)  # (else both ran on the same kernels)
