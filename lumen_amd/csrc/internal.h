@@ -56,8 +56,8 @@ struct lumen_ctx {
     int *err_host = nullptr;
     float *gemm_ws = nullptr;      // split-K workspace of the prefill GEMM, grown on demand
     size_t gemm_ws_bytes = 0;
-    unsigned *kv_range = nullptr;  // largest magnitudes of a prompt attention's keys and values, grown on demand
-    size_t kv_range_bytes = 0;
+    float *attn_ws = nullptr;      // a prompt attention's unfinished rows and its keys' and values' largest magnitudes, grown on demand
+    size_t attn_ws_bytes = 0;
     float *mixer_ws = nullptr;     // per-chunk operands of the recurrences, grown on demand
     size_t mixer_ws_bytes = 0;
     // this device's address of the fixed scratch array behind lumen_attn_decode_static_f32
@@ -401,7 +401,11 @@ struct AttnPrefillArgs {
     float norm_eps;
     float *q_rot;    // scratch [B, S, Hq, D]
     int *out_exp;    // not null: the rows of out are left split (f16_split.h) with their exponents here [B, S]
-    const unsigned *kv_range;  // set by the launcher: largest magnitudes of the cached keys and values
+    // set by the launcher: largest magnitudes of the cached keys and values; keys per part and the parts' unfinished rows [b s hq][parts][d] and
+    // (maximum, sum) of theirs
+    const unsigned *kv_range;
+    int key_chunk;
+    float *part, *part_ml;
     // q, k and v may arrive as in_splits partial sums (a GEMM's K splits), copy i at pointer + i * in_split_stride
     // floats, to be added in index order; 0 or 1 = plain values.
     int in_splits;

@@ -16,6 +16,8 @@
 // the next product reads them split.
 // Bound by the matrix instructions and the softmax between them, which wait for each other within a wavefront; two per SIMD overlap.
 // With three bf16 parts: 420 us for 3968 positions of 32 heads of 64 (4 KV heads), with f16 pairs 286; 509 of 32 heads of 128: 61 -> 47.
+// Few positions behind a long cache leave most compute units without a block of queries: the keys are then cut into parts (128 positions
+// behind 2900, 32 heads of 64: 111 us in one part, 33 in 16; 256 behind 2900, 16 heads of 128: 198 -> 56).
 //
 // Per wavefront (32 rows) and key tile, everything transposed so that a lane owns one query row:
 //   S^T = K Q^T       K from LDS ([part][key][element], split on its way in) is the A operand, Q
@@ -82,7 +84,9 @@ __global__ __launch_bounds__(256) void kv_range_kernel(const float *k, const flo
 
 // KT: key tiles of 32 per trip of the loop (2 for head_dim 64: one barrier pair, one row maximum and one rescale of
 // O per 64 keys; 1 for head_dim 128, whose K and V tiles fill LDS twice as fast).
-template <int D, int NREP, int KT>
+// PART: blockIdx.z / b is a part of the keys (a.key_chunk each, whole trips); the unfinished rows go to a.part and a.part_ml for
+// merge_parts_kernel.
+template <int D, int NREP, int KT, bool PART>
 __global__ __launch_bounds__(FA_THREADS, 2) void attn_prefill_f16x2_kernel(AttnPrefillArgs a) {
     constexpr int BQ = FA_ROWS / NREP;  // positions per workgroup
     constexpr int KEYS = FA_KEYS * KT;   // keys per trip
@@ -96,10 +100,11 @@ __global__ __launch_bounds__(FA_THREADS, 2) void attn_prefill_f16x2_kernel(AttnP
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int c = lane & 31, half = lane >> 5;
     // workgroups are dealt in index order: the blocks of late positions (most keys) go first
-    const int q0 = (int)(gridDim.x - 1 - blockIdx.x) * BQ, hk = blockIdx.y, bb = blockIdx.z;
+    const int q0 = (int)(gridDim.x - 1 - blockIdx.x) * BQ, hk = blockIdx.y, bb = PART ? (int)blockIdx.z % a.b : (int)blockIdx.z;
+    const int key_part = PART ? (int)blockIdx.z / a.b : 0;
     const int L = a.past_len + a.s;
     // exponents of this head's keys and values; of all heads' values, which no output exceeds
-    const unsigned *kr = a.kv_range + ((size_t)bb * a.hkv + hk / a.kv_div) * FA_CHUNKS, *vr = kr + (size_t)gridDim.z * a.hkv * FA_CHUNKS;
+    const unsigned *kr = a.kv_range + ((size_t)bb * a.hkv + hk / a.kv_div) * FA_CHUNKS, *vr = kr + (size_t)a.b * a.hkv * FA_CHUNKS;
     const unsigned k_top = wave_umax(kr[c]), v_top = wave_umax(vr[c]);
     const int ek = row_exponent(k_top), ev = row_exponent(v_top);
     const float k_scale = exp2_int(ek), v_scale = exp2_int(ev);
@@ -141,7 +146,9 @@ __global__ __launch_bounds__(FA_THREADS, 2) void attn_prefill_f16x2_kernel(AttnP
     }
 
     const int q_last = min(q0 + BQ, a.s) - 1;
-    const int kmax = a.causal ? min(L, a.past_len + q_last + 1) : L;
+    const int kbeg = PART ? key_part * a.key_chunk : 0;
+    int kmax = a.causal ? min(L, a.past_len + q_last + 1) : L;
+    if (PART) kmax = min(kmax, kbeg + a.key_chunk);
     const int wave_i_last = min(q0 + (wave * 32 + 31) / NREP, a.s - 1);
     const int wave_kmax = a.causal ? min(L, a.past_len + wave_i_last + 1) : L;
     // keys [0, wave_kfull) are visible to every row of this wavefront: no mask needed below it
@@ -176,8 +183,8 @@ __global__ __launch_bounds__(FA_THREADS, 2) void attn_prefill_f16x2_kernel(AttnP
     };
 
     constexpr int PA_[3] = {1, 0, 0}, PB_[3] = {0, 1, 0};  // part products by ascending size: lo hi, hi lo, hi hi
-    if (kmax > 0) fetch(0);
-    for (int j0 = 0; j0 < kmax; j0 += KEYS) {
+    if (kmax > kbeg) fetch(kbeg);
+    for (int j0 = kbeg; j0 < kmax; j0 += KEYS) {
 #pragma unroll
         for (int p = 0; p < PIECES; ++p) {
             const int idx = tid + p * FA_THREADS;
@@ -286,13 +293,30 @@ __global__ __launch_bounds__(FA_THREADS, 2) void attn_prefill_f16x2_kernel(AttnP
         __syncthreads();
     }
 
+    if (PART) {
+        const float l = l_run + __shfl_xor(l_run, 32, 64);
+        const int i = q0 + my_row / NREP;
+        if (i < a.s) {
+            const size_t n = (((size_t)bb * a.s + i) * a.hq + (size_t)hk * NREP + my_row % NREP) * (gridDim.z / a.b) + key_part;
+            if (half == 0) {
+                a.part_ml[2 * n] = m_run;
+                a.part_ml[2 * n + 1] = l;
+            }
+#pragma unroll
+            for (int t = 0; t < DT; ++t)
+#pragma unroll
+                for (int g = 0; g < 4; ++g)
+                    *(v4f *)(a.part + n * D + 32 * t + 8 * g + 4 * half) = v4f{O[t][4 * g], O[t][4 * g + 1], O[t][4 * g + 2], O[t][4 * g + 3]};
+        }
+        return;
+    }
     // out = ctx / (sum + 1e-9), self_attention.rs:670-676; [B,S,Hq,D]
     const float inv = 1.0f / fmaf(l_run + __shfl_xor(l_run, 32, 64), exp2_int(-FA_P_EXP), 1e-9f);
     const float v_unit = ldexpf(1.0f, -(ev + FA_P_EXP));
     const int i = q0 + my_row / NREP;
     float o_scale = 0.f;
     if (a.out_exp) {  // (uniform) the rows go out split, all with the exponent of the largest value there is
-        const unsigned *all = a.kv_range + ((size_t)gridDim.z + bb) * a.hkv * FA_CHUNKS;
+        const unsigned *all = a.kv_range + ((size_t)a.b + bb) * a.hkv * FA_CHUNKS;
         unsigned m = 0;
         for (int n = lane; n < a.hkv * FA_CHUNKS; n += 64) m = max(m, all[n]);
         const int eo = row_exponent(wave_umax(m));
@@ -314,46 +338,106 @@ __global__ __launch_bounds__(FA_THREADS, 2) void attn_prefill_f16x2_kernel(AttnP
     }
 }
 
+// The parts of a row's keys together, in part order; a thread takes four elements of a (position, head) row.
+__global__ __launch_bounds__(256) void merge_parts_kernel(AttnPrefillArgs a, int parts) {
+    const int per_pos = a.hq * a.d / 4, bb = blockIdx.z, at = (int)(blockIdx.y * 256 + threadIdx.x);
+    const size_t pos = (size_t)bb * a.s + blockIdx.x;
+    const unsigned *vr = a.kv_range + ((size_t)a.b + bb) * a.hkv * FA_CHUNKS;
+    unsigned top = 0;
+    if (a.out_exp) {
+        for (int n = threadIdx.x & 63; n < a.hkv * FA_CHUNKS; n += 64) top = max(top, vr[n]);
+        top = wave_umax(top);
+        if (at == 0) a.out_exp[pos] = row_exponent(top);
+    }
+    if (at >= per_pos) return;
+    const int head = at * 4 / a.d, e = at * 4 % a.d, kv = head / (a.hq / a.hkv);
+    unsigned v_top = 0;
+    for (int n = 0; n < FA_CHUNKS; ++n) v_top = max(v_top, vr[kv * FA_CHUNKS + n]);
+    const size_t n0 = (pos * a.hq + head) * parts;
+    float m = -INFINITY;
+    for (int p = 0; p < parts; ++p) m = fmaxf(m, a.part_ml[2 * (n0 + p)]);
+    const float ref = m > -INFINITY ? m : 0.f;
+    float l = 0.f;
+    v4f o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+    for (int p = 0; p < parts; ++p) {
+        const float w = fast_exp2(a.part_ml[2 * (n0 + p)] - ref);
+        const v4f x = *(const v4f *)(a.part + (n0 + p) * a.d + e);
+        l = fmaf(w, a.part_ml[2 * (n0 + p) + 1], l);
+        o.x = fmaf(w, x.x, o.x); o.y = fmaf(w, x.y, o.y); o.z = fmaf(w, x.z, o.z); o.w = fmaf(w, x.w, o.w);
+    }
+    const float inv = 1.0f / fmaf(l, exp2_int(-FA_P_EXP), 1e-9f), unit = ldexpf(1.0f, -(row_exponent(v_top) + FA_P_EXP));
+    o = v4f{o.x * inv * unit, o.y * inv * unit, o.z * inv * unit, o.w * inv * unit};
+    float *row = a.out + pos * a.hq * a.d;
+    if (a.out_exp) store_split4((uint16_t *)row, at * 4, o, exp2_int(row_exponent(top)));
+    else *(v4f *)(row + at * 4) = o;
+}
+
+// Parts the keys are cut into where the blocks of queries leave compute units idle: at least 128 keys each (two trips of the loop; a part costs
+// its start and its share of the pass that merges them), two workgroups per compute unit, 32 at most.
+static int fa_key_parts(int num_cus, int blocks, int keys) {
+    const int room = 2 * num_cus / (blocks > 0 ? blocks : 1), most = (keys + 127) / 128;
+    const int n = room < most ? room : most;
+    return n < 2 ? 1 : n < 32 ? n : 32;
+}
+
 template <int D>
 static int launch_fa_d(lumen_ctx *ctx, const AttnPrefillArgs &a_in) {
     AttnPrefillArgs a = a_in;
-    const int nrep = a.hq / a.hkv;
-    const size_t need = 2 * (size_t)a.b * a.hkv * FA_CHUNKS * sizeof(unsigned);
-    if (need > ctx->kv_range_bytes) {
-        HIP_TRY(hipStreamSynchronize(ctx->stream));
-        hipFree(ctx->kv_range);
-        ctx->kv_range = nullptr;
-        ctx->kv_range_bytes = 0;
-        HIP_TRY(hipMalloc((void **)&ctx->kv_range, need));
-        ctx->kv_range_bytes = need;
+    int nrep = a.hq / a.hkv;
+    if (!(nrep == 1 || nrep == 2 || nrep == 4 || nrep == 8)) {  // any other group size: one query head per grid row, its KV head = head / n_rep
+        a.kv_div = nrep;
+        nrep = 1;
     }
-    a.kv_range = ctx->kv_range;
-    hipLaunchKernelGGL(kv_range_kernel, dim3(FA_CHUNKS, a.b * a.hkv), dim3(256), 0, ctx->stream, a.k_cache, a.v_cache, a.max_seq, D, a.past_len + a.s,
-                       ctx->kv_range);
-    dim3 block(FA_THREADS);
-#define LAUNCH_FA(NR)                                                                                    \
-    hipLaunchKernelGGL((attn_prefill_f16x2_kernel<D, NR, (D == 64 ? 2 : 1)>), dim3((a.s + FA_ROWS / NR - 1) / (FA_ROWS / NR), a.hkv, a.b), \
-                       block, 0, ctx->stream, a)
+    const int L = a.past_len + a.s, trip = FA_KEYS * (D == 64 ? 2 : 1);
+    dim3 grid((a.s + FA_ROWS / nrep - 1) / (FA_ROWS / nrep), a.hq / nrep, a.b);
+    int parts = fa_key_parts(ctx->num_cus, (int)(grid.x * grid.y * grid.z), L);
+    if (parts > 1) {
+        a.key_chunk = ((L + parts - 1) / parts + trip - 1) / trip * trip;
+        parts = (L + a.key_chunk - 1) / a.key_chunk;
+    }
+    const size_t rows = parts > 1 ? (size_t)a.b * a.s * a.hq * parts : 0, range = 2 * (size_t)a.b * a.hkv * FA_CHUNKS;
+    const size_t need = (range + rows * (D + 2)) * sizeof(float);
+    if (need > ctx->attn_ws_bytes) {
+        HIP_TRY(hipStreamSynchronize(ctx->stream));
+        hipFree(ctx->attn_ws);
+        ctx->attn_ws = nullptr;
+        ctx->attn_ws_bytes = 0;
+        HIP_TRY(hipMalloc((void **)&ctx->attn_ws, need));
+        ctx->attn_ws_bytes = need;
+    }
+    a.part = ctx->attn_ws;
+    a.part_ml = a.part + rows * D;
+    unsigned *kv_range = (unsigned *)(a.part_ml + 2 * rows);
+    a.kv_range = kv_range;
+    hipLaunchKernelGGL(kv_range_kernel, dim3(FA_CHUNKS, a.b * a.hkv), dim3(256), 0, ctx->stream, a.k_cache, a.v_cache, a.max_seq, D, L, kv_range);
+    grid.z *= parts;
+#define LAUNCH_FA(NR)                                                                                                                        \
+    do {                                                                                                                                     \
+        if (parts > 1) hipLaunchKernelGGL((attn_prefill_f16x2_kernel<D, NR, (D == 64 ? 2 : 1), true>), grid, dim3(FA_THREADS), 0, ctx->stream, a); \
+        else hipLaunchKernelGGL((attn_prefill_f16x2_kernel<D, NR, (D == 64 ? 2 : 1), false>), grid, dim3(FA_THREADS), 0, ctx->stream, a);     \
+    } while (0)
     switch (nrep) {
         case 1: LAUNCH_FA(1); break;
         case 2: LAUNCH_FA(2); break;
         case 4: LAUNCH_FA(4); break;
-        case 8: LAUNCH_FA(8); break;
-        default: {  // any other group size: one query head per grid row, its KV head = head / n_rep
-            AttnPrefillArgs b = a;
-            b.kv_div = nrep;
-            hipLaunchKernelGGL((attn_prefill_f16x2_kernel<D, 1, (D == 64 ? 2 : 1)>), dim3((a.s + FA_ROWS - 1) / FA_ROWS, a.hq, a.b), block, 0,
-                               ctx->stream, b);
-        }
+        default: LAUNCH_FA(8); break;
     }
 #undef LAUNCH_FA
+    if (parts > 1)
+        hipLaunchKernelGGL(merge_parts_kernel, dim3(a.s, (a.hq * D / 4 + 255) / 256, a.b), dim3(256), 0, ctx->stream, a, parts);
     LUMEN_CHECK_LAUNCH();
     return LUMEN_OK;
 }
 
-// Worth it from a few hundred positions on: below that the tile loop of the few workgroups is
-// longer than the row loop of one workgroup per position.
-bool attn_prefill_mfma_supported(const AttnPrefillArgs &a) { return (a.d == 64 || a.d == 128) && a.s >= 96; }
+// Against the row loop (one workgroup per position and head or two: its walk over the keys is a chain, and every position repeats it): from 96
+// positions on, where the cache is long, and where positions times keys are many.  Measured, row loop / this, us: 32 heads of 64, 4 KV heads,
+// 64 positions behind 301: 18.5 / 18.6, 32 behind 600: 18.8 / 18.0, 2 behind 1000: 18.4 / 17.0, 64 behind 2900: 102 / 28; 32 heads of 128, 32
+// KV heads, 64 behind 301: 40 / 25, 2 behind 600: 35 / 23, 2 behind 301: 14 / 20.
+bool attn_prefill_mfma_supported(const AttnPrefillArgs &a) {
+    const long L = (long)a.past_len + a.s;
+    return (a.d == 64 || a.d == 128) && (a.s >= 96 || L * a.d >= 64000 || (long)a.b * a.s * a.hq * (a.past_len + a.s / 2) * a.d >= 44000000);
+}
 
 int launch_attn_prefill_mfma(lumen_ctx *ctx, const AttnPrefillArgs &a) {
     if (a.d == 64) return launch_fa_d<64>(ctx, a);
