@@ -1016,6 +1016,18 @@ static bool gemm_stream_applies(const GemmArgs &a) {
     return aligned && a.K > 0 && a.K % (a.w_bf16 ? 8 : 4) == 0 && a.M > GEMM_SKINNY_MAX_M && a.M <= gemm_stream_max_rows(a.w_bf16) &&
            !(a.epi == EPI_SWIGLU && (a.N & 1));
 }
+// Where the exponents of W's rows are known: f16 pairs (gemm_f16x2_stream_kernel), with bf16-stored weights for three to 32 rows, with f32 weights for
+// 17 to 32 where W has 5 Mi of them (at 23 rows: 2560 x 2048 12.1 -> 10.3 us, but 2048 x 2048 10.8 -> 11.1 and 1024 x 3072 10.6 -> 14).  Up to 16 rows of
+// f32 weights the f32 instruction needs only one row tile and no splitting (11264 x 2048: 22-23 us against 27-29 on pairs); from 33 rows on the tile
+// kernels win (48 rows of bf16 weights, 12288 x 4096: 40 us there, 49 here).  Prompt passes before and after, ms: Llama-2-7B shape, 8 layers, bf16, 3
+// rows 1.51 -> 1.12, 17 1.55 -> 1.33, 32 1.63 -> 1.48; TinyLlama 17 rows 2.29 -> 2.01, 32 2.30 -> 2.11; Pinavik 2048 wide, bf16, 20 rows 2.22 -> 1.84.
+static bool stream_pairs_shape(int M, int N, int K, int w_bf16) {
+    return M > (w_bf16 ? GEMM_SKINNY_MAX_M : 16) && M <= GEMM_STREAM_MAX_M && K > 0 && K % 64 == 0 && (w_bf16 || (long)N * K >= 5L << 20);
+}
+static bool stream_pairs_apply(const GemmArgs &a) {
+    const bool aligned = (((uintptr_t)a.A | (uintptr_t)a.W) & 15) == 0;
+    return a.w_exp && !a.a_split && aligned && stream_pairs_shape(a.M, a.N, a.K, a.w_bf16) && !(a.epi == EPI_SWIGLU && (a.N & 1));
+}
 // Workgroups along K per column tile of 16: about three workgroups per compute unit over the chip, at least four
 // blocks of K per wavefront, 16 splits at most (the split sum takes that many).
 static int gemm_stream_splits(const lumen_ctx *ctx, const GemmArgs &a) {
@@ -1046,9 +1058,14 @@ size_t gemm_workspace_bytes(const lumen_ctx *ctx, int M, int N, int K, int w_bf1
     GemmArgs a = {};
     a.M = M; a.N = N; a.K = K; a.w_bf16 = w_bf16;
     if (M <= 0 || N <= 0 || K <= 0 || K % (w_bf16 ? 8 : 4)) return 0;
+    size_t pairs = 0;  // (whether W's exponents are known is the caller's)
+    if (stream_pairs_shape(M, N, K, w_bf16)) {
+        const int sp = gemm_f16x2_stream_splits(ctx->num_cus, M, N, K);
+        if (sp > 1) pairs = (size_t)sp * M * N * sizeof(float);
+    }
     if (M > GEMM_SKINNY_MAX_M && M <= gemm_stream_max_rows(w_bf16)) {  // (alignment is the caller's: assume the streaming kernel)
         const int st = gemm_stream_splits(ctx, a);
-        return st > 1 ? (size_t)st * M * N * sizeof(float) : 0;
+        return std::max(pairs, st > 1 ? (size_t)st * M * N * sizeof(float) : 0);
     }
     if (split && gemm_takes_split(M, K, w_bf16)) {  // (the larger of what the two ways to add the splits take)
         const int sp = std::max(gemm_split_plan(ctx->num_cus, M, N, K, w_bf16, false).splits, gemm_split_plan(ctx->num_cus, M, N, K, w_bf16, true).splits);
@@ -1056,7 +1073,7 @@ size_t gemm_workspace_bytes(const lumen_ctx *ctx, int M, int N, int K, int w_bf1
     }
     int splits = gemm_big_splits(ctx, a);
     if (splits <= 0) splits = gemm_splits(ctx, a);
-    return splits > 1 ? (size_t)splits * M * N * sizeof(float) : 0;
+    return std::max(pairs, splits > 1 ? (size_t)splits * M * N * sizeof(float) : 0);
 }
 
 template <int MS, bool BF16>
@@ -1151,13 +1168,14 @@ int launch_gemm(lumen_ctx *ctx, const GemmArgs &a) {
     }
     if (a.epi == EPI_SWIGLU && (a.N & 1)) LUMEN_FAIL(LUMEN_ERR_SHAPE, "SwiGLU epilogue needs an even column count, got %d", a.N);
     GemmArgs g = a;
-    const bool stream = gemm_stream_applies(a);
+    const bool pairs = stream_pairs_apply(a), stream = !pairs && gemm_stream_applies(a);
     const bool split = a.a_split && !stream && gemm_takes_split(a.M, a.K, a.w_bf16);
     SplitPlan plan = {};
     if (split) plan = gemm_split_plan(ctx->num_cus, a.M, a.N, a.K, a.w_bf16, a.keep_splits && a.splits_used && a.epi == EPI_STORE);
-    int splits = stream ? 0 : split ? plan.splits : gemm_big_splits(ctx, a);
+    int splits = stream || pairs ? 0 : split ? plan.splits : gemm_big_splits(ctx, a);
     const bool big = !split && splits > 0;
-    if (stream) splits = gemm_stream_splits(ctx, a);
+    if (pairs) splits = gemm_f16x2_stream_splits(ctx->num_cus, a.M, a.N, a.K);
+    else if (stream) splits = gemm_stream_splits(ctx, a);
     else if (split) {}
     else if (!big) splits = gemm_splits(ctx, a);
     if (splits > 1) {
@@ -1165,7 +1183,9 @@ int launch_gemm(lumen_ctx *ctx, const GemmArgs &a) {
         g.part = ctx->gemm_ws;
     }
     dim3 grid((a.N + BN - 1) / BN, (a.M + BM - 1) / BM, splits);
-    if (stream) {
+    if (pairs) {
+        launch_gemm_f16x2_stream(g, splits, ctx->stream);
+    } else if (stream) {
         if (a.w_bf16) {
             launch_gemm_stream<1, true>(g, splits, ctx->stream);
         } else {

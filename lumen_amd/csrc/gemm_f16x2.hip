@@ -241,6 +241,154 @@ __global__ __launch_bounds__(64 * WM * WN, (FI * FJ > 8 ? 1 : 2)) void gemm_f16x
     store_scaled_tiles<EPI, PARTIAL, FI, FJ>(a, acc, ae_tile, we_tile, bm, bn, wrow, wcol, lane);
 }
 
+// Few rows of A (f32 rows).  The product is bound by the weights, which are streamed once and go straight into operand registers: a lane takes
+// two 16-byte pieces (bf16 weights: one) of its row per 32 of K, whose four lanes complete 64 bytes of every row, splits them there and multiplies
+// them by v_mfma_f32_16x16x32_f16 with the MT row tiles of A.  A workgroup's four wavefronts take 16 columns of C each and share A: chunks of 128 of K
+// lie in LDS in operand order, split on their way in, every row of a wavefront's share (EB blocks of 32 k) with an exponent of its own, found as it
+// passes; the sums of a share are scaled and added in f32.  What bounds it: the loads in flight (four blocks of W per wavefront; eight cost the
+// occupancy what they gained: 4096 x 12288, bf16, 3 rows 24 -> 27 us, 23 rows of f32 spilled) and the barrier per chunk.  Before (the f32
+// instruction, 32 cycles per four of K instead of 32 or 48 per 32, or three bf16 products on whole tiles) and now, N x K, us:
+//     f32 weights, 23 rows:  11264 x 2048 38.6 -> 33    2048 x 5632 22.8 -> 20.2    2560 x 2048 12.1 -> 10.3    6144 x 1024 16.6 -> 14.7
+//     bf16, 3-32 rows:       12288 x 4096 38 -> 24-34   4096 x 4096 19 -> 13-16     22016 x 4096 72 -> 47-66    4096 x 11008 42 -> 27-35
+// Error against 64 bits before and now, relative to the root mean square of C (f32 weights; half as many or fewer sums are rounded):
+//     16 rows 11264 x 2048 4.1e-7 -> 1.4e-7    23 rows 2048 x 5632 2.9e-7 -> 1.5e-7    3 rows 1000 x 192 1.3e-7 -> 0.9e-7
+#define SF_BLOCKS 4  // blocks of 32 k in a chunk, and of W in flight per wavefront
+template <bool WBF16, int MT, int EPI, bool PARTIAL>
+__global__ __launch_bounds__(256, 3) void gemm_f16x2_stream_kernel(GemmArgs a) {
+    constexpr int PW = WBF16 ? 1 : 2, NPROD = WBF16 ? 2 : 3, WP = WBF16 ? 1 : 2;
+    constexpr int EB = MT;          // blocks of a wavefront's share of a chunk of A: MT tiles x 4 blocks over 4 wavefronts
+    constexpr int PIECES = 2 * MT;  // 16-byte pieces of A per thread and chunk
+    __shared__ __align__(16) uint16_t As[2][SF_BLOCKS][MT][2][64][8];  // [half][block][tile][part][operand lane]
+    __shared__ int ae[2][SF_BLOCKS / EB][MT][16];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int c = lane & 15, g = lane >> 4;
+    const int M = a.M, N = a.N, K = a.K;
+    const int bn = blockIdx.x * 64 + wave * 16;
+    const int blocks = K / 32, per = (blocks + (int)gridDim.z - 1) / (int)gridDim.z;
+    const int b0 = min((int)blockIdx.z * per, blocks), n = min(per, blocks - b0);
+    const int col = bn + c, wrow = min(col, N - 1);
+    const int we = a.w_exp[wrow];
+    const float ws = exp2_int(we);
+    const char *wp = (const char *)a.W + ((size_t)wrow * K + (size_t)b0 * 32) * (WBF16 ? 2 : 4) + g * 16;
+    // this wavefront's share of a chunk of A: tile share_t, blocks share_b .. share_b + EB - 1; piece p of lane (row c, g): k 4 (4 p + g) of it
+    const int share_t = MT == 2 ? wave >> 1 : 0, share_b = MT == 2 ? (wave & 1) * 2 : wave;
+    const float *ap = a.A + (size_t)min(share_t * 16 + c, M - 1) * K + (size_t)b0 * 32 + share_b * 32 + g * 4;
+
+    v4f sum[MT];
+#pragma unroll
+    for (int t = 0; t < MT; ++t) sum[t] = v4f{0.f, 0.f, 0.f, 0.f};
+    v4u vw[SF_BLOCKS][WP];
+    v4f va[PIECES];
+    auto fetch_w = [&](int slot, int d) {
+#pragma unroll
+        for (int i = 0; i < WP; ++i) vw[slot][i] = __builtin_nontemporal_load((const v4u *)(wp + (size_t)min(d, n - 1) * (WBF16 ? 64 : 128) + i * 64));
+    };
+    auto fetch_a = [&](int d) {  // (past the end: the last k of the range, multiplied by nothing)
+#pragma unroll
+        for (int p = 0; p < PIECES; ++p) {
+            const int k = min(d * 32 + share_b * 32 + p * 16 + g * 4, n * 32 - 4) - share_b * 32 - g * 4;
+            va[p] = *(const v4f *)(ap + k);
+        }
+    };
+    auto stage_a = [&](int half) {
+        unsigned m = 0;
+#pragma unroll
+        for (int p = 0; p < PIECES; ++p) m = max(m, magnitude_bits(va[p]));
+        m = max(m, (unsigned)__shfl_xor((int)m, 16, 64));
+        m = max(m, (unsigned)__shfl_xor((int)m, 32, 64));
+        const int e = row_exponent(m);
+        const float s = exp2_int(e);
+        if (g == 0) ae[half][share_b / EB][share_t][c] = e;
+#pragma unroll
+        for (int p = 0; p < PIECES; ++p) {
+            unsigned h0, l0, h1, l1;
+            split_pair(va[p].x, va[p].y, s, h0, l0);
+            split_pair(va[p].z, va[p].w, s, h1, l1);
+            // k 16 (p & 1) + 4 g of block share_b + p / 2.  An operand lane (row, q) holds k 4 q .. + 3 and 16 + 4 q .. + 3 (bf16 weights: 8 q .. + 7)
+            const int q = WBF16 ? (p & 1) * 2 + (g >> 1) : g, at = WBF16 ? (g & 1) * 4 : (p & 1) * 4;
+            *(v2u *)&As[half][share_b + p / 2][share_t][0][q * 16 + c][at] = v2u{h0, h1};
+            *(v2u *)&As[half][share_b + p / 2][share_t][1][q * 16 + c][at] = v2u{l0, l1};
+        }
+    };
+    if (n > 0) {
+#pragma unroll
+        for (int j = 0; j < SF_BLOCKS; ++j) fetch_w(j, j);
+        fetch_a(0);
+        stage_a(0);
+    }
+    __syncthreads();
+    int half = 0;
+    for (int d = 0; d < n; d += SF_BLOCKS, half ^= 1) {
+        fetch_a(d + SF_BLOCKS);
+#pragma unroll
+        for (int e0 = 0; e0 < SF_BLOCKS; e0 += EB) {
+            v4f acc[MT];
+#pragma unroll
+            for (int t = 0; t < MT; ++t) acc[t] = v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int j = e0; j < e0 + EB; ++j) {
+                if (d + j >= n) break;  // (uniform)
+                f16x8 wf[PW];
+                if (WBF16) {
+                    const unsigned src[4] = {vw[j][0].x, vw[j][0].y, vw[j][0].z, vw[j][0].w};
+                    unsigned dst[4];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const f16x2_t h = {(_Float16)fmaf(__uint_as_float(src[e] << 16), ws, 0.f), (_Float16)fmaf(__uint_as_float(src[e] & 0xffff0000u), ws, 0.f)};
+                        dst[e] = __builtin_bit_cast(unsigned, h);
+                    }
+                    wf[0] = __builtin_bit_cast(f16x8, v4u{dst[0], dst[1], dst[2], dst[3]});
+                } else {
+                    unsigned h[4], l[4];
+#pragma unroll
+                    for (int i = 0; i < 2; ++i) {
+                        const v4u w = vw[j][WP == 2 ? i : 0];
+                        split_pair(__uint_as_float(w.x), __uint_as_float(w.y), ws, h[2 * i], l[2 * i]);
+                        split_pair(__uint_as_float(w.z), __uint_as_float(w.w), ws, h[2 * i + 1], l[2 * i + 1]);
+                    }
+                    wf[0] = __builtin_bit_cast(f16x8, v4u{h[0], h[1], h[2], h[3]});
+                    wf[PW - 1] = __builtin_bit_cast(f16x8, v4u{l[0], l[1], l[2], l[3]});
+                }
+                fetch_w(j, d + j + SF_BLOCKS);
+                f16x8 af[MT][2];
+#pragma unroll
+                for (int t = 0; t < MT; ++t)
+#pragma unroll
+                    for (int p = 0; p < 2; ++p) af[t][p] = __builtin_bit_cast(f16x8, *(const v4u *)&As[half][j][t][p][lane][0]);
+                constexpr int PA_[3] = {1, 0, 0}, PW_[3] = {0, 1, 0};  // lo hi, hi lo, hi hi (bf16 weights: lo w, hi w)
+#pragma unroll
+                for (int q = 0; q < NPROD; ++q)
+#pragma unroll
+                    for (int t = 0; t < MT; ++t)
+                        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[t][WBF16 ? 1 - q : PA_[q]], wf[WBF16 ? 0 : PW_[q]], acc[t], 0, 0, 0);
+            }
+#pragma unroll
+            for (int t = 0; t < MT; ++t)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) sum[t][r] = fmaf(acc[t][r], exp2_int(-ae[half][e0 / EB][t][4 * g + r]), sum[t][r]);
+        }
+        if (d + SF_BLOCKS < n) stage_a(half ^ 1);
+        __syncthreads();
+    }
+    float *part = PARTIAL ? a.part + (size_t)blockIdx.z * M * N : nullptr;
+#pragma unroll
+    for (int t = 0; t < MT; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int row = t * 16 + 4 * g + r;
+            const float v = ldexpf(sum[t][r], -we);
+            if (PARTIAL) {
+                if (row < M && col < N) part[(size_t)row * N + col] = v;
+            } else if (EPI == EPI_SWIGLU) {
+                const float up = __shfl_xor(v, 1, 64);
+                if (!(col & 1) && row < M && col < N) a.C[(size_t)row * (N >> 1) + (col >> 1)] = v / (1.0f + expf(-v)) * up;
+            } else if (row < M && col < N) {
+                const size_t o = (size_t)row * N + col;
+                a.C[o] = (EPI == EPI_RESIDUAL) ? fmaf(a.alpha, v, a.residual[o]) : v;
+            }
+        }
+}
+
 // ------------------------------------------------------------------------------------------ exponents, split rows
 // One wavefront per row of W.
 template <bool BF16>
@@ -404,6 +552,45 @@ void launch_gemm_f16x2(const GemmArgs &a, const SplitPlan &p, hipStream_t s) {
         if (a.w_bf16) launch_f16x2<true, 2, 2, 2>(a, grid, s);
         else launch_f16x2<false, 2, 2, 4>(a, grid, s);
     }
+}
+
+// K ranges of the few-row kernel over gridDim.z: the number that costs least, in units of what a workgroup takes for 32 of K (about 0.6 us).  A
+// compute unit runs its workgroups side by side, bound by their loads, two more units go into a workgroup's start and end, and a unit with one
+// workgroup alone does not keep enough loads in flight; partial products are written and read again at about 5.4 MB per block.  Best counts measured and this rule: 2048 x
+// 11264 4, 4; 5632 x 2048 8, 8; 4096 x 12288 4, 4; 4096 x 4096 8, 8; 4096 x 22016 2, 2; 11008 x 4096 8, 8 (K x N).
+int gemm_f16x2_stream_splits(int num_cus, int M, int N, int K) {
+    const int tiles = (N + 63) / 64, blocks = K / 32;
+    int best = 1;
+    double least = 0;
+    for (int s = 1; s <= 16 && s <= blocks; ++s) {
+        const int per_cu = (int)(((long)tiles * s + num_cus - 1) / num_cus);
+        double t = per_cu * ((blocks + s - 1) / s + 2.0) * (per_cu == 1 ? 1.25 : 1.0);
+        if (s > 1) t += (double)s * M * N * 8 / 5.4e6;
+        if (s == 1 || t < least) {
+            best = s;
+            least = t;
+        }
+    }
+    return best;
+}
+
+template <bool BF16, int MT>
+static void launch_f16x2_stream(const GemmArgs &a, dim3 grid, hipStream_t s) {
+    if (grid.z > 1) {
+        hipLaunchKernelGGL((gemm_f16x2_stream_kernel<BF16, MT, EPI_STORE, true>), grid, dim3(256), 0, s, a);
+        return;
+    }
+    switch (a.epi) {
+        case EPI_STORE: hipLaunchKernelGGL((gemm_f16x2_stream_kernel<BF16, MT, EPI_STORE, false>), grid, dim3(256), 0, s, a); break;
+        case EPI_RESIDUAL: hipLaunchKernelGGL((gemm_f16x2_stream_kernel<BF16, MT, EPI_RESIDUAL, false>), grid, dim3(256), 0, s, a); break;
+        default: hipLaunchKernelGGL((gemm_f16x2_stream_kernel<BF16, MT, EPI_SWIGLU, false>), grid, dim3(256), 0, s, a); break;
+    }
+}
+void launch_gemm_f16x2_stream(const GemmArgs &a, int splits, hipStream_t s) {
+    const dim3 grid((a.N + 63) / 64, 1, splits);
+    if (!a.w_bf16) launch_f16x2_stream<false, 2>(a, grid, s);
+    else if (a.M <= 16) launch_f16x2_stream<true, 1>(a, grid, s);
+    else launch_f16x2_stream<true, 2>(a, grid, s);
 }
 
 LUMEN_DEFINE_WARM(gemm_f16x2)

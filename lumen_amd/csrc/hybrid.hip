@@ -1023,7 +1023,8 @@ static bool split_rows(const lumen_hybrid *m, int s, int K) {
 }
 static GemmArgs gemm_args(const lumen_hybrid *m, const float *A, const int *a_exp, const void *w, const int *w_exp, float *C, int M, int N, int K) {
     GemmArgs g = gemm_args(m, A, w, C, M, N, K);
-    if (a_exp) { g.a_split = (const uint16_t *)A; g.a_exp = a_exp; g.w_exp = w_exp; }
+    g.w_exp = w_exp;
+    if (a_exp) { g.a_split = (const uint16_t *)A; g.a_exp = a_exp; }
     return g;
 }
 // rows that only a product reads, split in place: their exponents, or null where the product takes f32 rows

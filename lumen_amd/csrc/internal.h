@@ -229,6 +229,8 @@ struct SplitPlan {
 };
 SplitPlan gemm_split_plan(int num_cus, int M, int N, int K, int w_bf16, bool sum_later);
 void launch_gemm_f16x2(const GemmArgs &a, const SplitPlan &p, hipStream_t s);
+int gemm_f16x2_stream_splits(int num_cus, int M, int N, int K);
+void launch_gemm_f16x2_stream(const GemmArgs &a, int splits, hipStream_t s);
 int launch_reduce_swiglu_split(lumen_ctx *ctx, const GemmArgs &a, int splits);
 int launch_gemm(lumen_ctx *ctx, const GemmArgs &a);
 int launch_gemm_grouped(lumen_ctx *ctx, const GemmArgs &a, int max_tiles);  // M: total rows

@@ -839,7 +839,8 @@ static int run_prefill(lumen_llama *m, const std::vector<int> &ids, float *logit
     const bool split = takes_split_rows(m, s);
     int *e_n = split ? m->p_exp : nullptr, *e_attn = split ? m->p_exp + s : nullptr, *e_act = split ? m->p_exp + 2 * (size_t)s : nullptr;
     auto split_input = [&](GemmArgs &g, const int *a_exp, const int *w_exp) {
-        if (split) { g.a_split = (const uint16_t *)g.A; g.a_exp = a_exp; g.w_exp = w_exp; }
+        g.w_exp = w_exp;
+        if (split) { g.a_split = (const uint16_t *)g.A; g.a_exp = a_exp; }
     };
     for (int l = 0; l < c.num_hidden_layers; ++l) {
         const LayerW &w = m->layers[l];

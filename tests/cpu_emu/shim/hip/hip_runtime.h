@@ -181,6 +181,35 @@ static inline V emu_mfma_32x32x16f16(A a, A b, V c) {
     return c;
 }
 #define __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, x, y, z) emu_mfma_32x32x16f16((a), (b), (c))
+// v_mfma_f32_16x16x32_f16: A[i][8 g + t] and B[8 g + t][j] in element t of lane (i or j) + 16 g, D[4 g + r][j] in element r of lane j + 16 g
+template <typename A, typename V>
+static inline V emu_mfma_16x16x32f16(A a, A b, V c) {
+    static_assert(sizeof(A) == 16, "eight f16 values");
+    const int lane = (int)(threadIdx.x & 63), j = lane & 15, g = lane >> 4;
+    uint32_t aw[4], bw[4];
+    memcpy(aw, &a, 16);
+    memcpy(bw, &b, 16);
+    auto half = [](uint32_t u, int odd) {
+        const uint16_t h = (uint16_t)(u >> (16 * odd));
+        _Float16 f;
+        memcpy(&f, &h, 2);
+        return (float)f;
+    };
+    float bk[32];
+    for (int k = 0; k < 32; k += 2) {
+        const uint32_t u = emu::wave_exchange(bw[(k & 7) / 2], (k >> 3) * 16 + j);
+        bk[k] = half(u, 0);
+        bk[k + 1] = half(u, 1);
+    }
+    for (int r = 0; r < 4; ++r)
+        for (int k = 0; k < 32; k += 2) {
+            const uint32_t u = emu::wave_exchange(aw[(k & 7) / 2], (k >> 3) * 16 + 4 * g + r);
+            c[r] = fmaf(half(u, 0), bk[k], c[r]);
+            c[r] = fmaf(half(u, 1), bk[k + 1], c[r]);
+        }
+    return c;
+}
+#define __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, x, y, z) emu_mfma_16x16x32f16((a), (b), (c))
 // v_mfma_f32_16x16x4_f32: D[i][j] = C[i][j] + sum over k < 4 of A[i][k] B[k][j]; lane l gives A[l % 16][l / 16] and
 // B[l / 16][l % 16] and holds D[4 (l / 16) + r][l % 16] in element r.  (The order of the four products inside the
 // instruction is the hardware's; results are compared to a tolerance.)

@@ -1,5 +1,5 @@
-"""GPU parity of the prompt products that run on f16 pairs (prompts of more than 32 rows, 47 with bf16-stored weights, inner sizes that
-are multiples of 64): row and column counts around the tiles' edges, one piece of K and many, rows of very different
+"""GPU parity of the prompt products that run on f16 pairs (prompts of more than 32 rows, 47 with bf16-stored weights, and of few rows, three to
+32 with bf16-stored weights and 17 to 32 with f32 ones; inner sizes that are multiples of 64): row and column counts around the tiles' edges, one piece of K and many, rows of very different
 magnitudes, rows of zeros and rows that are not finite, against the CPU oracle.
 
 Tolerance: the suite's 1e-4 of the largest logit for f32 weights, and the same for bf16-stored ones, whose values the oracle
@@ -46,6 +46,27 @@ def magnitudes(params, rng):
         elif "o_proj" in n or "down_proj" in n:
             a *= np.exp2(rng.integers(-30, 6, (len(a), 1))).astype(np.float32)
             a[5] = 0
+
+
+@pytest.mark.parametrize("bf16", [False, True], ids=["f32", "bf16"])
+@pytest.mark.parametrize("cfg,rows", [
+    (config(64, 64, 4, 2), (3, 17, 32)),                       # two blocks of K: half a chunk
+    (config(128, 192, 4, 1, vocab=257), (4, 16, 19)),          # columns that fill no tile
+    (config(320, 704, 5, 5), (3, 16, 17, 31)),                 # chunks of K that end early, K splits
+    (config(1024, 2824, 16, 4, layers=1), (3, 15, 18, 32)),    # (f32 weights: from 5 Mi of them on)
+    (config(64, 64, 4, 2, layers=1, vocab=81925), (17, 32)),
+], ids=["64", "128", "320", "1024", "vocab"])
+def test_prompts_of_few_rows(cfg, rows, bf16):
+    gpu, ora = build(cfg, bf16, magnitudes)
+    for s in rows:
+        ids = synth.make_tokens(s, cfg["vocab_size"], seed=s)
+        gpu.reset_kv_caches()
+        ora.reset()
+        got = gpu.forward(ids, all_rows=True)
+        rc, ref = ora.forward(ids)
+        assert rc == lo.LO_OK
+        for t in range(s):
+            assert max_rel(got[t], ref[t]) <= 1e-4, (s, t)
 
 
 @pytest.mark.parametrize("bf16", [False, True], ids=["f32", "bf16"])
