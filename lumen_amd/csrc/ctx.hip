@@ -99,7 +99,7 @@ extern "C" int lumen_ctx_set_stream(lumen_ctx *ctx, void *hip_stream) {
 }
 
 // after a synchronisation: did a bounded wait inside an operator-level launch run out?
-static int check_wait_flag(lumen_ctx *ctx) {
+int check_wait_flag(lumen_ctx *ctx) {
     if (!ctx->err_host || !*(volatile int *)ctx->err_host) return LUMEN_OK;
     *(volatile int *)ctx->err_host = 0;
     LUMEN_FAIL(LUMEN_ERR_HIP, "a workgroup gave up waiting for values handed over inside a launch; the results of the "

@@ -1,5 +1,6 @@
 // Dense C[M,N] = A[M,K] W[N,K]^T for the M > 1 (prompt prefill) branch of
-// ops::matmul::matmul, src/ops/matmul.rs:70-92, on the gfx950 matrix cores.
+// ops::matmul::matmul, src/ops/matmul.rs:70-92, on the gfx950 matrix cores.  (Where a caller
+// knows the exponents of the rows, as the models' prompt passes do: gemm_f16x2.hip.)
 //
 // The reference computes in f32.  The f32 matrix instruction (v_mfma_f32_32x32x2_f32) runs at 1/16
 // of the bf16 rate on this chip, so the product is taken on the bf16 matrix cores instead without
@@ -239,9 +240,9 @@ __global__ __launch_bounds__(256) void gemm_bf16x3_kernel(GemmArgs a) {
 // kernel were bank conflicts).
 //   F = 4: 256x256 output tile, all 256 accumulator registers of a wavefront, one workgroup per compute
 //          unit.  A 4x4 register tile reads half the LDS bytes per matrix instruction of a 2x2 one, which
-//          is what bounds gemm_bf16x3_kernel.  For thousands of prompt rows.
+//          is what bounds gemm_bf16x3_kernel.  For thousands of rows.
 //   F = 2: 128x128, two or three workgroups per compute unit: the tile grid and K splits of
-//          gemm_bf16x3_kernel, for shorter prompts with f32 weights.
+//          gemm_bf16x3_kernel, for fewer rows with f32 weights.
 #define GB_M 256  // the F = 4 tile
 #define GB_N 256
 #define GB_K 16   // slice depth of the pipelined kernel
@@ -574,7 +575,7 @@ __global__ __launch_bounds__(SK_THREADS) void gemm_skinny_kernel(GemmArgs a, int
     }
 }
 
-// Prompts of three to 32 rows (a chat turn's new tokens, the tail of a chunked prompt): the product is bound by the
+// Three to 32 rows (a chat turn's new tokens, the tail of a chunked prompt; where gemm_f16x2_stream_kernel does not take them): the product is bound by the
 // weights, and the tile kernels above take the same ~100 us per layer for 5 rows as for 128.  This kernel streams W once
 // and multiplies on the matrix cores without sharing anything between wavefronts: a wavefront owns 16 rows of W (a column
 // tile of C; N / 16 tiles spread evenly over the compute units where N / 32 would not) over a range of K and all

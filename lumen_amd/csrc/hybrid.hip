@@ -915,10 +915,10 @@ static int launch_step(lumen_hybrid *m) {
     return LUMEN_OK;
 }
 
-// after a synchronisation: did the arg-max tail's wait run into its limit?
-static int check_handover(lumen_hybrid *m) {
+// Waits for the work in flight, brings n words of src to the host and asks: did the arg-max tail's wait run into its limit?
+static int fetch_checked(lumen_hybrid *m, void *dst_host, const void *src, size_t n) {
     int err = 0;
-    HIP_TRY(hipMemcpy(&err, m->d_err, sizeof(int), hipMemcpyDeviceToHost));
+    LUMEN_TRY(fetch_words(m->ctx, dst_host, src, n, m->d_err, &err));
     if (!err) return LUMEN_OK;
     HIP_TRY(hipMemset(m->d_err, 0, sizeof(int)));
     LUMEN_FAIL(LUMEN_ERR_HIP, "decode: a workgroup gave up waiting for a value handed over inside a launch; the results of this call are invalid");
@@ -1279,7 +1279,8 @@ static int run_prompt(lumen_hybrid *m, const int32_t *ids, int s, const int *wan
         else LUMEN_TRY(launch_rmsnorm(ctx, m->p_rows, m->final_norm, m->p_n, n_want, W, m->eps_w));
         LUMEN_TRY(launch_gemm(ctx, gemm_args(m, m->p_n, m->head, m->p_logits, n_want, V, W)));
         if (c.logit_softcap > 0.f) LUMEN_TRY(launch_softcap(ctx, m->p_logits, c.logit_softcap, (size_t)n_want * V));
-        return lumen_download(ctx, logits_host, m->p_logits, sizeof(float) * (size_t)n_want * V);
+        LUMEN_TRY(fetch_words(ctx, logits_host, m->p_logits, (size_t)n_want * V, nullptr, nullptr));
+        return check_wait_flag(ctx);
     }
     // (nothing to bring back: the ids' upload must still be done before the caller's array goes)
     HIP_TRY(hipStreamSynchronize(ctx->stream));
@@ -1311,16 +1312,14 @@ extern "C" int lumen_hybrid_forward(lumen_hybrid *m, const int32_t *ids, int s, 
         if (n > 1) {
             LUMEN_TRY(run_prompt(m, ids + t, n, rows.data(), nw, lg, &tap));
         } else {
-            hipStream_t st = m->ctx->stream;
-            HIP_TRY(hipMemcpyAsync(m->d_tok, ids + t, sizeof(int), hipMemcpyHostToDevice, st));
-            HIP_TRY(hipStreamSynchronize(st));
+            LUMEN_TRY(launch_put_word(m->ctx, m->d_tok, ids[t]));
             if (residual_host) LUMEN_TRY(enqueue_decode_step(m, &tap));
             else LUMEN_TRY(launch_step(m));
             m->len += 1;
             m->step += 1;
             if (nw) {
-                LUMEN_TRY(lumen_download(m->ctx, lg, m->logits, sizeof(float) * (size_t)V));
-                LUMEN_TRY(check_handover(m));
+                LUMEN_TRY(fetch_checked(m, lg, m->logits, (size_t)V));
+                LUMEN_TRY(check_wait_flag(m->ctx));
             }
         }
         w += nw;
@@ -1339,8 +1338,7 @@ extern "C" int lumen_hybrid_decode_greedy(lumen_hybrid *m, int first_id, int n, 
     LUMEN_TRY(check_room(m, n));
     hipStream_t st = m->ctx->stream;
     const size_t V = (size_t)m->cfg.vocab_size;
-    HIP_TRY(hipMemcpyAsync(m->d_tok, &first, sizeof(int), hipMemcpyHostToDevice, st));
-    HIP_TRY(hipStreamSynchronize(st));
+    LUMEN_TRY(launch_put_word(m->ctx, m->d_tok, first));
     const int len0 = m->len;
     for (int t = 0; t < n; ++t) {
         LUMEN_TRY(launch_step(m));
@@ -1348,10 +1346,8 @@ extern "C" int lumen_hybrid_decode_greedy(lumen_hybrid *m, int first_id, int n, 
         m->step += 1;
         if (logits_out) HIP_TRY(hipMemcpyAsync(logits_out + (size_t)t * V, m->logits, sizeof(float) * V, hipMemcpyDeviceToHost, st));
     }
-    HIP_TRY(hipStreamSynchronize(st));
     // the arg-max tail leaves every pick at the index of the position it is the token of
-    if (ids_out) HIP_TRY(hipMemcpy(ids_out, m->tok_hist + len0 + 1, sizeof(int) * (size_t)n, hipMemcpyDeviceToHost));
-    return check_handover(m);
+    return fetch_checked(m, ids_out, m->tok_hist + len0 + 1, ids_out ? (size_t)n : 0);
 }
 
 extern "C" int lumen_hybrid_decode_profile(lumen_hybrid *m, int first_id, int n, double *ms_sum_out, int *count_out, int n_classes) {
@@ -1363,8 +1359,7 @@ extern "C" int lumen_hybrid_decode_profile(lumen_hybrid *m, int first_id, int n,
     HIP_TRY(hipSetDevice(m->ctx->device));
     LUMEN_TRY(check_room(m, n));
     hipStream_t st = m->ctx->stream;
-    HIP_TRY(hipMemcpyAsync(m->d_tok, &first, sizeof(int), hipMemcpyHostToDevice, st));
-    HIP_TRY(hipStreamSynchronize(st));
+    LUMEN_TRY(launch_put_word(m->ctx, m->d_tok, first));
     int rc = LUMEN_OK;
     for (int t = 0; t < n && rc == LUMEN_OK; ++t) {
         Probe probe;
@@ -1390,7 +1385,7 @@ extern "C" int lumen_hybrid_decode_profile(lumen_hybrid *m, int first_id, int n,
             lumen_set_error("hybrid_decode_profile step %d: %s", t, hipGetErrorString(e));
             rc = LUMEN_ERR_HIP;
         }
-        if (rc == LUMEN_OK) rc = check_handover(m);
+        if (rc == LUMEN_OK) rc = fetch_checked(m, nullptr, nullptr, 0);
     }
     return rc;
 }

@@ -241,6 +241,9 @@ __device__ __forceinline__ float expert_act(float g, float u, float limit) {
     return g / (1.0f + expf(-1.702f * g)) * (u + 1.0f);
 }
 int gemm_reserve_workspace(lumen_ctx *ctx, size_t bytes);  // grows the split-K workspace (synchronises the stream when it does)
+int check_wait_flag(lumen_ctx *ctx);
+int launch_put_word(lumen_ctx *ctx, int *dst, int v);
+int fetch_words(lumen_ctx *ctx, void *dst_host, const void *src, size_t n, const int *flag, int *flag_out);
 size_t gemm_workspace_bytes(const lumen_ctx *ctx, int M, int N, int K, int w_bf16, bool split = false);
 
 // One empty kernel per translation unit with kernels.  The runtime loads a translation unit's device code at the first

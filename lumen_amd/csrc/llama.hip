@@ -745,16 +745,19 @@ extern "C" int lumen_llama_get_decode_mode(const lumen_llama *m, int *mode_out) 
     return LUMEN_OK;
 }
 
-// after a synchronisation: did a wait inside the attention -> o_proj chain run into its limit?
-static int check_handover(lumen_llama *m) {
+// Waits for the work in flight, brings n words of src to the host and asks: did a wait inside the attention -> o_proj chain run into its limit?
+static int fetch_checked(lumen_llama *m, void *dst_host, const void *src, size_t n) {
     int err = 0;
-    HIP_TRY(hipMemcpy(&err, m->d_err, sizeof(int), hipMemcpyDeviceToHost));
+    LUMEN_TRY(fetch_words(m->ctx, dst_host, src, n, m->d_err, &err));
     if (!err) return LUMEN_OK;
     HIP_TRY(hipMemset(m->d_err, 0, sizeof(int)));
     LUMEN_FAIL(LUMEN_ERR_HIP, "decode: a workgroup gave up waiting for a value handed over inside a launch (poll "
                               "limit %u); the results of this call are invalid, reset the model", m->spin_limit);
 }
 
+// inside a pass, whose end waits for it
+static int set_device_pos(lumen_llama *m) { return launch_put_word(m->ctx, m->d_pos, m->len); }
+// by itself a copy is the shorter way: to launch a kernel on an idle stream and wait for it takes 20 us more
 static int sync_pos_to_device(lumen_llama *m) {
     HIP_TRY(hipMemcpyAsync(m->d_pos, &m->len, sizeof(int), hipMemcpyHostToDevice, m->ctx->stream));
     HIP_TRY(hipStreamSynchronize(m->ctx->stream));
@@ -898,16 +901,25 @@ static int run_prefill(lumen_llama *m, const std::vector<int> &ids, float *logit
         split_input(g, e_n, m->e_head);
         LUMEN_TRY(launch_gemm(ctx, g));
         m->len += s;
-        if (logits_host) LUMEN_TRY(lumen_download(ctx, logits_host, m->p_logits, sizeof(float) * (size_t)s * V));
+        LUMEN_TRY(set_device_pos(m));
+        if (logits_host) {
+            LUMEN_TRY(fetch_words(ctx, logits_host, m->p_logits, (size_t)s * V, nullptr, nullptr));
+            return check_wait_flag(ctx);
+        }
     } else {  // what its caller keeps, main.rs:155-163
         GemvArgs g = {};
         g.W = m->lm_head; g.x = m->p_x + (size_t)(s - 1) * H; g.y = m->logits; g.N = V; g.K = H; g.w_bf16 = head_bf16;
         g.pro = PRO_RMSNORM; g.norm_w = m->final_norm; g.eps = c.rms_norm_eps; g.epi = EPI_STORE;
         LUMEN_TRY(launch_gemv(ctx, g));
         m->len += s;
-        if (logits_host) LUMEN_TRY(lumen_download(ctx, logits_host, m->logits, sizeof(float) * (size_t)V));
+        LUMEN_TRY(set_device_pos(m));
+        if (logits_host) {
+            LUMEN_TRY(fetch_words(ctx, logits_host, m->logits, (size_t)V, nullptr, nullptr));
+            return check_wait_flag(ctx);
+        }
     }
-    return sync_pos_to_device(m);
+    HIP_TRY(hipStreamSynchronize(ctx->stream));
+    return LUMEN_OK;
 }
 
 extern "C" int lumen_llama_forward(lumen_llama *m, const float *ids_host, int s, float *logits_host, int all_rows) {
@@ -920,14 +932,12 @@ extern "C" int lumen_llama_forward(lumen_llama *m, const float *ids_host, int s,
     if (s > 1) return run_prefill(m, ids, logits_host, all_rows);
     // S == 1: the decode path (self_attention.rs:125)
     LUMEN_TRY(ensure_decode_graph(m));
-    hipStream_t st = m->ctx->stream;
-    HIP_TRY(hipMemcpyAsync(m->d_tok, ids.data(), sizeof(int), hipMemcpyHostToDevice, st));
-    HIP_TRY(hipStreamSynchronize(st));
+    LUMEN_TRY(launch_put_word(m->ctx, m->d_tok, ids[0]));
     HIP_TRY(launch_step(m));
     m->len += 1;
     if (logits_host) {
-        LUMEN_TRY(lumen_download(m->ctx, logits_host, m->logits, sizeof(float) * (size_t)m->cfg.vocab_size));
-        return check_handover(m);
+        LUMEN_TRY(fetch_checked(m, logits_host, m->logits, (size_t)m->cfg.vocab_size));
+        return check_wait_flag(m->ctx);
     }
     // (no logits wanted: the step stays in flight, and a wait that gave up inside it is reported by the next call
     // that synchronises -- lumen_llama_forward with logits, lumen_llama_decode_greedy, lumen_llama_decode_profile)
@@ -945,8 +955,7 @@ extern "C" int lumen_llama_decode_greedy(lumen_llama *m, int first_id, int n, in
     LUMEN_TRY(ensure_decode_graph(m));
     hipStream_t st = m->ctx->stream;
     const size_t V = (size_t)m->cfg.vocab_size;
-    HIP_TRY(hipMemcpyAsync(m->d_tok, &first_id, sizeof(int), hipMemcpyHostToDevice, st));
-    HIP_TRY(hipStreamSynchronize(st));
+    LUMEN_TRY(launch_put_word(m->ctx, m->d_tok, first_id));
     // the arg-max epilogue leaves every pick in tok_hist at the index of the position it is the token of
     const int len0 = m->len;
     int rc = LUMEN_OK;
@@ -964,11 +973,8 @@ extern "C" int lumen_llama_decode_greedy(lumen_llama *m, int first_id, int n, in
             m->len += 1;
         }
     }
-    hipError_t e = hipStreamSynchronize(st);
-    if (rc == LUMEN_OK && e == hipSuccess && ids_out)
-        e = hipMemcpy(ids_out, m->tok_hist + len0 + 1, sizeof(int) * (size_t)n, hipMemcpyDeviceToHost);
-    if (rc == LUMEN_OK && e != hipSuccess) LUMEN_FAIL(LUMEN_ERR_HIP, "decode_greedy: %s", hipGetErrorString(e));
-    if (rc == LUMEN_OK) rc = check_handover(m);
+    if (rc == LUMEN_OK) return fetch_checked(m, ids_out, m->tok_hist + len0 + 1, ids_out ? (size_t)n : 0);
+    (void)hipStreamSynchronize(st);
     return rc;
 }
 
@@ -986,8 +992,7 @@ extern "C" int lumen_llama_decode_profile(lumen_llama *m, int first_id, int n, d
     HIP_TRY(hipSetDevice(m->ctx->device));
     LUMEN_TRY(check_room(m, n));
     hipStream_t st = m->ctx->stream;
-    HIP_TRY(hipMemcpyAsync(m->d_tok, &first_id, sizeof(int), hipMemcpyHostToDevice, st));
-    HIP_TRY(hipStreamSynchronize(st));
+    LUMEN_TRY(launch_put_word(m->ctx, m->d_tok, first_id));
     int rc = LUMEN_OK;
     for (int t = 0; t < n && rc == LUMEN_OK; ++t) {
         StepProbe pr;
@@ -1014,7 +1019,7 @@ extern "C" int lumen_llama_decode_profile(lumen_llama *m, int first_id, int n, d
             lumen_set_error("decode_profile step %d: %s", t, hipGetErrorString(e));
             rc = LUMEN_ERR_HIP;
         }
-        if (rc == LUMEN_OK) rc = check_handover(m);  // (figures of a step whose wait gave up would mean nothing)
+        if (rc == LUMEN_OK) rc = fetch_checked(m, nullptr, nullptr, 0);  // (figures of a step whose wait gave up would mean nothing)
     }
     return rc;
 }
