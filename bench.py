@@ -25,8 +25,10 @@ if ROOT not in sys.path:
 HBM_PEAK_GBS = 8000.0  # MI355X published HBM3E bandwidth
 MFMA_FP32_PEAK_TF = 157.3  # MI355X dense fp32 matrix peak, TFLOP/s
 MFMA_BF16_PEAK_TF = 2500.0  # MI355X dense bf16 matrix peak, TFLOP/s
-# the prompt-pass GEMM takes an f32 product as six bf16 matrix products (three bf16 parts per f32 value)
+# the operator's GEMM takes an f32 product as six bf16 matrix products (three bf16 parts per f32 value), the models' prompt passes
+# as three f16 ones (pairs of f16, the same matrix rate)
 GEMM_BF16_PRODUCTS = 6
+PROMPT_F16_PRODUCTS = 3
 
 
 def main():
@@ -288,10 +290,10 @@ def prefill_report(cfg, S, ms):
     gemm_flops = 2.0 * S * L * per_layer + 2.0 * V * H
     attn_flops = 4.0 * L * hq * D * S * S / 2.0
     tf = (gemm_flops + attn_flops) / (ms * 1e-3) / 1e12
-    issued = (GEMM_BF16_PRODUCTS * gemm_flops) / (ms * 1e-3) / 1e12  # bf16 matrix flops the GEMMs issue
+    issued = (PROMPT_F16_PRODUCTS * gemm_flops) / (ms * 1e-3) / 1e12  # f16 matrix flops the GEMMs issue (bf16 rate)
     return {"tokens": S, "ms": round(ms, 3), "tokens_per_s": round(S / ms * 1e3, 1),
             "gemm_flops": gemm_flops, "attention_flops": attn_flops, "achieved_TFLOPs": round(tf, 2),
-            "matrix_path": "GEMM: f32 values as 3 bf16 parts, 6 v_mfma_f32_32x32x16_bf16 products per f32 product; "
+            "matrix_path": "GEMM: f32 values as 2 f16 parts with an exponent per row, 3 v_mfma_f32_32x32x16_f16 products per f32 product; "
                            "attention: the same scheme",
             "mfma_fp32_peak_TFLOPs": MFMA_FP32_PEAK_TF, "vs_mfma_fp32_peak": round(tf / MFMA_FP32_PEAK_TF, 4),
             "gemm_bf16_TFLOPs_issued": round(issued, 1), "mfma_bf16_peak_TFLOPs": MFMA_BF16_PEAK_TF,
