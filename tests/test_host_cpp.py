@@ -2,7 +2,7 @@
 
 tests/host_cpp/test_host.cpp holds the checks themselves (every one through the C ABI, compared with the
 CPU checker); this file compiles the header on its own, runs the device-free part here and the whole
-program on the GPU.  The program is built by tests/host_cpp/Makefile (and by __graft_entry__.build()).
+program on the GPU.  The program is built by tests/host_cpp/Makefile.
 """
 import os
 import subprocess
@@ -15,8 +15,7 @@ BINARY = os.path.join(HERE, "build", "test_host")
 
 
 def _binary():
-    if not os.path.exists(BINARY):
-        subprocess.run(["make", "-C", HERE], check=True, stdout=subprocess.DEVNULL)
+    subprocess.run(["make", "-C", HERE], check=True, stdout=subprocess.DEVNULL)
     return BINARY
 
 
