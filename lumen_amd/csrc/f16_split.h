@@ -1,6 +1,7 @@
 // An f32 value as two f16 values: x 2^e = hi + lo, e one exponent per row of an operand that takes the row's largest
-// magnitude into [2^14, 2^15).  hi carries 11 bits of x 2^e and lo the next 11 (12 with its sign), down to 2^-25 absolute: an
-// element up to 2^18 times smaller than its row's largest keeps its 22 to 23 bits, smaller ones an error of 2^-40 of that largest.
+// magnitude into [2^14, 2^15) (rows that stay below 2^-112 take ROW_EXP_MAX, which leaves them smaller).  hi carries 11 bits of x 2^e and lo
+// the next 11 (12 with its sign), down to 2^-25 absolute: an element up to 2^18 times smaller than its row's largest keeps its 22 to
+// 23 bits, smaller ones an error of 2^-40 of that largest.
 #pragma once
 
 #include "internal.h"
@@ -29,7 +30,19 @@ __device__ __forceinline__ unsigned magnitude_bits(const f32x4_t v) {
     return ab > cd ? ab : cd;
 }
 
-// (a, b) s -> two dwords of f16 pairs, s a power of two.  Both roundings are to nearest; x s and x s - hi are exact in f32.
+// Elements below this (bits), zeros aside, lose bits as pairs beside an element of magnitude `top_bits`.
+__device__ __forceinline__ unsigned small_limit(unsigned top_bits) {
+    const unsigned ex = top_bits >> 23;
+    return ex > 18 ? (ex - 18) << 23 : 1u;
+}
+__device__ __forceinline__ bool is_small(unsigned bits, unsigned limit) { return bits - 1u < limit - 1u; }
+
+// What holds too many small elements for pairs is multiplied by f32 matrix instructions; its exponent is marked.
+#define SPLIT_WIDE 1024
+__device__ __forceinline__ bool is_wide(int code) { return code > SPLIT_WIDE / 2; }
+__device__ __forceinline__ int code_exponent(int code) { return is_wide(code) ? code - SPLIT_WIDE : code; }
+
+// (a, b) s -> two dwords of f16 pairs.  Both roundings are to nearest; with s a power of two x s and x s - hi are exact in f32.
 __device__ __forceinline__ void split_pair(float a, float b, float s, unsigned &hi, unsigned &lo) {
     const f16x2_t h = {(_Float16)fmaf(a, s, 0.f), (_Float16)fmaf(b, s, 0.f)};
     const f16x2_t l = {(_Float16)fmaf(a, s, -(float)h.x), (_Float16)fmaf(b, s, -(float)h.y)};

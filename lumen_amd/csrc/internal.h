@@ -56,7 +56,7 @@ struct lumen_ctx {
     int *err_host = nullptr;
     float *gemm_ws = nullptr;      // split-K workspace of the prefill GEMM, grown on demand
     size_t gemm_ws_bytes = 0;
-    float *attn_ws = nullptr;      // a prompt attention's unfinished rows and its keys' and values' largest magnitudes, grown on demand
+    float *attn_ws = nullptr;      // a prompt attention's unfinished rows and the exponents of its tiles, grown on demand
     size_t attn_ws_bytes = 0;
     float *mixer_ws = nullptr;     // per-chunk operands of the recurrences, grown on demand
     size_t mixer_ws_bytes = 0;
@@ -406,9 +406,9 @@ struct AttnPrefillArgs {
     float norm_eps;
     float *q_rot;    // scratch [B, S, Hq, D]
     int *out_exp;    // not null: the rows of out are left split (f16_split.h) with their exponents here [B, S]
-    // set by the launcher: largest magnitudes of the cached keys and values; keys per part and the parts' unfinished rows [b s hq][parts][d] and
+    // set by the launcher: exponents of the tiles of cached keys and values; keys per part and the parts' unfinished rows [b s hq][parts][d] and
     // (maximum, sum) of theirs
-    const unsigned *kv_range;
+    const int *kv_tiles;
     int key_chunk;
     float *part, *part_ml;
     // q, k and v may arrive as in_splits partial sums (a GEMM's K splits), copy i at pointer + i * in_split_stride

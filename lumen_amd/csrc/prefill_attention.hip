@@ -10,12 +10,15 @@
 // cache serves all n_rep heads of the group and 128 / n_rep positions at once.
 //
 // The products run on the f16 matrix cores at f32 accuracy, as the prompt products of gemm_f16x2.hip do: every operand is the sum of two f16
-// values (f16_split.h), a product the three part products down to 2^-22, accumulated in f32 by v_mfma_f32_32x32x16_f16.  One
-// exponent serves the keys of a head and one its values (kv_range_kernel finds their largest magnitudes), every query has its own, a
-// softmax weight takes 2^14.  No output exceeds the largest value, so its exponent also serves the output rows where
-// the next product reads them split.
+// values (f16_split.h), a product the three part products down to 2^-22, accumulated in f32 by v_mfma_f32_32x32x16_f16.  A tile of
+// keys has one exponent for its keys and one for its values (kv_tiles_kernel), every query its own, and a lane keeps the sum of its row in the units
+// that its largest contribution so far -- weight times the tile's largest value -- asks for.  A tile in which some keys or channels are
+// 2^18 times smaller than others, which pairs cannot hold beside each other, or a query row of that kind, sends the workgroups that meet
+// it to f32 matrix instructions, from the f32 values: about three times slower, and met by no values of usual spread.
+// So the error of a row does not depend on the magnitude of keys that it does not see, nor on that of other tiles.
 // Bound by the matrix instructions and the softmax between them, which wait for each other within a wavefront; two per SIMD overlap.
-// With three bf16 parts: 420 us for 3968 positions of 32 heads of 64 (4 KV heads), with f16 pairs 286; 509 of 32 heads of 128: 61 -> 47.
+// With three bf16 parts: 420 us for 3968 positions of 32 heads of 64 (4 KV heads), with f16 pairs 305 (288 with one exponent for all keys of a
+// head, which is unsound); 509 of 32 heads of 128: 61 -> 47.
 // Few positions behind a long cache leave most compute units without a block of queries: the keys are then cut into parts (128 positions
 // behind 2900, 32 heads of 64: 111 us in one part, 33 in 16; 256 behind 2900, 16 heads of 128: 198 -> 56).
 //
@@ -33,14 +36,15 @@
 #include "attn_device.h"
 #include "f16_split.h"
 
+#include <type_traits>
+
 typedef float v16f __attribute__((ext_vector_type(16)));
 
 #define FA_ROWS 128  // (position, head) rows per workgroup
 #define FA_KEYS 32   // keys per tile
 #define FA_THREADS 256
 
-#define FA_CHUNKS 32  // parts a head's keys and values are searched in for their largest magnitude
-#define FA_P_EXP 14   // softmax weights are split as p 2^14
+#define FA_P_EXP 14  // the largest weight of a tile that counts is split as 2^14
 
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef unsigned int v4u __attribute__((ext_vector_type(4)));
@@ -55,31 +59,61 @@ __device__ __forceinline__ void fa_split4(const v4f x, float s, v2u (&part)[2]) 
     part[1] = v2u{l0, l1};
 }
 
-// Largest finite magnitude (bits) of each part of the L cached keys, and values, of a KV head: range [2][b hkv][FA_CHUNKS]
-__global__ __launch_bounds__(256) void kv_range_kernel(const float *k, const float *v, int max_seq, int d, int L, unsigned *range) {
+// Exponents (f16_split.h; marked where the tile takes f32 instructions) of the keys, and values, of each tile of KEYS of the L cached rows of a KV
+// head: tiles [2][b hkv][ceil(L / KEYS)].  Small elements that a tile may hold as pairs: fewer than FA_SMALL, which is less than a key's
+// or a channel's worth of them; 4096 normally distributed values hold 0.05.
+#define FA_SMALL 16
+template <int D, int KEYS>
+__global__ __launch_bounds__(256) void kv_tiles_kernel(const float *k, const float *v, int max_seq, int L, int *tiles) {
+    constexpr int PIECES = D * KEYS / 1024;
     __shared__ unsigned top[2][4];
-    const int tid = threadIdx.x, head = blockIdx.y;
-    const size_t base = (size_t)head * max_seq * d;
-    const int per = (L + FA_CHUNKS - 1) / FA_CHUNKS;
-    const size_t at = (size_t)min((int)blockIdx.x * per, L) * d, end = (size_t)min(((int)blockIdx.x + 1) * per, L) * d;
+    __shared__ float low[2][4];
+    const int tid = threadIdx.x, head = blockIdx.y, j0 = (int)blockIdx.x * KEYS;
+    const size_t base = ((size_t)head * max_seq + j0) * D;
+    v4f x[2][PIECES];
     unsigned m[2] = {0u, 0u};
-    for (size_t i = at + tid * 4; i < end; i += 1024) {
-        const v4f x[2] = {*(const v4f *)(k + base + i), *(const v4f *)(v + base + i)};
 #pragma unroll
-        for (int w = 0; w < 2; ++w)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const unsigned u = magnitude_bits(x[w][e]);
-                m[w] = max(m[w], u < 0x7f800000u ? u : 0u);
-            }
+    for (int p = 0; p < PIECES; ++p) {
+        const int at = (tid + p * 256) * 4;
+        const bool in = j0 + at / D < L;
+        x[0][p] = in ? *(const v4f *)(k + base + at) : v4f{0.f, 0.f, 0.f, 0.f};
+        x[1][p] = in ? *(const v4f *)(v + base + at) : v4f{0.f, 0.f, 0.f, 0.f};
     }
 #pragma unroll
     for (int w = 0; w < 2; ++w) {
+#pragma unroll
+        for (int p = 0; p < PIECES; ++p)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const unsigned u = magnitude_bits(x[w][p][e]);
+                m[w] = max(m[w], u < 0x7f800000u ? u : 0u);  // the largest finite one
+            }
         m[w] = wave_umax(m[w]);
         if ((tid & 63) == 0) top[w][tid >> 6] = m[w];
     }
     __syncthreads();
-    if (tid < 2) range[((size_t)tid * gridDim.y + head) * FA_CHUNKS + blockIdx.x] = max(max(top[tid][0], top[tid][1]), max(top[tid][2], top[tid][3]));
+#pragma unroll
+    for (int w = 0; w < 2; ++w) {
+        m[w] = max(max(top[w][0], top[w][1]), max(top[w][2], top[w][3]));
+        const unsigned limit = small_limit(m[w]);
+        int n = 0;
+#pragma unroll
+        for (int p = 0; p < PIECES; ++p)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const unsigned u = magnitude_bits(x[w][p][e]);
+                n += is_small(u, limit) ? 1 : u >= 0x7f800000u ? FA_SMALL : 0;
+            }
+        const float sum = wave_sum((float)n);
+        if ((tid & 63) == 0) low[w][tid >> 6] = sum;
+    }
+    __syncthreads();
+    if (tid < 2) {
+        const unsigned t = m[tid];
+        const int e = t ? row_exponent(t) : ROW_EXP_MAX;  // (zeros weigh nothing)
+        const bool wide = (low[tid][0] + low[tid][1]) + (low[tid][2] + low[tid][3]) >= (float)FA_SMALL;
+        tiles[((size_t)tid * gridDim.y + head) * gridDim.x + blockIdx.x] = wide ? e + SPLIT_WIDE : e;
+    }
 }
 
 // KT: key tiles of 32 per trip of the loop (2 for head_dim 64: one barrier pair, one row maximum and one rescale of
@@ -103,11 +137,8 @@ __global__ __launch_bounds__(FA_THREADS, 2) void attn_prefill_f16x2_kernel(AttnP
     const int q0 = (int)(gridDim.x - 1 - blockIdx.x) * BQ, hk = blockIdx.y, bb = PART ? (int)blockIdx.z % a.b : (int)blockIdx.z;
     const int key_part = PART ? (int)blockIdx.z / a.b : 0;
     const int L = a.past_len + a.s;
-    // exponents of this head's keys and values; of all heads' values, which no output exceeds
-    const unsigned *kr = a.kv_range + ((size_t)bb * a.hkv + hk / a.kv_div) * FA_CHUNKS, *vr = kr + (size_t)a.b * a.hkv * FA_CHUNKS;
-    const unsigned k_top = wave_umax(kr[c]), v_top = wave_umax(vr[c]);
-    const int ek = row_exponent(k_top), ev = row_exponent(v_top);
-    const float k_scale = exp2_int(ek), v_scale = exp2_int(ev);
+    const int n_tiles = (L + KEYS - 1) / KEYS;
+    const int *ktab = a.kv_tiles + ((size_t)bb * a.hkv + hk / a.kv_div) * n_tiles, *vtab = ktab + (size_t)a.b * a.hkv * n_tiles;
     const size_t head_base = ((size_t)bb * a.hkv + hk / a.kv_div) * a.max_seq * D;  // kv_div > 1: grid row = query head
     const float *Kc = a.k_cache + head_base, *Vc = a.v_cache + head_base;
 
@@ -115,36 +146,6 @@ __global__ __launch_bounds__(FA_THREADS, 2) void attn_prefill_f16x2_kernel(AttnP
     const int my_row = wave * 32 + c;
     const int my_i = min(q0 + my_row / NREP, a.s - 1);  // clamped: rows past S are computed and dropped
     const int my_pos = a.past_len + q0 + my_row / NREP;  // absolute position: keys up to it are visible
-    const float *qrow = a.q_rot + (((size_t)bb * a.s + my_i) * a.hq + (size_t)hk * NREP + my_row % NREP) * D;
-    const float qf_scale = a.scale * LUMEN_LOG2E;
-    // Q as the B operand of S^T = K Q^T: lane (column c, half g) holds elements ks * 16 + g * 8 .. + 7 of its row
-    v4u qp[D / 16][2];
-    float s_unit;  // what an accumulated score is to be multiplied by
-    {
-        v4f x[D / 16][2];
-        unsigned m = 0;
-#pragma unroll
-        for (int ks = 0; ks < D / 16; ++ks)
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                x[ks][h] = *(const v4f *)(qrow + ks * 16 + half * 8 + h * 4);
-                x[ks][h].x *= qf_scale; x[ks][h].y *= qf_scale; x[ks][h].z *= qf_scale; x[ks][h].w *= qf_scale;
-                m = max(m, magnitude_bits(x[ks][h]));
-            }
-        m = max(m, (unsigned)__shfl_xor((int)m, 32, 64));
-        const int eq = row_exponent(m);
-        const float q_scale = exp2_int(eq);
-        s_unit = ldexpf(1.0f, -(ek + eq));
-#pragma unroll
-        for (int ks = 0; ks < D / 16; ++ks) {
-            v2u lo[2], hi[2];
-            fa_split4(x[ks][0], q_scale, lo);
-            fa_split4(x[ks][1], q_scale, hi);
-#pragma unroll
-            for (int p = 0; p < 2; ++p) qp[ks][p] = (v4u){lo[p].x, lo[p].y, hi[p].x, hi[p].y};
-        }
-    }
-
     const int q_last = min(q0 + BQ, a.s) - 1;
     const int kbeg = PART ? key_part * a.key_chunk : 0;
     int kmax = a.causal ? min(L, a.past_len + q_last + 1) : L;
@@ -153,14 +154,6 @@ __global__ __launch_bounds__(FA_THREADS, 2) void attn_prefill_f16x2_kernel(AttnP
     const int wave_kmax = a.causal ? min(L, a.past_len + wave_i_last + 1) : L;
     // keys [0, wave_kfull) are visible to every row of this wavefront: no mask needed below it
     const int wave_kfull = a.causal ? min(L, a.past_len + q0 + (wave * 32) / NREP + 1) : L;
-
-    // O^T: register r of tile t belongs to element 32 t + 8 (r / 4) + 4 half + r % 4 of this lane's row
-    v16f O[DT];
-#pragma unroll
-    for (int t = 0; t < DT; ++t)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) O[t][r] = 0.f;
-    float m_run = -INFINITY, l_run = 0.f;  // of this lane's row; l, times 2^14, over this lane's half of the keys
 
     // V^T is staged with bits 2 and 3 of the key index exchanged: the 8 keys a lane holds of S^T (4 + 4,
     // eight apart) then sit next to each other for the 16-byte operand read.  A thread takes 4 elements
@@ -182,121 +175,243 @@ __global__ __launch_bounds__(FA_THREADS, 2) void attn_prefill_f16x2_kernel(AttnP
         }
     };
 
-    constexpr int PA_[3] = {1, 0, 0}, PB_[3] = {0, 1, 0};  // part products by ascending size: lo hi, hi lo, hi hi
-    if (kmax > kbeg) fetch(kbeg);
-    for (int j0 = kbeg; j0 < kmax; j0 += KEYS) {
+    // pairs or f32 instructions: one choice for all of this workgroup's tiles (a choice per tile keeps both forms' registers alive at once)
+    int first_k = 0, first_v = 0, tile_wide = 0;
+    if (kmax > kbeg) {
+        fetch(kbeg);
+        first_k = ktab[kbeg / KEYS];
+        first_v = vtab[kbeg / KEYS];
+    }
+    for (int t = kbeg / KEYS + tid; t < (kmax + KEYS - 1) / KEYS; t += FA_THREADS) tile_wide |= is_wide(ktab[t]) || is_wide(vtab[t]);
+    const float *qrow = a.q_rot + (((size_t)bb * a.s + my_i) * a.hq + (size_t)hk * NREP + my_row % NREP) * D;
+    const float qf_scale = a.scale * LUMEN_LOG2E;
+    // Q as the B operand of S^T = K Q^T: lane (column c, half g) holds elements ks * 16 + g * 8 .. + 7 of its row
+    __shared__ int wide_any[FA_THREADS / 64];
+    v4f x[D / 16][2];
+    int eq;
+    float q_scale;
+    bool q_wide;
+    {
+        unsigned m = 0;
 #pragma unroll
-        for (int p = 0; p < PIECES; ++p) {
-            const int idx = tid + p * FA_THREADS;
-            const int key = idx / (D / 4), k4 = (idx % (D / 4)) * 4;
-            v2u kp[2];
-            fa_split4(kreg[p], k_scale, kp);
+        for (int ks = 0; ks < D / 16; ++ks)
 #pragma unroll
-            for (int q = 0; q < 2; ++q) *(v2u *)&Ks[q][key][k4] = kp[q];
-        }
+            for (int h = 0; h < 2; ++h) {
+                x[ks][h] = *(const v4f *)(qrow + ks * 16 + half * 8 + h * 4);
+                x[ks][h].x *= qf_scale; x[ks][h].y *= qf_scale; x[ks][h].z *= qf_scale; x[ks][h].w *= qf_scale;
+                m = max(m, magnitude_bits(x[ks][h]));
+            }
+        m = max(m, (unsigned)__shfl_xor((int)m, 32, 64));
+        eq = row_exponent(m);
+        q_scale = exp2_int(eq);
+        const unsigned limit = small_limit(m);
+        int small = 0;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            v2u vp[2];
-            fa_split4((v4f){vreg[0][e], vreg[1][e], vreg[2][e], vreg[3][e]}, v_scale, vp);
+        for (int ks = 0; ks < D / 16; ++ks)
 #pragma unroll
-            for (int q = 0; q < 2; ++q) *(v2u *)&Vt[q][v_k4 + e][4 * v_g] = vp[q];
-        }
-        __syncthreads();
-        if (j0 + KEYS < kmax) fetch(j0 + KEYS);  // in flight during the matrix instructions below
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) small += is_small(magnitude_bits(x[ks][h][e]), limit);
+        small += __shfl_xor(small, 32, 64);
+        q_wide = small > D / 32 || m >= 0x7f800000u;
+    }
+    {
+        const int any = __any(q_wide || tile_wide);
+        if (lane == 0) wide_any[wave] = any;
+    }
+    __syncthreads();
+    const bool wide = (wide_any[0] | wide_any[1] | wide_any[2] | wide_any[3]) != 0;
 
-        if (j0 < wave_kmax) {  // uniform per wavefront: tiles wholly above the causal diagonal are skipped
-            // S^T = K Q^T: register r of tile kt holds key 32 kt + 8 (r / 4) + 4 half + r % 4 against this lane's row
-            v16f S[KT];
-#pragma unroll
-            for (int kt = 0; kt < KT; ++kt)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) S[kt][r] = 0.f;
+    auto rows = [&](auto form) {
+        constexpr bool WIDE = decltype(form)::value;
+        constexpr int PA_[3] = {1, 0, 0}, PB_[3] = {0, 1, 0};  // part products by ascending size: lo hi, hi lo, hi hi
+        v4u qp[D / 16][2];
+        if (!WIDE) {
 #pragma unroll
             for (int ks = 0; ks < D / 16; ++ks) {
-                f16x8 kf[KT][2];
+                v2u lo[2], hi[2];
+                fa_split4(x[ks][0], q_scale, lo);
+                fa_split4(x[ks][1], q_scale, hi);
 #pragma unroll
-                for (int kt = 0; kt < KT; ++kt)
-#pragma unroll
-                    for (int p = 0; p < 2; ++p)
-                        kf[kt][p] = __builtin_bit_cast(f16x8, *(const v4u *)&Ks[p][32 * kt + c][ks * 16 + half * 8]);
-#pragma unroll
-                for (int q = 0; q < 3; ++q)
-#pragma unroll
-                    for (int kt = 0; kt < KT; ++kt)
-                        S[kt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[kt][PA_[q]], __builtin_bit_cast(f16x8, qp[ks][PB_[q]]), S[kt], 0, 0, 0);
+                for (int p = 0; p < 2; ++p) qp[ks][p] = (v4u){lo[p].x, lo[p].y, hi[p].x, hi[p].y};
             }
-
-            // softmax of this lane's row, in the lane: half of the trip's keys here, half in lane ^ 32
-            float sc[16 * KT];
-            float m_tile = -INFINITY;
-            if (j0 + KEYS <= wave_kfull) {  // uniform per wavefront: every key of the trip is visible to every row
+        }
+        // O^T: register r of tile t belongs to element 32 t + 8 (r / 4) + 4 half + r % 4 of this lane's row
+        v16f O[DT];
 #pragma unroll
-                for (int kt = 0; kt < KT; ++kt)
+        for (int t = 0; t < DT; ++t)
 #pragma unroll
-                    for (int r = 0; r < 16; ++r) {
-                        sc[16 * kt + r] = S[kt][r] * s_unit;
-                        m_tile = fmaxf(m_tile, sc[16 * kt + r]);
-                    }
+            for (int r = 0; r < 16; ++r) O[t][r] = 0.f;
+        float m_run = -INFINITY, l_run = 0.f;  // of this lane's row; l over this lane's half of the keys
+        float o_run = -INFINITY;               // log2 of the largest contribution to O so far; O is in units of 2^(o_run - FA_P_EXP)
+        // f32 instructions read [key][element] and [element][key], in the bytes of Ks and Vt
+        float *Kf = (float *)&Ks[0][0][0], *Vf = (float *)&Vt[0][0][0];
+        int k_code = first_k, v_code = first_v;
+        for (int j0 = kbeg; j0 < kmax; j0 += KEYS) {
+            const int ek = code_exponent(k_code), ev = code_exponent(v_code);
+            const float k_scale = exp2_int(ek), v_scale = exp2_int(ev);
+            if (!WIDE) {
+#pragma unroll
+                for (int p = 0; p < PIECES; ++p) {
+                    const int idx = tid + p * FA_THREADS;
+                    const int key = idx / (D / 4), k4 = (idx % (D / 4)) * 4;
+                    v2u kp[2];
+                    fa_split4(kreg[p], k_scale, kp);
+#pragma unroll
+                    for (int q = 0; q < 2; ++q) *(v2u *)&Ks[q][key][k4] = kp[q];
+                }
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    v2u vp[2];
+                    fa_split4((v4f){vreg[0][e], vreg[1][e], vreg[2][e], vreg[3][e]}, v_scale, vp);
+#pragma unroll
+                    for (int q = 0; q < 2; ++q) *(v2u *)&Vt[q][v_k4 + e][4 * v_g] = vp[q];
+                }
             } else {
 #pragma unroll
+                for (int p = 0; p < PIECES; ++p) {
+                    const int idx = tid + p * FA_THREADS;
+                    const int key = idx / (D / 4), k4 = (idx % (D / 4)) * 4;
+                    *(v4f *)(Kf + key * LDK + k4) = (v4f){kreg[p].x * k_scale, kreg[p].y * k_scale, kreg[p].z * k_scale, kreg[p].w * k_scale};
+                }
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    *(v4f *)(Vf + (v_k4 + e) * LDV + v_key) =
+                        (v4f){vreg[0][e] * v_scale, vreg[1][e] * v_scale, vreg[2][e] * v_scale, vreg[3][e] * v_scale};
+            }
+            __syncthreads();
+            if (j0 + KEYS < kmax) {  // in flight during the matrix instructions below
+                fetch(j0 + KEYS);
+                k_code = ktab[j0 / KEYS + 1];
+                v_code = vtab[j0 / KEYS + 1];
+            }
+
+            if (j0 < wave_kmax) {  // uniform per wavefront: tiles wholly above the causal diagonal are skipped
+                // S^T = K Q^T: register r of tile kt holds key 32 kt + 8 (r / 4) + 4 half + r % 4 against this lane's row
+                v16f S[KT];
+#pragma unroll
                 for (int kt = 0; kt < KT; ++kt)
 #pragma unroll
-                    for (int r = 0; r < 16; ++r) {
-                        const int j = j0 + 32 * kt + 8 * (r >> 2) + 4 * half + (r & 3);
-                        const bool valid = j < L && (!a.causal || j <= my_pos);
-                        sc[16 * kt + r] = valid ? S[kt][r] * s_unit : -INFINITY;
-                        m_tile = fmaxf(m_tile, sc[16 * kt + r]);
+                    for (int r = 0; r < 16; ++r) S[kt][r] = 0.f;
+                if (WIDE) {  // instruction w of eight elements: element 4 half + w of both operands
+#pragma unroll 1
+                    for (int e8 = 0; e8 < D; e8 += 8) {
+                        v4f qx = *(const v4f *)(qrow + e8 + 4 * half), kx[KT];
+                        qx.x *= qf_scale; qx.y *= qf_scale; qx.z *= qf_scale; qx.w *= qf_scale;
+#pragma unroll
+                        for (int kt = 0; kt < KT; ++kt) kx[kt] = *(const v4f *)(Kf + (32 * kt + c) * LDK + e8 + 4 * half);
+#pragma unroll
+                        for (int w = 0; w < 4; ++w)
+#pragma unroll
+                            for (int kt = 0; kt < KT; ++kt) S[kt] = __builtin_amdgcn_mfma_f32_32x32x2f32(kx[kt][w], qx[w] * q_scale, S[kt], 0, 0, 0);
                     }
-            }
-            m_tile = fmaxf(m_tile, __shfl_xor(m_tile, 32, 64));
-            const float m_new = fmaxf(m_run, m_tile);
-            const float m_ref = m_new > -INFINITY ? m_new : 0.f;  // nothing visible yet: every weight below is exp2(-inf) = 0
-            const float alpha = fast_exp2(m_run - m_ref);
-            m_run = m_new;
-            float psum = 0.f;
+                } else
 #pragma unroll
-            for (int r = 0; r < 16 * KT; ++r) {
-                sc[r] = fast_exp2(sc[r] - (m_ref - FA_P_EXP));
-                psum += sc[r];
-            }
-            l_run = fmaf(l_run, alpha, psum);
+                for (int ks = 0; ks < D / 16; ++ks) {
+                    f16x8 kf[KT][2];
 #pragma unroll
-            for (int t = 0; t < DT; ++t)
+                    for (int kt = 0; kt < KT; ++kt)
 #pragma unroll
-                for (int r = 0; r < 16; ++r) O[t][r] *= alpha;
-
-            // O^T += V^T P^T: P^T is this lane's weights, already where the B operand wants them
-            // (registers 8 ks .. 8 ks + 7 are the keys at positions 16 ks + 8 half .. + 7 of V^T)
+                        for (int p = 0; p < 2; ++p)
+                            kf[kt][p] = __builtin_bit_cast(f16x8, *(const v4u *)&Ks[p][32 * kt + c][ks * 16 + half * 8]);
 #pragma unroll
-            for (int ks = 0; ks < KEYS / 16; ++ks) {
-                f16x8 pf[2];
-                {
-                    v2u lo[2], hi[2];
-                    fa_split4((v4f){sc[8 * ks], sc[8 * ks + 1], sc[8 * ks + 2], sc[8 * ks + 3]}, 1.0f, lo);
-                    fa_split4((v4f){sc[8 * ks + 4], sc[8 * ks + 5], sc[8 * ks + 6], sc[8 * ks + 7]}, 1.0f, hi);
+                    for (int q = 0; q < 3; ++q)
 #pragma unroll
-                    for (int p = 0; p < 2; ++p) pf[p] = __builtin_bit_cast(f16x8, (v4u){lo[p].x, lo[p].y, hi[p].x, hi[p].y});
+                        for (int kt = 0; kt < KT; ++kt)
+                            S[kt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[kt][PA_[q]], __builtin_bit_cast(f16x8, qp[ks][PB_[q]]), S[kt], 0, 0, 0);
                 }
-                f16x8 vf[DT][2];
+
+                // what an accumulated score is to be multiplied by (the bounds: a score that f32 does not hold, or that is next to nothing)
+                const float s_unit = exp2_int(min(max(-(ek + eq), -ROW_EXP_MAX), ROW_EXP_MAX));
+                // softmax of this lane's row, in the lane: half of the trip's keys here, half in lane ^ 32
+                float sc[16 * KT];
+                float m_tile = -INFINITY;
+                if (j0 + KEYS <= wave_kfull) {  // uniform per wavefront: every key of the trip is visible to every row
+#pragma unroll
+                    for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+                        for (int r = 0; r < 16; ++r) {
+                            sc[16 * kt + r] = S[kt][r] * s_unit;
+                            m_tile = fmaxf(m_tile, sc[16 * kt + r]);
+                        }
+                } else {
+#pragma unroll
+                    for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+                        for (int r = 0; r < 16; ++r) {
+                            const int j = j0 + 32 * kt + 8 * (r >> 2) + 4 * half + (r & 3);
+                            const bool valid = j < L && (!a.causal || j <= my_pos);
+                            sc[16 * kt + r] = valid ? S[kt][r] * s_unit : -INFINITY;
+                            m_tile = fmaxf(m_tile, sc[16 * kt + r]);
+                        }
+                }
+                m_tile = fmaxf(m_tile, __shfl_xor(m_tile, 32, 64));
+                const float m_new = fmaxf(m_run, m_tile);
+                const float m_ref = m_new > -INFINITY ? m_new : 0.f;  // nothing visible yet: every weight below is exp2(-inf) = 0
+                const float alpha = fast_exp2(m_run - m_ref);
+                m_run = m_new;
+                float psum = 0.f;
+#pragma unroll
+                for (int r = 0; r < 16 * KT; ++r) {
+                    sc[r] = fast_exp2(sc[r] - m_ref);
+                    psum += sc[r];
+                }
+                l_run = fmaf(l_run, alpha, psum);
+                // the tile's largest contribution is 2^(m_tile - ev), times a value's 2^15; its weight goes in as 2^FA_P_EXP or less
+                const float o_new = fmaxf(o_run, m_tile - (float)ev), o_ref = o_new > -INFINITY ? o_new : 0.f;
+                const float o_alpha = fast_exp2(o_run - o_ref), p_scale = fast_exp2(fminf(m_ref - (o_ref + (float)(ev - FA_P_EXP)), 120.f));
+                o_run = o_new;
 #pragma unroll
                 for (int t = 0; t < DT; ++t)
 #pragma unroll
-                    for (int p = 0; p < 2; ++p)
-                        vf[t][p] = __builtin_bit_cast(f16x8, *(const v4u *)&Vt[p][32 * t + c][ks * 16 + half * 8]);
+                    for (int r = 0; r < 16; ++r) O[t][r] *= o_alpha;
+
+                // O^T += V^T P^T: P^T is this lane's weights, already where the B operand wants them
+                // (registers 8 ks .. 8 ks + 7 are the keys at positions 16 ks + 8 half .. + 7 of V^T)
+                if (WIDE) {
 #pragma unroll
-                for (int q = 0; q < 3; ++q)
+                    for (int g = 0; g < 4 * KT; ++g) {  // registers 4 g .. 4 g + 3: keys 8 g + 4 half .. + 3
+                        v4f vx[DT];
+#pragma unroll
+                        for (int t = 0; t < DT; ++t) vx[t] = *(const v4f *)(Vf + (32 * t + c) * LDV + 8 * g + 4 * half);
+#pragma unroll
+                        for (int w = 0; w < 4; ++w)
+#pragma unroll
+                            for (int t = 0; t < DT; ++t) O[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(vx[t][w], sc[4 * g + w] * p_scale, O[t], 0, 0, 0);
+                    }
+                } else
+#pragma unroll
+                for (int ks = 0; ks < KEYS / 16; ++ks) {
+                    f16x8 pf[2];
+                    {
+                        v2u lo[2], hi[2];
+                        fa_split4((v4f){sc[8 * ks], sc[8 * ks + 1], sc[8 * ks + 2], sc[8 * ks + 3]}, p_scale, lo);
+                        fa_split4((v4f){sc[8 * ks + 4], sc[8 * ks + 5], sc[8 * ks + 6], sc[8 * ks + 7]}, p_scale, hi);
+#pragma unroll
+                        for (int p = 0; p < 2; ++p) pf[p] = __builtin_bit_cast(f16x8, (v4u){lo[p].x, lo[p].y, hi[p].x, hi[p].y});
+                    }
+                    f16x8 vf[DT][2];
 #pragma unroll
                     for (int t = 0; t < DT; ++t)
-                        O[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[t][PA_[q]], pf[PB_[q]], O[t], 0, 0, 0);
+#pragma unroll
+                        for (int p = 0; p < 2; ++p)
+                            vf[t][p] = __builtin_bit_cast(f16x8, *(const v4u *)&Vt[p][32 * t + c][ks * 16 + half * 8]);
+#pragma unroll
+                    for (int q = 0; q < 3; ++q)
+#pragma unroll
+                        for (int t = 0; t < DT; ++t)
+                            O[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[t][PA_[q]], pf[PB_[q]], O[t], 0, 0, 0);
+                }
             }
+            __syncthreads();
         }
-        __syncthreads();
-    }
 
-    if (PART) {
         const float l = l_run + __shfl_xor(l_run, 32, 64);
+        // O in the units of the weights' sum; in two steps, neither of which leaves f32's range where the result does not
+        const float o_unit = o_run > -INFINITY ? fast_exp2(o_run - m_run) : 0.f, p_unit = exp2_int(-FA_P_EXP);
         const int i = q0 + my_row / NREP;
-        if (i < a.s) {
+        if (i >= a.s) return;
+        if (PART) {
             const size_t n = (((size_t)bb * a.s + i) * a.hq + (size_t)hk * NREP + my_row % NREP) * (gridDim.z / a.b) + key_part;
             if (half == 0) {
                 a.part_ml[2 * n] = m_run;
@@ -306,71 +421,62 @@ __global__ __launch_bounds__(FA_THREADS, 2) void attn_prefill_f16x2_kernel(AttnP
             for (int t = 0; t < DT; ++t)
 #pragma unroll
                 for (int g = 0; g < 4; ++g)
-                    *(v4f *)(a.part + n * D + 32 * t + 8 * g + 4 * half) = v4f{O[t][4 * g], O[t][4 * g + 1], O[t][4 * g + 2], O[t][4 * g + 3]};
+                    *(v4f *)(a.part + n * D + 32 * t + 8 * g + 4 * half) =
+                        v4f{O[t][4 * g] * p_unit * o_unit, O[t][4 * g + 1] * p_unit * o_unit, O[t][4 * g + 2] * p_unit * o_unit, O[t][4 * g + 3] * p_unit * o_unit};
+            return;
         }
-        return;
-    }
-    // out = ctx / (sum + 1e-9), self_attention.rs:670-676; [B,S,Hq,D]
-    const float inv = 1.0f / fmaf(l_run + __shfl_xor(l_run, 32, 64), exp2_int(-FA_P_EXP), 1e-9f);
-    const float v_unit = ldexpf(1.0f, -(ev + FA_P_EXP));
-    const int i = q0 + my_row / NREP;
-    float o_scale = 0.f;
-    if (a.out_exp) {  // (uniform) the rows go out split, all with the exponent of the largest value there is
-        const unsigned *all = a.kv_range + ((size_t)a.b + bb) * a.hkv * FA_CHUNKS;
-        unsigned m = 0;
-        for (int n = lane; n < a.hkv * FA_CHUNKS; n += 64) m = max(m, all[n]);
-        const int eo = row_exponent(wave_umax(m));
-        o_scale = exp2_int(eo);
-        if (hk == 0 && my_row % NREP == 0 && half == 0 && i < a.s) a.out_exp[(size_t)bb * a.s + i] = eo;
-    }
-    if (i < a.s) {
-        const size_t head = (size_t)hk * NREP + my_row % NREP;
-        float *row = a.out + ((size_t)bb * a.s + i) * a.hq * D;
+        // out = ctx / (sum + 1e-9), self_attention.rs:670-676; [B,S,Hq,D]
+        const float inv = p_unit / (l + 1e-9f);
+        float *row = a.out + (((size_t)bb * a.s + i) * a.hq + (size_t)hk * NREP + my_row % NREP) * D;
 #pragma unroll
         for (int t = 0; t < DT; ++t)
 #pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const v4f v = {O[t][4 * g] * inv * v_unit, O[t][4 * g + 1] * inv * v_unit, O[t][4 * g + 2] * inv * v_unit, O[t][4 * g + 3] * inv * v_unit};
-                const int at = (int)head * D + 32 * t + 8 * g + 4 * half;
-                if (a.out_exp) store_split4((uint16_t *)row, at, v, o_scale);
-                else *(v4f *)(row + at) = v;
-            }
-    }
+            for (int g = 0; g < 4; ++g)
+                *(v4f *)(row + 32 * t + 8 * g + 4 * half) =
+                    v4f{O[t][4 * g] * inv * o_unit, O[t][4 * g + 1] * inv * o_unit, O[t][4 * g + 2] * inv * o_unit, O[t][4 * g + 3] * inv * o_unit};
+    };
+    if (wide) rows(std::true_type{});
+    else rows(std::false_type{});
 }
 
-// The parts of a row's keys together, in part order; a thread takes four elements of a (position, head) row.
-__global__ __launch_bounds__(256) void merge_parts_kernel(AttnPrefillArgs a, int parts) {
-    const int per_pos = a.hq * a.d / 4, bb = blockIdx.z, at = (int)(blockIdx.y * 256 + threadIdx.x);
-    const size_t pos = (size_t)bb * a.s + blockIdx.x;
-    const unsigned *vr = a.kv_range + ((size_t)a.b + bb) * a.hkv * FA_CHUNKS;
-    unsigned top = 0;
-    if (a.out_exp) {
-        for (int n = threadIdx.x & 63; n < a.hkv * FA_CHUNKS; n += 64) top = max(top, vr[n]);
-        top = wave_umax(top);
-        if (at == 0) a.out_exp[pos] = row_exponent(top);
-    }
-    if (at >= per_pos) return;
-    const int head = at * 4 / a.d, e = at * 4 % a.d, kv = head / (a.hq / a.hkv);
-    unsigned v_top = 0;
-    for (int n = 0; n < FA_CHUNKS; ++n) v_top = max(v_top, vr[kv * FA_CHUNKS + n]);
-    const size_t n0 = (pos * a.hq + head) * parts;
-    float m = -INFINITY;
-    for (int p = 0; p < parts; ++p) m = fmaxf(m, a.part_ml[2 * (n0 + p)]);
-    const float ref = m > -INFINITY ? m : 0.f;
-    float l = 0.f;
+// The parts of a row's keys together, in part order; a thread takes four elements of a (position, head) row.  SPLIT: a workgroup has the whole
+// row of a position and leaves it split, with an exponent of its own.
+template <bool SPLIT>
+__global__ __launch_bounds__(1024) void merge_parts_kernel(AttnPrefillArgs a, int parts) {
+    __shared__ unsigned wave_top[16];
+    const int per_pos = a.hq * a.d / 4, at = (int)(blockIdx.y * blockDim.x + threadIdx.x), tid = threadIdx.x;
+    const size_t pos = (size_t)blockIdx.z * a.s + blockIdx.x;
     v4f o = {0.f, 0.f, 0.f, 0.f};
+    if (at < per_pos) {
+        const int head = at * 4 / a.d, e = at * 4 % a.d;
+        const size_t n0 = (pos * a.hq + head) * parts;
+        float m = -INFINITY;
+        for (int p = 0; p < parts; ++p) m = fmaxf(m, a.part_ml[2 * (n0 + p)]);
+        const float ref = m > -INFINITY ? m : 0.f;
+        float l = 0.f;
 #pragma unroll 4
-    for (int p = 0; p < parts; ++p) {
-        const float w = fast_exp2(a.part_ml[2 * (n0 + p)] - ref);
-        const v4f x = *(const v4f *)(a.part + (n0 + p) * a.d + e);
-        l = fmaf(w, a.part_ml[2 * (n0 + p) + 1], l);
-        o.x = fmaf(w, x.x, o.x); o.y = fmaf(w, x.y, o.y); o.z = fmaf(w, x.z, o.z); o.w = fmaf(w, x.w, o.w);
+        for (int p = 0; p < parts; ++p) {
+            const float w = fast_exp2(a.part_ml[2 * (n0 + p)] - ref);
+            const v4f x = *(const v4f *)(a.part + (n0 + p) * a.d + e);
+            l = fmaf(w, a.part_ml[2 * (n0 + p) + 1], l);
+            o.x = fmaf(w, x.x, o.x); o.y = fmaf(w, x.y, o.y); o.z = fmaf(w, x.z, o.z); o.w = fmaf(w, x.w, o.w);
+        }
+        const float inv = 1.0f / (l + 1e-9f);
+        o = v4f{o.x * inv, o.y * inv, o.z * inv, o.w * inv};
     }
-    const float inv = 1.0f / fmaf(l, exp2_int(-FA_P_EXP), 1e-9f), unit = ldexpf(1.0f, -(row_exponent(v_top) + FA_P_EXP));
-    o = v4f{o.x * inv * unit, o.y * inv * unit, o.z * inv * unit, o.w * inv * unit};
     float *row = a.out + pos * a.hq * a.d;
-    if (a.out_exp) store_split4((uint16_t *)row, at * 4, o, exp2_int(row_exponent(top)));
-    else *(v4f *)(row + at * 4) = o;
+    if (!SPLIT) {
+        if (at < per_pos) *(v4f *)(row + at * 4) = o;
+        return;
+    }
+    const unsigned mine = wave_umax(magnitude_bits(o));
+    if ((tid & 63) == 0) wave_top[tid >> 6] = mine;
+    __syncthreads();
+    unsigned top = 0;
+    for (int w = 0; w < (int)blockDim.x >> 6; ++w) top = max(top, wave_top[w]);
+    const int e = row_exponent(top);
+    if (tid == 0) a.out_exp[pos] = e;
+    if (at < per_pos) store_split4((uint16_t *)row, at * 4, o, exp2_int(e));
 }
 
 // Parts the keys are cut into where the blocks of queries leave compute units idle: at least 128 keys each (two trips of the loop; a part costs
@@ -396,8 +502,9 @@ static int launch_fa_d(lumen_ctx *ctx, const AttnPrefillArgs &a_in) {
         a.key_chunk = ((L + parts - 1) / parts + trip - 1) / trip * trip;
         parts = (L + a.key_chunk - 1) / a.key_chunk;
     }
-    const size_t rows = parts > 1 ? (size_t)a.b * a.s * a.hq * parts : 0, range = 2 * (size_t)a.b * a.hkv * FA_CHUNKS;
-    const size_t need = (range + rows * (D + 2)) * sizeof(float);
+    const int tile = trip, tiles = (L + tile - 1) / tile;
+    const size_t rows = parts > 1 ? (size_t)a.b * a.s * a.hq * parts : 0, codes = 2 * (size_t)a.b * a.hkv * tiles;
+    const size_t need = (codes + rows * (D + 2)) * sizeof(float);
     if (need > ctx->attn_ws_bytes) {
         HIP_TRY(hipStreamSynchronize(ctx->stream));
         hipFree(ctx->attn_ws);
@@ -408,9 +515,10 @@ static int launch_fa_d(lumen_ctx *ctx, const AttnPrefillArgs &a_in) {
     }
     a.part = ctx->attn_ws;
     a.part_ml = a.part + rows * D;
-    unsigned *kv_range = (unsigned *)(a.part_ml + 2 * rows);
-    a.kv_range = kv_range;
-    hipLaunchKernelGGL(kv_range_kernel, dim3(FA_CHUNKS, a.b * a.hkv), dim3(256), 0, ctx->stream, a.k_cache, a.v_cache, a.max_seq, D, L, kv_range);
+    int *kv_tiles = (int *)(a.part_ml + 2 * rows);
+    a.kv_tiles = kv_tiles;
+    hipLaunchKernelGGL((kv_tiles_kernel<D, FA_KEYS * (D == 64 ? 2 : 1)>), dim3(tiles, a.b * a.hkv), dim3(256), 0, ctx->stream, a.k_cache, a.v_cache,
+                       a.max_seq, L, kv_tiles);
     grid.z *= parts;
 #define LAUNCH_FA(NR)                                                                                                                        \
     do {                                                                                                                                     \
@@ -424,9 +532,18 @@ static int launch_fa_d(lumen_ctx *ctx, const AttnPrefillArgs &a_in) {
         default: LAUNCH_FA(8); break;
     }
 #undef LAUNCH_FA
-    if (parts > 1)
-        hipLaunchKernelGGL(merge_parts_kernel, dim3(a.s, (a.hq * D / 4 + 255) / 256, a.b), dim3(256), 0, ctx->stream, a, parts);
+    const int pieces = a.hq * D / 4;  // of a position's row
+    bool split_done = false;
+    if (parts > 1) {
+        if (a.out_exp && pieces <= 1024) {
+            hipLaunchKernelGGL(merge_parts_kernel<true>, dim3(a.s, 1, a.b), dim3((pieces + 63) / 64 * 64), 0, ctx->stream, a, parts);
+            split_done = true;
+        } else {
+            hipLaunchKernelGGL(merge_parts_kernel<false>, dim3(a.s, (pieces + 255) / 256, a.b), dim3(256), 0, ctx->stream, a, parts);
+        }
+    }
     LUMEN_CHECK_LAUNCH();
+    if (a.out_exp && !split_done) return launch_split_rows(ctx, a.out, a.b * a.s, a.hq * D, a.out, a.out_exp);
     return LUMEN_OK;
 }
 

@@ -109,6 +109,7 @@ static inline float __int_as_float(int i) { return emu_bits_to<float>((uint32_t)
 #define __builtin_amdgcn_rcpf(x) (1.0f / (x))
 #define __builtin_amdgcn_s_waitcnt(x) ((void)0)
 #define __builtin_amdgcn_sched_group_barrier(a, b, c) ((void)0)
+#define __builtin_amdgcn_sched_barrier(a) ((void)0)
 void emu_sleep();
 #define __builtin_amdgcn_s_sleep(n) emu_sleep()
 unsigned long long wall_clock64();  // 100 MHz like the device's constant clock
@@ -226,6 +227,18 @@ static inline V emu_mfma_16x16x4f32(float a, float b, V c) {
     return c;
 }
 #define __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, x, y, z) emu_mfma_16x16x4f32((a), (b), (c))
+// v_mfma_f32_32x32x2_f32: A[l % 32][l / 32] and B[l / 32][l % 32] of lane l, D as for the other 32 x 32 ones
+template <typename V>
+static inline V emu_mfma_32x32x2f32(float a, float b, V c) {
+    const int lane = (int)(threadIdx.x & 63), j = lane & 31, g = lane >> 5;
+    float bk[2];
+    for (int k = 0; k < 2; ++k) bk[k] = emu_bits_to<float>(emu::wave_exchange(emu_bits_of(b), k * 32 + j));
+    for (int r = 0; r < 16; ++r)
+        for (int k = 0; k < 2; ++k)
+            c[r] = fmaf(emu_bits_to<float>(emu::wave_exchange(emu_bits_of(a), k * 32 + 8 * (r / 4) + 4 * g + r % 4)), bk[k], c[r]);
+    return c;
+}
+#define __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, x, y, z) emu_mfma_32x32x2f32((a), (b), (c))
 // On the GPU the lanes of a wavefront run in lockstep and the wave barrier only orders the compiler; here the lanes are
 // fibers of their own and have to meet.
 #define __builtin_amdgcn_wave_barrier() ((void)emu::wave_exchange(0u, 0))
