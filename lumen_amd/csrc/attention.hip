@@ -653,6 +653,7 @@ extern "C" int lumen_kv_cache_destroy(lumen_kv_cache *c) {
     }
     hipFree(c->part_tagged);
     hipFree(c->q_rot);
+    hipFree(c->prefill_ws);
     hipFree(c->d_pos);
     delete c;
     return LUMEN_OK;
@@ -879,23 +880,25 @@ extern "C" int lumen_attn_prefill_f32(lumen_kv_cache *c, lumen_rope *rope, const
     if (new_len > c->max_seq)  // self_attention.rs:341-346
         LUMEN_FAIL(LUMEN_ERR_KV_OVERFLOW, "KV cache overflow: new_len=%d > max_seq=%d", new_len, c->max_seq);
     if (s == 0) return LUMEN_OK;
-    // rotated queries: scratch kept on the cache, grown (with a stream synchronisation) only when a call needs more
-    const size_t q_floats = (size_t)c->b * s * h * c->d;
-    if (q_floats > c->q_rot_floats) {
+    // rotated queries and workspace: scratch kept on the cache, grown (with a stream synchronisation) only when a call has more positions (or heads)
+    auto grow = [&](float *&p, size_t &have, size_t need) {
+        if (need <= have) return LUMEN_OK;
         HIP_TRY(hipStreamSynchronize(c->ctx->stream));
-        hipFree(c->q_rot);
-        c->q_rot = nullptr;
-        c->q_rot_floats = 0;
-        HIP_TRY(hipMalloc((void **)&c->q_rot, sizeof(float) * q_floats));
-        c->q_rot_floats = q_floats;
-    }
-    float *q_rot = c->q_rot;
+        hipFree(p);
+        p = nullptr;
+        have = 0;
+        HIP_TRY(hipMalloc((void **)&p, sizeof(float) * need));
+        have = need;
+        return LUMEN_OK;
+    };
+    LUMEN_TRY(grow(c->q_rot, c->q_rot_floats, (size_t)c->b * s * h * c->d));
+    LUMEN_TRY(grow(c->prefill_ws, c->prefill_ws_floats, attn_prefill_workspace(c->ctx, c->b, s, h, c->h_kv, c->d, c->max_seq)));
     AttnPrefillArgs a = {};
     a.q = q; a.k = k; a.v = v; a.out = out; a.k_cache = c->k; a.v_cache = c->v;
     a.cos_t = rope->cos_dev; a.sin_t = rope->sin_dev;
     a.b = c->b; a.s = s; a.hq = h; a.hkv = c->h_kv; a.d = c->d; a.max_seq = c->max_seq; a.past_len = past_len;
     a.q_stride = h * c->d; a.k_stride = c->h_kv * c->d; a.v_stride = c->h_kv * c->d;
-    a.scale = scale; a.causal = causal; a.q_rot = q_rot;
+    a.scale = scale; a.causal = causal; a.q_rot = c->q_rot; a.ws = c->prefill_ws; a.ws_floats = c->prefill_ws_floats;
     const int rc = launch_attn_prefill(c->ctx, a);
     if (rc == LUMEN_OK) c->len = new_len;
     return rc;

@@ -84,7 +84,6 @@ extern "C" int lumen_ctx_destroy(lumen_ctx *ctx) {
     if (ctx->err_host) hipHostFree(ctx->err_host);
     if (ctx->gemm_ws) hipFree(ctx->gemm_ws);
     if (ctx->mixer_ws) hipFree(ctx->mixer_ws);
-    if (ctx->attn_ws) hipFree(ctx->attn_ws);
     hipEventDestroy(ctx->ev0);
     hipEventDestroy(ctx->ev1);
     hipStreamDestroy(ctx->own_stream);

@@ -56,8 +56,6 @@ struct lumen_ctx {
     int *err_host = nullptr;
     float *gemm_ws = nullptr;      // split-K workspace of the prefill GEMM, grown on demand
     size_t gemm_ws_bytes = 0;
-    float *attn_ws = nullptr;      // a prompt attention's unfinished rows and the exponents of its tiles, grown on demand
-    size_t attn_ws_bytes = 0;
     float *mixer_ws = nullptr;     // per-chunk operands of the recurrences, grown on demand
     size_t mixer_ws_bytes = 0;
     // this device's address of the fixed scratch array behind lumen_attn_decode_static_f32
@@ -91,8 +89,9 @@ struct lumen_kv_cache {
     unsigned merge_epoch = 0;
     int part_heads = 0;
     int *d_pos = nullptr;    // device copy of len for lumen_qkv_rope_append_f32, allocated at its first call
-    float *q_rot = nullptr;  // rotated queries of the prefill entry point, grown on demand
-    size_t q_rot_floats = 0;
+    // rotated queries of the prefill entry point, and its attention's workspace (attn_prefill_workspace), grown on demand
+    float *q_rot = nullptr, *prefill_ws = nullptr;
+    size_t q_rot_floats = 0, prefill_ws_floats = 0;
 };
 
 // ---------------------------------------------------------------- launchers
@@ -405,6 +404,8 @@ struct AttnPrefillArgs {
     const float *q_norm_w, *k_norm_w;
     float norm_eps;
     float *q_rot;    // scratch [B, S, Hq, D]
+    float *ws;       // scratch of attn_prefill_workspace floats; like q_rot, nobody else's while the launch runs
+    size_t ws_floats;
     int *out_exp;    // not null: the rows of out are left split (f16_split.h) with their exponents here [B, S]
     // set by the launcher: exponents of the tiles of cached keys and values; keys per part and the parts' unfinished rows [b s hq][parts][d] and
     // (maximum, sum) of theirs
@@ -419,6 +420,8 @@ struct AttnPrefillArgs {
 int launch_attn_prefill(lumen_ctx *ctx, const AttnPrefillArgs &a);
 // the scores / softmax / context part on the matrix cores (q_rot and the cache rows already written)
 bool attn_prefill_mfma_supported(const AttnPrefillArgs &a);
+// floats of AttnPrefillArgs::ws for any call of up to s positions over a cache of max_seq rows
+size_t attn_prefill_workspace(const lumen_ctx *ctx, int b, int s, int hq, int hkv, int d, int max_seq);
 int launch_attn_prefill_mfma(lumen_ctx *ctx, const AttnPrefillArgs &a);
 
 int attn_decode_nsplit(int max_seq, int d);

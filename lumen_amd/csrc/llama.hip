@@ -80,7 +80,8 @@ struct lumen_llama {
     // prefill buffers (grown on demand, kept)
     int pf_cap = 0, pf_logit_cap = 0;
     float *p_x = nullptr, *p_h = nullptr, *p_n = nullptr, *p_qkv = nullptr, *p_qrot = nullptr, *p_attn = nullptr,
-          *p_act = nullptr, *p_logits = nullptr;
+          *p_act = nullptr, *p_logits = nullptr, *p_attn_ws = nullptr;  // (p_attn_ws: the attention's workspace)
+    size_t p_attn_ws_floats = 0;
     int *p_ids = nullptr, *p_exp = nullptr;  // (p_exp: exponents of p_n's, p_attn's and p_act's rows)
     std::vector<void *> allocs;
 };
@@ -113,7 +114,7 @@ extern "C" int lumen_llama_destroy(lumen_llama *m) {
     if (m->graph) hipGraphDestroy(m->graph);
     for (void *p : m->allocs) hipFree(p);
     hipFree(m->p_x); hipFree(m->p_h); hipFree(m->p_n); hipFree(m->p_qkv); hipFree(m->p_qrot);
-    hipFree(m->p_attn); hipFree(m->p_act); hipFree(m->p_logits); hipFree(m->p_ids); hipFree(m->p_exp);
+    hipFree(m->p_attn); hipFree(m->p_act); hipFree(m->p_logits); hipFree(m->p_ids); hipFree(m->p_exp); hipFree(m->p_attn_ws);
     delete m;
     return LUMEN_OK;
 }
@@ -795,8 +796,9 @@ static int ensure_prefill_buffers(lumen_llama *m, int s, bool all_rows) {
     if (s > m->pf_cap) {
         HIP_TRY(hipStreamSynchronize(m->ctx->stream));
         hipFree(m->p_x); hipFree(m->p_h); hipFree(m->p_n); hipFree(m->p_qkv); hipFree(m->p_qrot);
-        hipFree(m->p_attn); hipFree(m->p_act); hipFree(m->p_ids); hipFree(m->p_exp);
-        m->p_x = m->p_h = m->p_n = m->p_qkv = m->p_qrot = m->p_attn = m->p_act = nullptr;
+        hipFree(m->p_attn); hipFree(m->p_act); hipFree(m->p_ids); hipFree(m->p_exp); hipFree(m->p_attn_ws);
+        m->p_x = m->p_h = m->p_n = m->p_qkv = m->p_qrot = m->p_attn = m->p_act = m->p_attn_ws = nullptr;
+        m->p_attn_ws_floats = 0;
         m->p_ids = m->p_exp = nullptr;
         m->pf_cap = 0;
         const size_t S = (size_t)s;
@@ -809,6 +811,8 @@ static int ensure_prefill_buffers(lumen_llama *m, int s, bool all_rows) {
         HIP_TRY(hipMalloc((void **)&m->p_act, S * c.intermediate_size * 4));
         HIP_TRY(hipMalloc((void **)&m->p_ids, S * sizeof(int)));
         HIP_TRY(hipMalloc((void **)&m->p_exp, 3 * S * sizeof(int)));
+        m->p_attn_ws_floats = attn_prefill_workspace(m->ctx, 1, s, c.num_attention_heads, c.num_key_value_heads, m->D, c.max_seq_len);
+        HIP_TRY(hipMalloc((void **)&m->p_attn_ws, m->p_attn_ws_floats * sizeof(float)));
         m->pf_cap = s;
         // the split-K workspace of the four products at this many rows, so that no launch has to grow it
         const int H = c.hidden_size, I = c.intermediate_size;
@@ -867,7 +871,7 @@ static int run_prefill(lumen_llama *m, const std::vector<int> &ids, float *logit
         a.max_seq = c.max_seq_len; a.past_len = m->len;
         a.q_stride = a.k_stride = a.v_stride = m->qkvd;
         a.scale = m->scale; a.causal = 1; a.q_norm_w = w.q_norm; a.k_norm_w = w.k_norm; a.norm_eps = c.rms_norm_eps;
-        a.q_rot = m->p_qrot;
+        a.q_rot = m->p_qrot; a.ws = m->p_attn_ws; a.ws_floats = m->p_attn_ws_floats;
         a.out_exp = attn_prefill_mfma_supported(a) ? e_attn : nullptr;
         LUMEN_TRY(launch_attn_prefill(ctx, a));
         if (split && !a.out_exp) LUMEN_TRY(launch_split_rows(ctx, m->p_attn, s, m->qd, m->p_attn, e_attn));

@@ -36,6 +36,7 @@
 #include "attn_device.h"
 #include "f16_split.h"
 
+#include <algorithm>
 #include <type_traits>
 
 typedef float v16f __attribute__((ext_vector_type(16)));
@@ -487,6 +488,15 @@ static int fa_key_parts(int num_cus, int blocks, int keys) {
     return n < 2 ? 1 : n < 32 ? n : 32;
 }
 
+// At most fa_key_parts' parts; a block of queries holds FA_ROWS rows, so parts times rows stay below two blocks per compute unit.
+size_t attn_prefill_workspace(const lumen_ctx *ctx, int b, int s, int hq, int hkv, int d, int max_seq) {
+    if (d != 64 && d != 128) return 0;
+    const int trip = FA_KEYS * (d == 64 ? 2 : 1);
+    const size_t most = std::min((max_seq + 127) / 128, 32);
+    const size_t rows = most < 2 ? 0 : std::min(most * b * s * hq, (size_t)2 * ctx->num_cus * FA_ROWS);
+    return 2 * (size_t)b * hkv * ((max_seq + trip - 1) / trip) + rows * (d + 2);
+}
+
 template <int D>
 static int launch_fa_d(lumen_ctx *ctx, const AttnPrefillArgs &a_in) {
     AttnPrefillArgs a = a_in;
@@ -504,16 +514,9 @@ static int launch_fa_d(lumen_ctx *ctx, const AttnPrefillArgs &a_in) {
     }
     const int tile = trip, tiles = (L + tile - 1) / tile;
     const size_t rows = parts > 1 ? (size_t)a.b * a.s * a.hq * parts : 0, codes = 2 * (size_t)a.b * a.hkv * tiles;
-    const size_t need = (codes + rows * (D + 2)) * sizeof(float);
-    if (need > ctx->attn_ws_bytes) {
-        HIP_TRY(hipStreamSynchronize(ctx->stream));
-        hipFree(ctx->attn_ws);
-        ctx->attn_ws = nullptr;
-        ctx->attn_ws_bytes = 0;
-        HIP_TRY(hipMalloc((void **)&ctx->attn_ws, need));
-        ctx->attn_ws_bytes = need;
-    }
-    a.part = ctx->attn_ws;
+    const size_t need = codes + rows * (D + 2);
+    if (!a.ws || need > a.ws_floats) LUMEN_FAIL(LUMEN_ERR_INVALID, "prompt attention: workspace of %zu floats, %zu wanted", a.ws_floats, need);
+    a.part = a.ws;
     a.part_ml = a.part + rows * D;
     int *kv_tiles = (int *)(a.part_ml + 2 * rows);
     a.kv_tiles = kv_tiles;

@@ -5,9 +5,9 @@
 // attention workgroups per head (slices + fold), rotated and un-rotated (q/k-norm) hand-over, f32 and bf16 weights;
 // the gate|up -> down chain; the few-row product of short prompts with ragged shapes and all three epilogues; the
 // streaming vector-matrix product and the stand-alone decode attention those forms fall back to, the latter also
-// at operator level over a sliced cache (slices merged inside the launch).
+// at operator level over a sliced cache (slices merged inside the launch); prompt attention of two caches, one of them recorded.
 //
-//   emu_test [case ...]      cases: chain sliced qknorm bf16 skinny attn layerop (default: all)
+//   emu_test [case ...]      cases: chain sliced qknorm bf16 skinny attn layerop shapes caches (default: all)
 #include <math.h>
 #include <stdio.h>
 #include <stdlib.h>
@@ -15,6 +15,8 @@
 
 #include <string>
 #include <vector>
+
+#include <hip/hip_runtime.h>
 
 #include "../../include/lumen_hip.h"
 extern "C" {
@@ -466,6 +468,55 @@ static void case_shapes(lumen_ctx *ctx) {
     printf("  worst max rel err %.2e\n", worst);
 }
 
+// A recorded prompt attention of one cache, replayed after another cache's call has needed more scratch than it had.
+static void case_caches(lumen_ctx *ctx) {
+    printf("caches: a recorded prompt attention beside a larger one on another cache\n");
+    const int h = 2, d = 64, s = 97;
+    lumen_rope *rope = nullptr;
+    OK(lumen_rope_create(ctx, d, 1024, 10000.f, &rope));
+    std::vector<float> cs((size_t)1024 * d), sn((size_t)1024 * d);
+    lo_rope_table(cs.data(), sn.data(), d, 1024, 10000.f);
+    lumen_kv_cache *small = nullptr, *large = nullptr;
+    OK(lumen_kv_cache_create(ctx, 1, h, 128, d, &small));
+    OK(lumen_kv_cache_create(ctx, 1, h, 1024, d, &large));
+    lo_kv_cache *co = lo_kv_cache_new(1, h, 128, d);
+    const size_t n = (size_t)s * h * d;
+    std::vector<float> x[3], got(n), ref(n);
+    void *dx[3], *dout, *dother;
+    for (int i = 0; i < 3; ++i) {
+        x[i] = randn(n, 1.f);
+        OK(lumen_malloc(ctx, n * 4, &dx[i]));
+        OK(lumen_upload(ctx, dx[i], x[i].data(), n * 4));
+    }
+    OK(lumen_malloc(ctx, n * 4, &dout));
+    OK(lumen_malloc(ctx, n * 4, &dother));
+    auto prompt = [&](lumen_kv_cache *c, void *out) {
+        OK(lumen_attn_prefill_f32(c, rope, (const float *)dx[0], (const float *)dx[1], (const float *)dx[2], (float *)out, s, h, 0.125f, 1));
+    };
+    prompt(small, dout);  // (the call that allocates)
+    OK(lumen_kv_cache_set_len(small, 0));
+    hipGraph_t graph;
+    hipGraphExec_t exec;
+    if (hipStreamBeginCapture(nullptr, hipStreamCaptureModeThreadLocal) != hipSuccess) exit(2);
+    prompt(small, dout);
+    if (hipStreamEndCapture(nullptr, &graph) != hipSuccess || hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0) != hipSuccess) exit(2);
+    OK(lumen_kv_cache_set_len(large, 1024 - s));
+    prompt(large, dother);
+    if (hipGraphLaunch(exec, nullptr) != hipSuccess) exit(2);
+    OK(lumen_download(ctx, got.data(), dout, n * 4));
+    CHECK(lo_attn_prefill_f32(co, x[0].data(), x[1].data(), x[2].data(), ref.data(), s, h, cs.data(), sn.data(), 1024, 0.125f, 1) == LO_OK, "checker");
+    const double e = max_rel(got.data(), ref.data(), n);
+    printf("  replayed: max rel err %.2e\n", e);
+    CHECK(e <= 2e-5, "replayed prompt attention: %.3g", e);
+    hipGraphExecDestroy(exec);
+    hipGraphDestroy(graph);
+    for (void *p : {dx[0], dx[1], dx[2], dout, dother}) OK(lumen_free(ctx, p));
+    OK(lumen_kv_cache_destroy(small));
+    OK(lumen_kv_cache_destroy(large));
+    lo_kv_cache_free(co);
+    OK(lumen_rope_destroy(rope));
+}
+
 int main(int argc, char **argv) {
     lo_set_threads(4);
     lumen_ctx *ctx = nullptr;
@@ -475,7 +526,7 @@ int main(int argc, char **argv) {
         return 0;  // (reached only if nothing stopped the program: the test expects a sanitizer report instead)
     }
     struct { const char *name; void (*fn)(lumen_ctx *); } cases[] = {
-        {"chain", case_chain}, {"sliced", case_sliced}, {"qknorm", case_qknorm}, {"bf16", case_bf16}, {"skinny", case_skinny}, {"attn", case_attn}, {"layerop", case_layerop}, {"shapes", case_shapes}};
+        {"chain", case_chain}, {"sliced", case_sliced}, {"qknorm", case_qknorm}, {"bf16", case_bf16}, {"skinny", case_skinny}, {"attn", case_attn}, {"layerop", case_layerop}, {"shapes", case_shapes}, {"caches", case_caches}};
     for (const auto &c : cases) {
         bool run = argc <= 1;
         for (int i = 1; i < argc; ++i) run = run || !strcmp(argv[i], c.name);
