@@ -660,6 +660,7 @@ extern "C" int lumen_hybrid_set_param(lumen_hybrid *m, const char *name, const v
         }
         if (p.exps) LUMEN_TRY(launch_row_exponents(m->ctx, p.dst, !to_f32, (int)p.rows, (int)p.ld, 0, 1, p.exps));
         if (p.exps2) LUMEN_TRY(launch_row_exponents(m->ctx, p.dst2, !to_f32, (int)p.rows, (int)p.ld, 0, 1, p.exps2));
+        HIP_TRY(hipStreamSynchronize(m->ctx->stream));  // (the next call may be on another stream)
         return LUMEN_OK;
     }
     LUMEN_FAIL(LUMEN_ERR_INVALID, "Parameter %s not found in model", name);

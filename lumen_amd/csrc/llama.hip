@@ -330,7 +330,8 @@ void bf16_to_f32_host(const uint16_t *src, float *dst, size_t n) {
 
 // Copies a [rows, cols] host matrix (src dtype) into device memory of dst dtype
 // whose row r lands at dst + (row0 + r*row_step) * cols.
-// exps not null: the exponents of the rows go there, by the rows' places in dst.
+// exps not null: the exponents of the rows go there, by the rows' places in dst.  Nothing is in flight when it returns: the next call may be on
+// another stream.
 static int upload_matrix(lumen_llama *m, void *dst, bool dst_bf16, const void *src, int src_dtype, size_t rows,
                          size_t cols, size_t row0, size_t row_step, int *exps = nullptr) {
     const size_t dsz = dst_bf16 ? 2 : 4;
@@ -353,7 +354,11 @@ static int upload_matrix(lumen_llama *m, void *dst, bool dst_bf16, const void *s
                                  m->ctx->stream));
         HIP_TRY(hipStreamSynchronize(m->ctx->stream));
     }
-    return exps ? launch_row_exponents(m->ctx, dst, dst_bf16, (int)rows, (int)cols, (int)row0, (int)row_step, exps) : LUMEN_OK;
+    if (exps) {
+        LUMEN_TRY(launch_row_exponents(m->ctx, dst, dst_bf16, (int)rows, (int)cols, (int)row0, (int)row_step, exps));
+        HIP_TRY(hipStreamSynchronize(m->ctx->stream));
+    }
+    return LUMEN_OK;
 }
 
 static int want_shape(const char *name, const int64_t *shape, int ndim, int64_t a, int64_t b) {

@@ -86,7 +86,7 @@ struct Engine {
 Engine E;
 bool g_capturing = false;
 struct emu_graph_impl { std::vector<Launch> nodes; };
-unsigned long g_launches = 0;
+unsigned long g_launches = 0, g_unwaited = 0;  // launches; those no synchronisation of their stream has followed
 void capture_node(Launch &&L);
 
 void annotate_leave(void **fake_save, const void *to_bottom, size_t to_size) {
@@ -209,6 +209,7 @@ void run(const Launch &L) {
     const int n = (int)(L.block.x * L.block.y * L.block.z);
     if (n <= 0 || n > MAX_THREADS || L.block.y != 1 || L.block.z != 1) emu::not_emulated("workgroup shape");
     ++g_launches;
+    ++g_unwaited;
     if (!E.main_stack_bottom) {
         pthread_attr_t attr;
         pthread_getattr_np(pthread_self(), &attr);
@@ -312,7 +313,11 @@ hipError_t hipGetDeviceProperties(hipDeviceProp_t *p, int) {
 }
 hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned) { *s = new emu_stream(); return hipSuccess; }
 hipError_t hipStreamDestroy(hipStream_t s) { delete s; return hipSuccess; }
-hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t) {
+    g_unwaited = 0;
+    return hipSuccess;
+}
+extern "C" unsigned long emu_launches_in_flight() { return g_unwaited; }  // on a GPU they could still run
 hipError_t hipEventCreate(hipEvent_t *e) { *e = new emu_event(); return hipSuccess; }
 hipError_t hipEventDestroy(hipEvent_t e) { delete e; return hipSuccess; }
 hipError_t hipEventRecord(hipEvent_t e, hipStream_t) { e->t = std::chrono::steady_clock::now(); return hipSuccess; }

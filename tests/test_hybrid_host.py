@@ -156,6 +156,39 @@ def emulation():
                 ASAN_OPTIONS="detect_leaks=0")
 
 
+IN_FLIGHT = """
+import ctypes, os
+from lumen_amd import synth
+from lumen_amd.hybrid import HybridModel, pinavik_config
+from lumen_amd.models import LlamaModel
+from tests import hybrid_util as hu
+in_flight = ctypes.CDLL(os.environ["LUMEN_HIP_LIB"]).emu_launches_in_flight
+in_flight.restype = ctypes.c_ulong
+def check(model, params):
+    model.sync()
+    for name, value in params.items():
+        model.set_param(name, value)
+        assert in_flight() == 0, name
+cfg = dict(vocab_size=11, hidden_size=64, intermediate_size=64, num_hidden_layers=1, num_attention_heads=2, num_key_value_heads=1,
+           rms_norm_eps=1e-5, max_seq_len=16, rope_theta=10000.0)
+llama = LlamaModel(cfg)
+llama.sync = lambda: llama.forward([1, 2])
+check(llama, synth.make_params(cfg, seed=1))
+cfg = hu.config(24, 30, [hu.delta(2, 1, 6, 8, ff=20), hu.attention(2, 1, 6, 8, 5), hu.wkv(2, 6)], loop=(0, 2, 2))
+params = hu.make_params(cfg, seed=1)
+hybrid = HybridModel(pinavik_config(cfg, lambda name: params[name].shape, 64, "float32"))
+hybrid.sync = lambda: hybrid.step([1, 2], [1])
+check(hybrid, params)
+print("nothing in flight")
+"""
+
+
+def test_a_set_parameter_leaves_nothing_in_flight(emulation):
+    """The next call may come on another stream, which does not wait for this one."""
+    r = subprocess.run([sys.executable, "-c", IN_FLIGHT], cwd=ROOT, env=emulation, capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0 and "nothing in flight" in r.stdout, (r.stdout[-3000:], r.stderr[-3000:])
+
+
 # (single cases of the GPU suite: both recurrences over portions, the three forms of window attention, the row
 # operations, and one model end to end -- prompt, portions, decoding)
 @pytest.mark.parametrize("cases", [
