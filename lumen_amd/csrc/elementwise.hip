@@ -43,7 +43,6 @@ template <int VPT, bool SPLIT>
 __global__ __launch_bounds__(256) void rmsnorm_vec_kernel(const float *__restrict__ x, const float *__restrict__ w,
                                                           float *__restrict__ out, int dim, float eps, int *__restrict__ exps) {
     __shared__ float red[4];
-    __shared__ unsigned top[4];
     const float *xr = x + (size_t)blockIdx.x * dim;
     float *o = out + (size_t)blockIdx.x * dim;
     const int tid = threadIdx.x;
@@ -72,7 +71,6 @@ __global__ __launch_bounds__(256) void rmsnorm_vec_kernel(const float *__restric
     const float tot = (red[0] + red[1]) + (red[2] + red[3]);
     const float rms = sqrtf(tot / (float)dim + eps);
     const float inv = 1.0f / rms;
-    unsigned m = 0;
 #pragma unroll
     for (int i = 0; i < VPT; ++i) {
         const int k = (tid + i * 256) * 4;
@@ -81,25 +79,10 @@ __global__ __launch_bounds__(256) void rmsnorm_vec_kernel(const float *__restric
         r.y = v[i].y * inv * g[i].y;
         r.z = v[i].z * inv * g[i].z;
         r.w = v[i].w * inv * g[i].w;
-        if (SPLIT) {  // (past the end: zeros)
-            v[i] = r;
-            m = max(m, magnitude_bits(r));
-        } else if (k < dim) {
-            *(v4f *)(o + k) = r;
-        }
+        if (SPLIT) v[i] = r;  // (past the end: zeros)
+        else if (k < dim) *(v4f *)(o + k) = r;
     }
-    if (!SPLIT) return;
-    m = wave_umax(m);
-    if ((tid & 63) == 0) top[tid >> 6] = m;
-    __syncthreads();
-    const int e = row_exponent(max(max(top[0], top[1]), max(top[2], top[3])));
-    const float s = exp2_int(e);
-    if (tid == 0) exps[blockIdx.x] = e;
-#pragma unroll
-    for (int i = 0; i < VPT; ++i) {
-        const int k = (tid + i * 256) * 4;
-        if (k < dim) store_split4((uint16_t *)o, k, v[i], s);
-    }
+    if (SPLIT) leave_row<VPT>(v, dim, o, exps + blockIdx.x);
 }
 
 int launch_rmsnorm(lumen_ctx *ctx, const float *x, const float *w, float *out, int rows, int dim, float eps, int *exps) {
@@ -334,7 +317,6 @@ template <int VPT, bool SPLIT>
 __global__ __launch_bounds__(1024) void polynorm_vec_kernel(const float *z, const float *__restrict__ coef, float *out, int dim,
                                                             int stride, float eps, int *__restrict__ exps) {
     __shared__ float red[3][16];
-    __shared__ unsigned top[16];
     const float *zr = z + (size_t)blockIdx.x * stride;
     float *o = out + (size_t)blockIdx.x * stride;
     const int tid = threadIdx.x, nt = blockDim.x, nw = nt >> 6;
@@ -375,34 +357,16 @@ __global__ __launch_bounds__(1024) void polynorm_vec_kernel(const float *z, cons
     }
     const float n = (float)dim;
     const float a1 = coef[0] / sqrtf(s1 / n + eps), a2 = coef[1] / sqrtf(s2 / n + eps), a3 = coef[2] / sqrtf(s3 / n + eps), c3 = coef[3];
-    unsigned m = 0;
 #pragma unroll
     for (int i = 0; i < VPT; ++i) {
         const int k = (tid + i * nt) * 4;
         v4f r;
 #pragma unroll
         for (int e = 0; e < 4; ++e) r[e] = k + e < dim ? fmaf(fmaf(fmaf(a3, v[i][e], a2), v[i][e], a1), v[i][e], c3) : 0.f;
-        if (SPLIT) {
-            v[i] = r;
-            m = max(m, magnitude_bits(r));
-        } else if (k < stride) {
-            *(v4f *)(o + k) = r;
-        }
+        if (SPLIT) v[i] = r;
+        else if (k < stride) *(v4f *)(o + k) = r;
     }
-    if (!SPLIT) return;
-    m = wave_umax(m);
-    if ((tid & 63) == 0) top[tid >> 6] = m;
-    __syncthreads();
-    m = 0;
-    for (int w = 0; w < nw; ++w) m = max(m, top[w]);
-    const int e = row_exponent(m);
-    const float s = exp2_int(e);
-    if (tid == 0) exps[blockIdx.x] = e;
-#pragma unroll
-    for (int i = 0; i < VPT; ++i) {
-        const int k = (tid + i * nt) * 4;
-        if (k < stride) store_split4((uint16_t *)o, k, v[i], s);
-    }
+    if (SPLIT) leave_row<VPT>(v, stride, o, exps + blockIdx.x);
 }
 
 template <bool SPLIT>
@@ -466,11 +430,9 @@ template <int VPT>
 __global__ __launch_bounds__(256) void token_shift_split_kernel(const float *__restrict__ h, const float *__restrict__ mu,
                                                                 const float *__restrict__ prev, float *__restrict__ next,
                                                                 float *__restrict__ mixes, int s, int dim, int *__restrict__ exps) {
-    __shared__ unsigned top[4];
     const int t = blockIdx.x, mix = blockIdx.y, tid = threadIdx.x;
     const float *cur = h + (size_t)t * dim, *bef = t ? cur - dim : prev;
     v4f r[VPT];
-    unsigned m = 0;
 #pragma unroll
     for (int i = 0; i < VPT; ++i) {
         const int k = (tid + i * 256) * 4;
@@ -479,22 +441,11 @@ __global__ __launch_bounds__(256) void token_shift_split_kernel(const float *__r
             const v4f c = *(const v4f *)(cur + k), d = *(const v4f *)(bef + k) - c, f = *(const v4f *)(mu + (size_t)mix * dim + k);
 #pragma unroll
             for (int e = 0; e < 4; ++e) r[i][e] = fmaf(d[e], f[e], c[e]);
-            m = max(m, magnitude_bits(r[i]));
             if (mix == 0 && t == s - 1) *(v4f *)(next + k) = c;
         }
     }
-    m = wave_umax(m);
-    if ((tid & 63) == 0) top[tid >> 6] = m;
-    __syncthreads();
-    const int e = row_exponent(max(max(top[0], top[1]), max(top[2], top[3])));
-    const float sc = exp2_int(e);
     const size_t row = (size_t)mix * s + t;
-    if (tid == 0) exps[row] = e;
-#pragma unroll
-    for (int i = 0; i < VPT; ++i) {
-        const int k = (tid + i * 256) * 4;
-        if (k < dim) store_split4((uint16_t *)(mixes + row * dim), k, r[i], sc);
-    }
+    leave_row<VPT>(r, dim, mixes + row * dim, exps + row);
 }
 
 int launch_token_shift(lumen_ctx *ctx, const float *h, const float *mu, const float *prev, float *next, float *mixes, int n,

@@ -827,7 +827,6 @@ template <bool SPLIT>
 __global__ __launch_bounds__(256) void gemm_reduce_norm_kernel(GemmArgs a, int splits) {
     typedef float v4 __attribute__((ext_vector_type(4)));
     __shared__ float red[4];
-    __shared__ unsigned top[4];
     const int row = blockIdx.x, tid = threadIdx.x, N = a.N;
     const size_t MN = (size_t)a.M * N, base = (size_t)row * N;
     v4 v[GEMM_ROW_VPT], g[GEMM_ROW_VPT];
@@ -864,7 +863,6 @@ __global__ __launch_bounds__(256) void gemm_reduce_norm_kernel(GemmArgs a, int s
     __syncthreads();
     const float tot = (red[0] + red[1]) + (red[2] + red[3]);
     const float inv = 1.0f / sqrtf(tot / (float)N + a.norm_eps);
-    unsigned m = 0;
 #pragma unroll
     for (int i = 0; i < GEMM_ROW_VPT; ++i) {
         const int k = (tid + i * 256) * 4;
@@ -873,25 +871,10 @@ __global__ __launch_bounds__(256) void gemm_reduce_norm_kernel(GemmArgs a, int s
         r.y = v[i].y * inv * g[i].y;
         r.z = v[i].z * inv * g[i].z;
         r.w = v[i].w * inv * g[i].w;
-        if (SPLIT) {  // (past the end: zeros)
-            v[i] = r;
-            m = max(m, magnitude_bits(r));
-        } else if (k < N) {
-            *(v4 *)(a.norm_out + base + k) = r;
-        }
+        if (SPLIT) v[i] = r;  // (past the end: zeros)
+        else if (k < N) *(v4 *)(a.norm_out + base + k) = r;
     }
-    if (!SPLIT) return;
-    m = wave_umax(m);
-    if ((tid & 63) == 0) top[tid >> 6] = m;
-    __syncthreads();
-    const int e = row_exponent(max(max(top[0], top[1]), max(top[2], top[3])));
-    const float s = exp2_int(e);
-    if (tid == 0) a.norm_exp[row] = e;
-#pragma unroll
-    for (int i = 0; i < GEMM_ROW_VPT; ++i) {
-        const int k = (tid + i * 256) * 4;
-        if (k < N) store_split4((uint16_t *)(a.norm_out + base), k, v[i], s);
-    }
+    if (SPLIT) leave_row<GEMM_ROW_VPT>(v, N, a.norm_out + base, a.norm_exp + row);
 }
 
 // Any K / alignment: one thread per output element.

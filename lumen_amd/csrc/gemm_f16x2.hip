@@ -28,9 +28,10 @@ typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 
 // In LDS a slice of 32 k is four planes of 8 k, [k / 8][row][8 f16] with two rows of padding: an operand read of 32 rows is 512
 // contiguous bytes, and a staging write of two rows' pieces (the planes start 32 bytes apart, modulo the banks) covers all banks once.
-template <int EPI, bool PARTIAL, int FI, int FJ>
-__device__ __forceinline__ void store_scaled_tiles(const GemmArgs &a, const v16f (&acc)[FI][FJ], const int *ae_tile, const int *we_tile, int bm, int bn,
-                                                   int wrow, int wcol, int lane) {
+// SCALED: the sums are in units of the rows' exponents.
+template <int EPI, bool PARTIAL, bool SCALED, int FI, int FJ>
+__device__ __forceinline__ void store_tiles(const GemmArgs &a, const v16f (&acc)[FI][FJ], const int *ae_tile, const int *we_tile, int bm, int bn, int wrow,
+                                            int wcol, int lane) {
     const int M = a.M, N = a.N;
     float *part = PARTIAL ? a.part + (size_t)blockIdx.z * M * N : nullptr;
     int we[FJ];
@@ -45,7 +46,7 @@ __device__ __forceinline__ void store_scaled_tiles(const GemmArgs &a, const v16f
 #pragma unroll
             for (int j = 0; j < FJ; ++j) {
                 const int col = bn + wcol + j * 32 + (lane & 31);
-                const float v = ldexpf(acc[i][j][r], -(ae + we[j]));
+                const float v = SCALED ? ldexpf(acc[i][j][r], -(ae + we[j])) : acc[i][j][r];
                 if (PARTIAL) {
                     if (row < M && col < N) part[(size_t)row * N + col] = v;
                 } else if (EPI == EPI_SWIGLU) {
@@ -57,6 +58,72 @@ __device__ __forceinline__ void store_scaled_tiles(const GemmArgs &a, const v16f
                 }
             }
         }
+}
+
+// A wavefront's share of a tile that meets a row of either operand pairs cannot hold: f32 matrix instructions on the f32 values, straight from memory;
+// a row of A that is pairs all the same is put together (hi + lo is exact).  32 x 64 of C at a time, 16 of K in flight: the f32 instruction takes
+// five times the pairs' three, so that is what bounds it.
+template <bool WBF16, int EPI, bool PARTIAL, int FI, int FJ>
+__device__ __forceinline__ void wide_tiles(const GemmArgs &a, const int *ae_tile, const int *we_tile, int bm, int bn, int wrow, int wcol, int lane, int k0, int k1) {
+    const int c = lane & 31, half = lane >> 5, K = a.K;
+    static_assert(FJ % 2 == 0, "two tiles side by side");
+#pragma unroll 1
+    for (int at = 0; at < FI * FJ / 2; ++at) {
+        const int i = at / (FJ / 2), col0 = wcol + at % (FJ / 2) * 64;
+        const char *wp[2];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) wp[j] = (const char *)a.W + (size_t)min(bn + col0 + j * 32 + c, a.N - 1) * K * (WBF16 ? 2 : 4);
+        const int row = min(bm + wrow + i * 32 + c, a.M - 1), code = ae_tile[wrow + i * 32 + c];
+        const bool plain = is_wide(code);
+        const float unit = plain ? 1.f : exp2_int(-code);
+        const char *ap = (const char *)a.a_split + (size_t)row * K * 4;
+        v16f acc[1][2];
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[0][j][r] = 0.f;
+        // elements 8 t + 4 half .. + 3 of 16 k (both operands of instruction w of eight elements: element 4 half + w)
+        v2u x[2][2][2];
+        v4u w[2][2][2];
+        auto fetch = [&](int set, int k) {
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                const int e = 8 * t + 4 * half;
+                x[set][t][0] = *(const v2u *)(ap + (size_t)k * 4 + (plain ? e * 4 : e * 2));
+                x[set][t][1] = *(const v2u *)(ap + (size_t)k * 4 + (plain ? e * 4 + 8 : 32 + e * 2));
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    if (WBF16) {
+                        const v2u b = *(const v2u *)(wp[j] + (size_t)(k + e) * 2);
+                        w[set][t][j] = v4u{b.x << 16, b.x & 0xffff0000u, b.y << 16, b.y & 0xffff0000u};
+                    } else {
+                        w[set][t][j] = *(const v4u *)(wp[j] + (size_t)(k + e) * 4);
+                    }
+                }
+            }
+        };
+        auto product = [&](int set) {
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                const unsigned b[4] = {x[set][t][0].x, x[set][t][0].y, x[set][t][1].x, x[set][t][1].y};
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const f16x2_t hi = __builtin_bit_cast(f16x2_t, b[e >> 1]), lo = __builtin_bit_cast(f16x2_t, b[2 + (e >> 1)]);
+                    const float v = plain ? __uint_as_float(b[e]) : ((float)hi[e & 1] + (float)lo[e & 1]) * unit;
+#pragma unroll
+                    for (int j = 0; j < 2; ++j) acc[0][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(v, __uint_as_float(w[set][t][j][e]), acc[0][j], 0, 0, 0);
+                }
+            }
+        };
+        if (k0 < k1) fetch(0, k0);
+        for (int k = k0; k < k1; k += 32) {  // (whole slices of 64 of K: the launcher's condition)
+            fetch(1, k + 16);
+            product(0);
+            fetch(0, min(k + 32, k1 - 16));
+            product(1);
+        }
+        store_tiles<EPI, PARTIAL, false>(a, acc, ae_tile, we_tile, bm, bn, wrow + i * 32, col0, lane);
+    }
 }
 
 // WM x WN wavefronts, FI x FJ tiles of 32 x 32 each; slices of HK of K in a ring of RING in LDS, D slices in flight from memory.  All operands of a
@@ -77,7 +144,7 @@ __global__ __launch_bounds__(64 * WM * WN, (FI * FJ > 8 ? 1 : 2)) void gemm_f16x
     constexpr int GROUPS = KS * FJ;                   // groups of FI NPROD matrix instructions of a slice
     __shared__ __align__(16) uint16_t As[RING][KS][2][2][TM + APAD][8];   // [slot][k / 16][part][k half][row]
     __shared__ __align__(16) uint16_t Ws[RING][PW][KS][2][TN + WPAD][8];
-    __shared__ int ae_tile[TM], we_tile[TN];
+    __shared__ int ae_tile[TM], we_tile[TN], wide_any[WM * WN];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wrow = wave / WN * (32 * FI), wcol = wave % WN * (32 * FJ);
     const int bm = blockIdx.y * TM, bn = blockIdx.x * TN;
@@ -196,8 +263,9 @@ __global__ __launch_bounds__(64 * WM * WN, (FI * FJ > 8 ? 1 : 2)) void gemm_f16x
     };
     static_assert(D % 2 == 0 && (64 / HK) % D == 0, "a piece of K is a whole number of turns of the register sets");
     static_assert(FI <= FJ, "a group of matrix instructions per row tile whose operands are read under it");
-    for (int i = tid; i < TM; i += T) ae_tile[i] = a.a_exp[min(bm + i, M - 1)];
-    for (int i = tid; i < TN; i += T) we_tile[i] = a.w_exp[min(bn + i, N - 1)];
+    int wide = 0;
+    for (int i = tid; i < TM; i += T) wide |= is_wide(ae_tile[i] = a.a_exp[min(bm + i, M - 1)]);
+    for (int i = tid; i < TN; i += T) wide |= is_wide(we_tile[i] = a.w_exp[min(bn + i, N - 1)]);
     auto fetch = [&](int r, int s) {
 #pragma unroll
         for (int i = 0; i < AST; ++i) fetch_a(r, i, min(s, n - 1));
@@ -221,7 +289,16 @@ __global__ __launch_bounds__(64 * WM * WN, (FI * FJ > 8 ? 1 : 2)) void gemm_f16x
         stage(1, 1);
         fetch(1, 3);
     }
+    wide = __any(wide);
+    if (lane == 0) wide_any[wave] = wide;
     __syncthreads();
+    wide = 0;
+#pragma unroll
+    for (int w = 0; w < WM * WN; ++w) wide |= wide_any[w];
+    if (wide) {
+        wide_tiles<WBF16, EPI, PARTIAL, FI, FJ>(a, ae_tile, we_tile, bm, bn, wrow, wcol, lane, s0 * HK, (s0 + n) * HK);
+        return;
+    }
     if (n > 0) {
 #pragma unroll
         for (int i = 0; i < FI; ++i) read_a(0, 0, 0, i);
@@ -238,14 +315,16 @@ __global__ __launch_bounds__(64 * WM * WN, (FI * FJ > 8 ? 1 : 2)) void gemm_f16x
             }
         }
     }
-    store_scaled_tiles<EPI, PARTIAL, FI, FJ>(a, acc, ae_tile, we_tile, bm, bn, wrow, wcol, lane);
+    store_tiles<EPI, PARTIAL, true, FI, FJ>(a, acc, ae_tile, we_tile, bm, bn, wrow, wcol, lane);
 }
 
 // Few rows of A (f32 rows).  The product is bound by the weights, which are streamed once and go straight into operand registers: a lane takes
 // two 16-byte pieces (bf16 weights: one) of its row per 32 of K, whose four lanes complete 64 bytes of every row, splits them there and multiplies
 // them by v_mfma_f32_16x16x32_f16 with the MT row tiles of A.  A workgroup's four wavefronts take 16 columns of C each and share A: chunks of 128 of K
 // lie in LDS in operand order, split on their way in, every row of a wavefront's share (EB blocks of 32 k) with an exponent of its own, found as it
-// passes; the sums of a share are scaled and added in f32.  What bounds it: the loads in flight (four blocks of W per wavefront; eight cost the
+// passes; the sums of a share are scaled and added in f32.  A chunk in which a lane's 8 or 16 values of A hold more than one that pairs would round away,
+// and all of a wavefront whose rows of W hold too many, are multiplied by f32 instructions: W from the same registers, A's f32 rows
+// from memory.  What bounds it: the loads in flight (four blocks of W per wavefront; eight cost the
 // occupancy what they gained: 4096 x 12288, bf16, 3 rows 24 -> 27 us, 23 rows of f32 spilled) and the barrier per chunk.  Before (the f32
 // instruction, 32 cycles per four of K instead of 32 or 48 per 32, or three bf16 products on whole tiles) and now, N x K, us:
 //     f32 weights, 23 rows:  11264 x 2048 38.6 -> 33    2048 x 5632 22.8 -> 20.2    2560 x 2048 12.1 -> 10.3    6144 x 1024 16.6 -> 14.7
@@ -260,6 +339,7 @@ __global__ __launch_bounds__(256, 3) void gemm_f16x2_stream_kernel(GemmArgs a) {
     constexpr int PIECES = 2 * MT;  // 16-byte pieces of A per thread and chunk
     __shared__ __align__(16) uint16_t As[2][SF_BLOCKS][MT][2][64][8];  // [half][block][tile][part][operand lane]
     __shared__ int ae[2][SF_BLOCKS / EB][MT][16];
+    __shared__ int wide_share[2][4];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int c = lane & 15, g = lane >> 4;
     const int M = a.M, N = a.N, K = a.K;
@@ -267,8 +347,9 @@ __global__ __launch_bounds__(256, 3) void gemm_f16x2_stream_kernel(GemmArgs a) {
     const int blocks = K / 32, per = (blocks + (int)gridDim.z - 1) / (int)gridDim.z;
     const int b0 = min((int)blockIdx.z * per, blocks), n = min(per, blocks - b0);
     const int col = bn + c, wrow = min(col, N - 1);
-    const int we = a.w_exp[wrow];
+    const int w_code = a.w_exp[wrow], we = code_exponent(w_code);
     const float ws = exp2_int(we);
+    const bool w_wide = __any(is_wide(w_code));
     const char *wp = (const char *)a.W + ((size_t)wrow * K + (size_t)b0 * 32) * (WBF16 ? 2 : 4) + g * 16;
     // this wavefront's share of a chunk of A: tile share_t, blocks share_b .. share_b + EB - 1; piece p of lane (row c, g): k 4 (4 p + g) of it
     const int share_t = MT == 2 ? wave >> 1 : 0, share_b = MT == 2 ? (wave & 1) * 2 : wave;
@@ -298,6 +379,22 @@ __global__ __launch_bounds__(256, 3) void gemm_f16x2_stream_kernel(GemmArgs a) {
         m = max(m, (unsigned)__shfl_xor((int)m, 32, 64));
         const int e = row_exponent(m);
         const float s = exp2_int(e);
+        const unsigned limit = small_limit(m);
+        unsigned least = ~0u;  // (a zero is the largest here)
+#pragma unroll
+        for (int p = 0; p < PIECES; ++p)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) least = min(least, magnitude_bits(va[p][i]) - 1u);
+        int wide = __any(least < limit - 1u);
+        if (wide) {  // uniform
+            int small = 0;
+#pragma unroll
+            for (int p = 0; p < PIECES; ++p)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) small += is_small(magnitude_bits(va[p][i]), limit);
+            wide = __any(small > 1);
+        }
+        if (lane == 0) wide_share[half][wave] = wide;
         if (g == 0) ae[half][share_b / EB][share_t][c] = e;
 #pragma unroll
         for (int p = 0; p < PIECES; ++p) {
@@ -319,7 +416,36 @@ __global__ __launch_bounds__(256, 3) void gemm_f16x2_stream_kernel(GemmArgs a) {
     __syncthreads();
     int half = 0;
     for (int d = 0; d < n; d += SF_BLOCKS, half ^= 1) {
+        const int wide = wide_share[half][0] | wide_share[half][1] | wide_share[half][2] | wide_share[half][3];
         fetch_a(d + SF_BLOCKS);
+        if (w_wide || __builtin_amdgcn_readlane(wide, 0)) {
+#pragma unroll
+            for (int j = 0; j < SF_BLOCKS; ++j) {
+                if (d + j >= n) break;
+                // instruction (i, e): element e of this lane's piece i of the block, of both operands
+                v4f ax[MT][2];
+#pragma unroll
+                for (int t = 0; t < MT; ++t) {
+                    const float *row = a.A + (size_t)min(t * 16 + c, M - 1) * K + (size_t)(b0 + d + j) * 32;
+#pragma unroll
+                    for (int i = 0; i < 2; ++i) ax[t][i] = *(const v4f *)(row + (WBF16 ? 8 * g + 4 * i : 16 * i + 4 * g));
+                }
+                float w[8];
+                if (WBF16) {
+                    const unsigned src[4] = {vw[j][0].x, vw[j][0].y, vw[j][0].z, vw[j][0].w};
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) w[e] = __uint_as_float(e & 1 ? src[e >> 1] & 0xffff0000u : src[e >> 1] << 16);
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) w[e] = __uint_as_float(vw[j][WP == 2 ? e >> 2 : 0][e & 3]);
+                }
+                fetch_w(j, d + j + SF_BLOCKS);
+#pragma unroll
+                for (int e = 0; e < 8; ++e)
+#pragma unroll
+                    for (int t = 0; t < MT; ++t) sum[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(ax[t][e >> 2][e & 3], w[e], sum[t], 0, 0, 0);
+            }
+        } else
 #pragma unroll
         for (int e0 = 0; e0 < SF_BLOCKS; e0 += EB) {
             v4f acc[MT];
@@ -365,7 +491,7 @@ __global__ __launch_bounds__(256, 3) void gemm_f16x2_stream_kernel(GemmArgs a) {
 #pragma unroll
             for (int t = 0; t < MT; ++t)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) sum[t][r] = fmaf(acc[t][r], exp2_int(-ae[half][e0 / EB][t][4 * g + r]), sum[t][r]);
+                for (int r = 0; r < 4; ++r) sum[t][r] += ldexpf(acc[t][r], -(ae[half][e0 / EB][t][4 * g + r] + we));
         }
         if (d + SF_BLOCKS < n) stage_a(half ^ 1);
         __syncthreads();
@@ -376,7 +502,7 @@ __global__ __launch_bounds__(256, 3) void gemm_f16x2_stream_kernel(GemmArgs a) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const int row = t * 16 + 4 * g + r;
-            const float v = ldexpf(sum[t][r], -we);
+            const float v = sum[t][r];
             if (PARTIAL) {
                 if (row < M && col < N) part[(size_t)row * N + col] = v;
             } else if (EPI == EPI_SWIGLU) {
@@ -390,57 +516,45 @@ __global__ __launch_bounds__(256, 3) void gemm_f16x2_stream_kernel(GemmArgs a) {
 }
 
 // ------------------------------------------------------------------------------------------ exponents, split rows
-// One wavefront per row of W.
+// One wavefront per row of W.  (The second pass over a row counts its small elements; it is paid once, when the weight is set.)
 template <bool BF16>
 __global__ __launch_bounds__(256) void row_exponents_kernel(const void *W, int rows, int cols, int row0, int step, int *exps) {
     const int r = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (r >= rows) return;
     const size_t row = (size_t)row0 + (size_t)r * step;
+    auto bits = [&](int k) { return BF16 ? (unsigned)(((const uint16_t *)W)[row * cols + k] & 0x7fffu) << 16 : magnitude_bits(((const float *)W)[row * cols + k]); };
     unsigned m = 0;
-    for (int k = lane; k < cols; k += 64)
-        m = max(m, BF16 ? (unsigned)(((const uint16_t *)W)[row * cols + k] & 0x7fffu) << 16 : magnitude_bits(((const float *)W)[row * cols + k]));
+    for (int k = lane; k < cols; k += 64) m = max(m, bits(k));
     m = wave_umax(m);
-    if (lane == 0) exps[row] = row_exponent(m);
+    const unsigned limit = small_limit<BF16 ? 31u : 18u>(m);
+    int small = 0;
+    for (int k = lane; k < cols; k += 64) small += is_small(bits(k), limit);
+    const bool wide = wave_sum((float)small) * (float)SPLIT_ROW_SMALL > (float)cols;
+    if (lane == 0) exps[row] = row_exponent(m) + (wide ? SPLIT_WIDE : 0);
 }
 
 // One workgroup per row, which is in registers before the first of it is stored (x and out may be the same).
 template <int VPT>
 __global__ __launch_bounds__(256) void split_rows_kernel(const float *x, int dim, float *out, int *exps) {
-    __shared__ unsigned top[4];
     const int tid = threadIdx.x;
     const size_t base = (size_t)blockIdx.x * dim;
     v4f v[VPT];
-    unsigned m = 0;
 #pragma unroll
     for (int i = 0; i < VPT; ++i) {
         const int k = (tid + i * 256) * 4;
         v[i] = v4f{0.f, 0.f, 0.f, 0.f};
         if (k < dim) v[i] = *(const v4f *)(x + base + k);
     }
-#pragma unroll
-    for (int i = 0; i < VPT; ++i) m = max(m, magnitude_bits(v[i]));
-    m = wave_umax(m);
-    if ((tid & 63) == 0) top[tid >> 6] = m;
-    __syncthreads();
-    const int e = row_exponent(max(max(top[0], top[1]), max(top[2], top[3])));
-    const float s = exp2_int(e);
-    if (tid == 0) exps[blockIdx.x] = e;
-#pragma unroll
-    for (int i = 0; i < VPT; ++i) {
-        const int k = (tid + i * 256) * 4;
-        if (k < dim) store_split4((uint16_t *)(out + base), k, v[i], s);
-    }
+    leave_row<VPT>(v, dim, out + base, exps + blockIdx.x);
 }
 
 // Adds the K splits of a gate|up product in split order, applies silu(gate) * up and leaves the row split: one workgroup of 1024 per row
 // (a few hundred rows: what counts is that a thread has at most VPT trips to memory).
 template <int VPT>
 __global__ __launch_bounds__(1024) void reduce_swiglu_split_kernel(GemmArgs a, int splits) {
-    __shared__ unsigned top[16];
     const int tid = threadIdx.x, I = a.N >> 1;
     const size_t MN = (size_t)a.M * a.N, base = (size_t)blockIdx.x * a.N;
     v4f v[VPT];
-    unsigned m = 0;
 #pragma unroll
     for (int i = 0; i < VPT; ++i) {
         const int k = (tid + i * 1024) * 4;  // of the I results; gate and up alternate in the product's columns
@@ -455,23 +569,9 @@ __global__ __launch_bounds__(1024) void reduce_swiglu_split_kernel(GemmArgs a, i
             }
             v[i] = v4f{p0.x / (1.0f + expf(-p0.x)) * p0.y, p0.z / (1.0f + expf(-p0.z)) * p0.w, p1.x / (1.0f + expf(-p1.x)) * p1.y,
                        p1.z / (1.0f + expf(-p1.z)) * p1.w};
-            m = max(m, magnitude_bits(v[i]));
         }
     }
-    m = wave_umax(m);
-    if ((tid & 63) == 0) top[tid >> 6] = m;
-    __syncthreads();
-    m = 0;
-#pragma unroll
-    for (int w = 0; w < 16; ++w) m = max(m, top[w]);
-    const int e = row_exponent(m);
-    const float s = exp2_int(e);
-    if (tid == 0) a.c_exp[blockIdx.x] = e;
-#pragma unroll
-    for (int i = 0; i < VPT; ++i) {
-        const int k = (tid + i * 1024) * 4;
-        if (k < I) store_split4((uint16_t *)(a.C + (size_t)blockIdx.x * I), k, v[i], s);
-    }
+    leave_row<VPT>(v, I, a.C + (size_t)blockIdx.x * I, a.c_exp + blockIdx.x);
 }
 
 int launch_row_exponents(lumen_ctx *ctx, const void *W, int w_bf16, int rows, int cols, int row0, int step, int *exps) {

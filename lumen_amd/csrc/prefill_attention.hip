@@ -444,7 +444,6 @@ __global__ __launch_bounds__(FA_THREADS, 2) void attn_prefill_f16x2_kernel(AttnP
 // row of a position and leaves it split, with an exponent of its own.
 template <bool SPLIT>
 __global__ __launch_bounds__(1024) void merge_parts_kernel(AttnPrefillArgs a, int parts) {
-    __shared__ unsigned wave_top[16];
     const int per_pos = a.hq * a.d / 4, at = (int)(blockIdx.y * blockDim.x + threadIdx.x), tid = threadIdx.x;
     const size_t pos = (size_t)blockIdx.z * a.s + blockIdx.x;
     v4f o = {0.f, 0.f, 0.f, 0.f};
@@ -470,14 +469,8 @@ __global__ __launch_bounds__(1024) void merge_parts_kernel(AttnPrefillArgs a, in
         if (at < per_pos) *(v4f *)(row + at * 4) = o;
         return;
     }
-    const unsigned mine = wave_umax(magnitude_bits(o));
-    if ((tid & 63) == 0) wave_top[tid >> 6] = mine;
-    __syncthreads();
-    unsigned top = 0;
-    for (int w = 0; w < (int)blockDim.x >> 6; ++w) top = max(top, wave_top[w]);
-    const int e = row_exponent(top);
-    if (tid == 0) a.out_exp[pos] = e;
-    if (at < per_pos) store_split4((uint16_t *)row, at * 4, o, exp2_int(e));
+    const v4f all[1] = {o};
+    leave_row<1>(all, per_pos * 4, row, a.out_exp + pos);
 }
 
 // Parts the keys are cut into where the blocks of queries leave compute units idle: at least 128 keys each (two trips of the loop; a part costs

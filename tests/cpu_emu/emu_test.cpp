@@ -5,9 +5,10 @@
 // attention workgroups per head (slices + fold), rotated and un-rotated (q/k-norm) hand-over, f32 and bf16 weights;
 // the gate|up -> down chain; the few-row product of short prompts with ragged shapes and all three epilogues; the
 // streaming vector-matrix product and the stand-alone decode attention those forms fall back to, the latter also
-// at operator level over a sliced cache (slices merged inside the launch); prompt attention of two caches, one of them recorded.
+// at operator level over a sliced cache (slices merged inside the launch); prompt attention of two caches, one of them recorded; the products on f16 pairs, with rows that
+// pairs cannot hold.
 //
-//   emu_test [case ...]      cases: chain sliced qknorm bf16 skinny attn layerop shapes caches (default: all)
+//   emu_test [case ...]      cases: chain sliced qknorm bf16 skinny attn layerop shapes caches pairs ranges (default: all)
 #include <math.h>
 #include <stdio.h>
 #include <stdlib.h>
@@ -18,7 +19,7 @@
 
 #include <hip/hip_runtime.h>
 
-#include "../../include/lumen_hip.h"
+#include "internal.h"
 extern "C" {
 #include "lumen_oracle.h"
 }
@@ -84,9 +85,24 @@ struct Model {
     int D = 0;
 };
 
+// not 0: channels 2^g_hide above the others that the next product multiplies by zero -- a channel of every norm's gain, of the values (head dimension
+// element 9, one KV head) and of the up projection
+static int g_hide = 0;
+static void hide(std::vector<float> &v, const std::string &name, size_t rows, size_t cols, int D) {
+    auto has = [&](const char *s) { return name.find(s) != std::string::npos; };
+    const float f = ldexpf(1.f, g_hide);
+    if (!cols) v[3] = f;
+    else if (has("down_proj")) for (size_t r = 0; r < rows; ++r) v[r * cols + 11] = 0.f;
+    else if (has("o_proj")) for (size_t i = 0; i < rows * cols; ++i) v[i] = (int)(i % cols) % D == 9 ? 0.f : v[i];
+    else if (!has("embed")) for (size_t r = 0; r < rows; ++r) v[r * cols + 3] = 0.f;
+    if (has("v_proj") || has("up_proj"))
+        for (size_t k = 0; k < cols; ++k) v[(has("v_proj") ? 9 : 11) * cols + k] *= f;
+}
+
 static const float *param(Model &m, const std::string &name, size_t rows, size_t cols, float std_, float mean, bool bf16) {
     m.keep.push_back(randn(rows * (cols ? cols : 1), std_, mean));
     std::vector<float> &v = m.keep.back();
+    if (g_hide) hide(v, name, rows, cols, m.D);
     if (bf16 && cols) to_bf16_values(v);
     const int64_t shape[2] = {(int64_t)rows, (int64_t)cols};
     OK(lumen_llama_set_param(m.gpu, name.c_str(), v.data(), LUMEN_DTYPE_F32, shape, cols ? 2 : 1));
@@ -517,6 +533,113 @@ static void case_caches(lumen_ctx *ctx) {
     OK(lumen_rope_destroy(rope));
 }
 
+// The products on f16 pairs by themselves: whole tiles of both sizes with and without K splits, few rows, edges of tiles, one piece of K and
+// several; then with rows pairs cannot hold (an element 2^30 above the others that the other operand multiplies by zero): in A, in W, in both, in
+// some rows of a tile only.  Against sums in 64 bits, 1e-6 of the largest result: sums of 320 f32 terms.
+static void case_pairs(lumen_ctx *ctx) {
+    printf("pairs: products on f16 pairs, whole tiles and few rows\n");
+    struct Shape { int M, N, K, big, splits, epi; };  // big < 0: the few-row kernel
+    const Shape shapes[] = {{33, 70, 64, 0, 1, EPI_STORE},    {129, 130, 128, 0, 1, EPI_SWIGLU}, {127, 257, 192, 0, 2, EPI_STORE},  {48, 64, 320, 0, 3, EPI_STORE},
+                            {65, 131, 64, 0, 1, EPI_RESIDUAL}, {33, 70, 64, 1, 1, EPI_STORE},    {257, 130, 128, 1, 1, EPI_SWIGLU}, {255, 259, 192, 1, 2, EPI_STORE},
+                            {129, 300, 64, 1, 1, EPI_RESIDUAL}, {3, 70, 64, -1, 1, EPI_STORE},   {16, 130, 320, -1, 1, EPI_SWIGLU}, {17, 65, 320, -1, 3, EPI_STORE},
+                            {32, 129, 128, -1, 1, EPI_RESIDUAL}};
+    double worst[2] = {0, 0};
+    for (const Shape &t : shapes)
+        for (int bf16 = 0; bf16 < 2; ++bf16)
+            for (int wide = 0; wide < 4; ++wide) {  // bit 0: rows of A, bit 1: rows of W
+                if (t.big < 0 && !bf16 && t.M <= 16) continue;  // (two row tiles always: 17 rows stand for these)
+                const int M = t.M, N = t.N, K = t.K, hid_a = 5, hid_w = K - 2;
+                std::vector<float> A = randn((size_t)M * K, 1.f), W = randn((size_t)N * K, 0.1f), R = randn((size_t)M * N, 1.f);
+                for (int i = 0; i < M; ++i) {
+                    A[(size_t)i * K + hid_w] = 0.f;
+                    if ((wide & 1) && i % 3 == 1) A[(size_t)i * K + hid_a] = ldexpf(1.f, 30);
+                }
+                for (int j = 0; j < N; ++j) {
+                    W[(size_t)j * K + hid_a] = 0.f;
+                    if ((wide & 2) && j % 5 == 1) W[(size_t)j * K + hid_w] = ldexpf(1.f, bf16 ? 40 : 30);
+                }
+                std::vector<uint16_t> bits(W.size());
+                if (bf16) {
+                    to_bf16_values(W);
+                    for (size_t i = 0; i < W.size(); ++i) {
+                        uint32_t u;
+                        memcpy(&u, &W[i], 4);
+                        bits[i] = (uint16_t)(u >> 16);
+                    }
+                }
+                const size_t c_n = (size_t)M * (t.epi == EPI_SWIGLU ? N / 2 : N);
+                void *dA, *dW, *dC, *dR, *dP, *dS, *ea, *ew;
+                OK(lumen_malloc(ctx, A.size() * 4, &dA));
+                OK(lumen_malloc(ctx, A.size() * 4, &dS));
+                OK(lumen_malloc(ctx, W.size() * (bf16 ? 2 : 4), &dW));
+                OK(lumen_malloc(ctx, c_n * 4, &dC));
+                OK(lumen_malloc(ctx, R.size() * 4, &dR));
+                OK(lumen_malloc(ctx, (size_t)t.splits * M * N * 4, &dP));
+                OK(lumen_malloc(ctx, (size_t)M * 4, &ea));
+                OK(lumen_malloc(ctx, (size_t)N * 4, &ew));
+                OK(lumen_upload(ctx, dA, A.data(), A.size() * 4));
+                OK(lumen_upload(ctx, dW, bf16 ? (const void *)bits.data() : W.data(), W.size() * (bf16 ? 2 : 4)));
+                OK(lumen_upload(ctx, dR, R.data(), R.size() * 4));
+                OK(launch_row_exponents(ctx, dW, bf16, N, K, 0, 1, (int *)ew));
+                GemmArgs g = {};
+                g.A = (const float *)dA; g.W = dW; g.C = (float *)dC; g.M = M; g.N = N; g.K = K; g.w_bf16 = bf16; g.epi = t.epi;
+                g.residual = (const float *)dR; g.alpha = 0.5f; g.part = (float *)dP; g.w_exp = (const int *)ew;
+                if (t.big >= 0) {
+                    OK(launch_split_rows(ctx, (const float *)dA, M, K, (float *)dS, (int *)ea));
+                    g.a_split = (const uint16_t *)dS;
+                    g.a_exp = (const int *)ea;
+                    launch_gemm_f16x2(g, SplitPlan{t.big != 0, t.splits}, nullptr);
+                } else {
+                    launch_gemm_f16x2_stream(g, t.splits, nullptr);
+                }
+                std::vector<float> C(c_n), P((size_t)t.splits * M * N);
+                OK(lumen_download(ctx, C.data(), dC, C.size() * 4));
+                OK(lumen_download(ctx, P.data(), dP, P.size() * 4));
+                double e = 0, scale = 1e-30;
+                std::vector<double> row(N);
+                for (int i = 0; i < M; ++i) {
+                    for (int j = 0; j < N; ++j) {
+                        row[j] = 0;
+                        for (int k = 0; k < K; ++k) row[j] += (double)A[(size_t)i * K + k] * W[(size_t)j * K + k];
+                    }
+                    for (int j = 0; j < (t.epi == EPI_SWIGLU ? N / 2 : N); ++j) {
+                        double want = row[j], got = 0;
+                        if (t.splits > 1) for (int s = 0; s < t.splits; ++s) got += P[((size_t)s * M + i) * N + j];
+                        else if (t.epi == EPI_SWIGLU) got = C[(size_t)i * (N / 2) + j];
+                        else got = C[(size_t)i * N + j];
+                        if (t.epi == EPI_SWIGLU) want = row[2 * j] / (1 + exp(-row[2 * j])) * row[2 * j + 1];
+                        else if (t.epi == EPI_RESIDUAL) want = want * 0.5 + R[(size_t)i * N + j];
+                        scale = fmax(scale, fabs(want));
+                        e = fmax(e, isnan(got) ? INFINITY : fabs(got - want));
+                    }
+                }
+                e /= scale;
+                worst[wide != 0] = fmax(worst[wide != 0], e);
+                CHECK(e <= 1e-6, "%d x %d x %d%s, %s tiles, %d split(s), wide rows %d: %.3g", M, N, K, bf16 ? " bf16 weights" : "",
+                      t.big < 0 ? "no" : t.big ? "large" : "small", t.splits, wide, e);
+                for (void *p : {dA, dS, dW, dC, dR, dP, ea, ew}) OK(lumen_free(ctx, p));
+            }
+    printf("  worst error of the largest result %.2e, with wide rows %.2e\n", worst[0], worst[1]);
+}
+
+// Every row-producing step of a prompt pass leaves an element 2^24 above the others that the next product multiplies by zero.
+static void case_ranges(lumen_ctx *ctx) {
+    printf("ranges: hidden channels of other magnitudes through whole prompt passes\n");
+    for (int bf16 = 0; bf16 < 2; ++bf16) {
+        g_hide = 24;
+        Model m = build(ctx, 67, 128, 192, 1, 2, 1, 0, 160, false, false, bf16 != 0);
+        g_hide = 0;
+        for (int rows : {17, 50, 98}) {
+            std::vector<int> ids(rows);
+            for (int i = 0; i < rows; ++i) ids[i] = (i * 29 + 3) % 67;
+            OK(lumen_llama_reset(m.gpu));
+            lo_llama_reset(m.ora);
+            forward_both(m, ids, 1e-5, bf16 ? "hidden channels, bf16 weights" : "hidden channels");
+        }
+        destroy(m);
+    }
+}
+
 int main(int argc, char **argv) {
     lo_set_threads(4);
     lumen_ctx *ctx = nullptr;
@@ -526,7 +649,8 @@ int main(int argc, char **argv) {
         return 0;  // (reached only if nothing stopped the program: the test expects a sanitizer report instead)
     }
     struct { const char *name; void (*fn)(lumen_ctx *); } cases[] = {
-        {"chain", case_chain}, {"sliced", case_sliced}, {"qknorm", case_qknorm}, {"bf16", case_bf16}, {"skinny", case_skinny}, {"attn", case_attn}, {"layerop", case_layerop}, {"shapes", case_shapes}, {"caches", case_caches}};
+        {"chain", case_chain}, {"sliced", case_sliced}, {"qknorm", case_qknorm}, {"bf16", case_bf16}, {"skinny", case_skinny}, {"attn", case_attn}, {"layerop", case_layerop}, {"shapes", case_shapes}, {"caches", case_caches}, {"pairs", case_pairs},
+        {"ranges", case_ranges}};
     for (const auto &c : cases) {
         bool run = argc <= 1;
         for (int i = 1; i < argc; ++i) run = run || !strcmp(argv[i], c.name);

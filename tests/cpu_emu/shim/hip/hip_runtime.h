@@ -52,6 +52,7 @@ void yield();
 
 // ------------------------------------------------------------------ device builtins
 static inline void __syncthreads() { emu::workgroup_barrier(); }
+static inline void __threadfence() {}  // (stores take place in order here)
 template <typename T>
 static inline T emu_bits_to(uint32_t u) {
     static_assert(sizeof(T) == 4, "32-bit values only");

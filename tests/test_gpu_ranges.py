@@ -6,11 +6,14 @@ by itself, at any factor."""
 import numpy as np
 import pytest
 
+from lumen_amd import synth
 from lumen_amd._lib import check, lib
 from lumen_amd.autograd import Tensor
 from lumen_amd.layers import KVCacheInner, RotaryEmbedding
+from lumen_amd.models import LlamaModel
 from oracle import lumen_oracle as lo
-from tests.gpu_util import dev
+from tests import hybrid_util, nufapel_util
+from tests.gpu_util import dev, max_rel
 
 pytestmark = pytest.mark.gpu
 
@@ -86,3 +89,78 @@ def test_attention_without_a_mask(d, h, h_kv, past, s, batch):
     """All keys for every position, keys in parts and in one, also with tiles that lie far apart in magnitude."""
     for change in (lambda q, k, v: None, later("v", past + s - 20, -30), later("v", past + s - 20, 30)):
         assert row_error(*attention_rows(d, h, h_kv, past, s, change, causal=False, batch=batch)) <= 2e-5
+
+
+def hide(params, e, dim, weights_only):
+    """Channels 2^e above the others that the next product multiplies by zero: one of every norm's gain (weights_only: the weights are the large ones and
+    the gain is zero), one of every KV head's values, one of the up projection; in the up projection's case every third row of its input weights too."""
+    f = np.float32(2.0 ** e)
+    for n, a in params.items():
+        if a.ndim == 1:
+            a[3] = 0 if weights_only else f
+        elif "down_proj" in n:
+            a[:, 11] = 0
+        elif "o_proj" in n:
+            a[:, 9::dim] = 0
+        elif "embed" not in n:
+            a[:, 3] = 0
+            if weights_only:
+                a[1::3, 3] = f
+        if "v_proj" in n:
+            a[9::dim] *= f
+        elif "up_proj" in n:
+            a[11] *= f
+
+
+@pytest.mark.parametrize("e", [16, 20, 24, 30, 40])
+@pytest.mark.parametrize("weights_only", [False, True], ids=["rows", "weights"])
+@pytest.mark.parametrize("bf16", [False, True], ids=["f32", "bf16"])
+@pytest.mark.parametrize("hidden,inter,heads,kv_heads,vocab,rows", [
+    (256, 448, 4, 2, 301, (3, 17, 32, 33, 130)), (1024, 2816, 16, 4, 301, (4, 20, 50)), (128, 320, 2, 1, 82001, (24, 400))])
+def test_prompt_with_hidden_channels(hidden, inter, heads, kv_heads, vocab, rows, bf16, weights_only, e):
+    """Few rows and tiles, f32 and bf16-stored weights (a channel of values stays below what the attention's own test covers)."""
+    cfg = dict(vocab_size=vocab, hidden_size=hidden, intermediate_size=inter, num_hidden_layers=1, num_attention_heads=heads,
+               num_key_value_heads=kv_heads, rms_norm_eps=1e-5, max_seq_len=416, rope_theta=10000.0)
+    params = synth.make_params(cfg, seed=5, std=0.05, gains_one=False)
+    hide(params, e, hidden // heads, weights_only)
+    gcfg, bits = dict(cfg), {}
+    if bf16:
+        gcfg["weight_dtype"] = "bf16"
+        bits = {n: synth.bf16_round(a).reshape(a.shape) for n, a in params.items() if a.ndim == 2}
+        params = {n: synth.bf16_widen(bits[n]) if n in bits else a for n, a in params.items()}
+    gpu, ora = LlamaModel(gcfg), lo.Llama(cfg, params)
+    for n, a in params.items():
+        gpu.set_param(n, bits.get(n, a))
+    for s in rows:
+        ids = synth.make_tokens(s, vocab, seed=s)
+        gpu.reset_kv_caches()
+        ora.reset()
+        got = gpu.forward(ids, all_rows=True)
+        rc, ref = ora.forward(ids)
+        assert rc == lo.LO_OK
+        assert row_error(got, ref) <= 2e-5, s
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("e", [24, 40])
+@pytest.mark.parametrize("name,tokens", [("pinavik", 320), ("nufapel", 449)])
+def test_hybrid_prompt_with_a_hidden_channel(tmp_path, name, tokens, e, dtype):
+    """A channel of every norm's gain 2^e above the others, zero in every matrix that reads the norm: the prompt at once, on split rows where they
+    are taken, against portions of two tokens, which take the f32 ones."""
+    f = np.float32(2.0 ** e)
+    if name == "pinavik":
+        util, cfg = hybrid_util, hybrid_util.config(1024, 307, [hybrid_util.attention(4, 2, 32, 32, 50, ff=320), hybrid_util.wkv(4, 32, ff=100),
+                                                                hybrid_util.delta(2, 1, 64, 32, ff=192)])
+    else:
+        util, cfg = nufapel_util, nufapel_util.config(1024, 307, [nufapel_util.parallel((4, 2, 32, 32), (2, 64, 64), nufapel_util.dense(320)),
+                                                                  nufapel_util.general(4, 32, nufapel_util.dense(100))])
+    params = util.make_params(cfg, seed=4)
+    for n, a in params.items():
+        if a.ndim == 1 and a.shape[0] == 1024 and n.endswith(("norm1", "norm2")):
+            a[3] = f
+        elif a.ndim == 2 and a.shape[1] == 1024 and n[0] == "l" and n[1].isdigit():
+            a[:, 3] = 0
+    model = hybrid_util.load(tmp_path, cfg, params, dtype)
+    ids = synth.make_tokens(tokens, 307, seed=tokens)
+    at_once, portions = (hybrid_util.run(model, ids, cuts) for cuts in ([tokens], [2]))
+    assert max_rel(at_once, portions) <= 2e-5
