@@ -25,10 +25,8 @@ if ROOT not in sys.path:
 HBM_PEAK_GBS = 8000.0  # MI355X published HBM3E bandwidth
 MFMA_FP32_PEAK_TF = 157.3  # MI355X dense fp32 matrix peak, TFLOP/s
 MFMA_BF16_PEAK_TF = 2500.0  # MI355X dense bf16 matrix peak, TFLOP/s
-# the operator's GEMM takes an f32 product as six bf16 matrix products (three bf16 parts per f32 value), the models' prompt passes
-# as three f16 ones (pairs of f16, the same matrix rate)
+# the operator's GEMM takes an f32 product as six bf16 matrix products (three bf16 parts per f32 value)
 GEMM_BF16_PRODUCTS = 6
-PROMPT_F16_PRODUCTS = 3
 
 
 def main():
@@ -280,6 +278,22 @@ def decode_bench(model_name, cfg, n_prompt, steps, warmup, mode, keep_host, head
     return out, model, params, prompt
 
 
+def prompt_products(cfg, S):
+    """16-bit matrix products that the GEMMs of an S-row prompt take per f32 product (None: they do not run on 16-bit matrix instructions, or not
+    all in the same way), and in words what they run on: the row limits of gemm.hip (gemm_takes_split, stream_pairs_shape)."""
+    bf16 = cfg.get("weight_dtype") == "bf16"
+    pairs = "f32 values as 2 f16 parts with an exponent per row, %d f16 matrix products per f32 product" % (2 if bf16 else 3)
+    if S > (47 if bf16 else 32):
+        return (2 if bf16 else 3), "GEMM: %s (v_mfma_f32_32x32x16_f16)" % pairs
+    if S > 32:
+        return 3, "GEMM: f32 values as 3 bf16 parts, 3 v_mfma_f32_32x32x16_bf16 products per f32 product with bf16-stored weights"
+    if S > 2 and bf16:
+        return 2, "GEMM: %s (v_mfma_f32_16x16x32_f16, weights straight from memory)" % pairs
+    if S > 16:
+        return None, "GEMM: matrices of 5 Mi weights or more %s (v_mfma_f32_16x16x32_f16), smaller ones v_mfma_f32_16x16x4_f32" % pairs
+    return None, "GEMM: v_mfma_f32_16x16x4_f32" if S > 2 else "GEMM: vector ALU"
+
+
 def prefill_report(cfg, S, ms):
     """Prompt pass: tokens/s and the share of the fp32 matrix-core peak its GEMM flops amount to
     (all projections on S rows, lm_head on the last row only, causal attention counted once)."""
@@ -290,14 +304,14 @@ def prefill_report(cfg, S, ms):
     gemm_flops = 2.0 * S * L * per_layer + 2.0 * V * H
     attn_flops = 4.0 * L * hq * D * S * S / 2.0
     tf = (gemm_flops + attn_flops) / (ms * 1e-3) / 1e12
-    issued = (PROMPT_F16_PRODUCTS * gemm_flops) / (ms * 1e-3) / 1e12  # f16 matrix flops the GEMMs issue (bf16 rate)
+    products, path = prompt_products(cfg, S)
+    issued = products * gemm_flops / (ms * 1e-3) / 1e12 if products else None  # 16-bit matrix flops the GEMMs issue
     return {"tokens": S, "ms": round(ms, 3), "tokens_per_s": round(S / ms * 1e3, 1),
             "gemm_flops": gemm_flops, "attention_flops": attn_flops, "achieved_TFLOPs": round(tf, 2),
-            "matrix_path": "GEMM: f32 values as 2 f16 parts with an exponent per row, 3 v_mfma_f32_32x32x16_f16 products per f32 product; "
-                           "attention: the same scheme",
+            "matrix_path": path,
             "mfma_fp32_peak_TFLOPs": MFMA_FP32_PEAK_TF, "vs_mfma_fp32_peak": round(tf / MFMA_FP32_PEAK_TF, 4),
-            "gemm_bf16_TFLOPs_issued": round(issued, 1), "mfma_bf16_peak_TFLOPs": MFMA_BF16_PEAK_TF,
-            "frac_of_mfma_bf16_peak": round(issued / MFMA_BF16_PEAK_TF, 4)}
+            "gemm_bf16_TFLOPs_issued": round(issued, 1) if products else None, "mfma_bf16_peak_TFLOPs": MFMA_BF16_PEAK_TF,
+            "frac_of_mfma_bf16_peak": round(issued / MFMA_BF16_PEAK_TF, 4) if products else None}
 
 
 def measured_traffic(kernel):
