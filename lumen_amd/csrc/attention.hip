@@ -568,7 +568,10 @@ static int launch_prefill_d(lumen_ctx *ctx, const AttnPrefillArgs &a) {
     if (attn_prefill_mfma_supported(a)) return launch_attn_prefill_mfma(ctx, a);  // head_dim 64 / 128: matrix cores
     // One workgroup per position and one or two query heads of a KV group: the rows the heads of a group share come from L2, and a workgroup's walk
     // over the keys is short.  (One workgroup for the 8 heads of a group: 23.6 us at 23 positions behind 301 cached ones, 162 behind 3000;
-    // one head each 11.6 and 74, two 12.3 and 70; at 64 positions 25.5 / 165, one 19.9 / 122, two 18.1 / 105.)
+    // one head each 11.6 and 74, two 12.3 and 70; at 64 positions 25.5 / 165, one 19.9 / 122, two 18.1 / 105.)  Heads of 16 and 32 take this kernel at any
+    // length; the whole group / this rule, us: 32 heads of 32 in groups of 8, 23 positions behind 300 24 / 9.6, 96 first 13.3 / 10.6, 512 68 / 54,
+    // 2048 608 / 511; 32 of 16 in groups of 8, 512 45 / 38, 2048 318 / 288; 16 of 32 in groups of 4, 512 34.5 / 31.5, 2048 281 / 285 (four heads
+    // per workgroup there: 283).
     const int nrep = a.hq / a.hkv, per = nrep % 2 == 0 && (long)a.s * a.hq * a.b > 3L * ctx->num_cus ? 2 : 1;
     AttnPrefillArgs b = a;
     b.kv_div = nrep / per;
