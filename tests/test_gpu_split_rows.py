@@ -75,8 +75,11 @@ def test_prompts_of_few_rows(cfg, rows, bf16):
     (config(128, 192, 4, 1, vocab=257), (127, 128, 129)),
     (config(320, 704, 5, 5), (255, 257, 300)),         # columns that fill no tile, several pieces, K splits
     (config(256, 320, 2, 1), (96, 161)),               # heads of 128
-    (config(1024, 2816, 16, 4, layers=1, max_seq=1152), (1101,)),  # large tiles
-], ids=["64", "128", "320", "256", "1024"])
+    (config(1024, 2816, 16, 4, layers=1, max_seq=1152), (1101,)),  # many tiles of 128
+    # 256 x 256 tiles: gate|up (32000 columns) and head (32001), whole K, four rows of tiles of which the last holds 132
+    (config(128, 16000, 2, 1, layers=1, vocab=32001, max_seq=1024), (900,)),
+    (config(1024, 16384, 16, 4, layers=1, max_seq=1024), (897,)),  # ... and K in 16: down (16384 inner values)
+], ids=["64", "128", "320", "256", "1024", "wide", "deep"])
 def test_prompts_at_the_edges_of_tiles(cfg, rows, bf16):
     gpu, ora = build(cfg, bf16)
     for s in rows:
