@@ -322,15 +322,16 @@ __global__ __launch_bounds__(64 * WM * WN, (FI * FJ > 8 ? 1 : 2)) void gemm_f16x
 // two 16-byte pieces (bf16 weights: one) of its row per 32 of K, whose four lanes complete 64 bytes of every row, splits them there and multiplies
 // them by v_mfma_f32_16x16x32_f16 with the MT row tiles of A.  A workgroup's four wavefronts take 16 columns of C each and share A: chunks of 128 of K
 // lie in LDS in operand order, split on their way in, every row of a wavefront's share (EB blocks of 32 k) with an exponent of its own, found as it
-// passes; the sums of a share are scaled and added in f32.  A chunk in which a lane's 8 or 16 values of A hold more than one that pairs would round away,
-// and all of a wavefront whose rows of W hold too many, are multiplied by f32 instructions: W from the same registers, A's f32 rows
-// from memory.  What bounds it: the loads in flight (four blocks of W per wavefront; eight cost the
+// passes; the sums of a share are scaled and added in f32.  A workgroup that met a share with more than SF_SMALL small values (f16_split.h) per 32, or a
+// marked row of W, takes its range again by f32 instructions on the f32 values, straight from memory (a choice per chunk costs every launch 4 %:
+// the branch stands between a chunk's barrier and its first operands).  What bounds it: the loads in flight (four blocks of W per wavefront; eight cost the
 // occupancy what they gained: 4096 x 12288, bf16, 3 rows 24 -> 27 us, 23 rows of f32 spilled) and the barrier per chunk.  Before (the f32
 // instruction, 32 cycles per four of K instead of 32 or 48 per 32, or three bf16 products on whole tiles) and now, N x K, us:
 //     f32 weights, 23 rows:  11264 x 2048 38.6 -> 33    2048 x 5632 22.8 -> 20.2    2560 x 2048 12.1 -> 10.3    6144 x 1024 16.6 -> 14.7
 //     bf16, 3-32 rows:       12288 x 4096 38 -> 24-34   4096 x 4096 19 -> 13-16     22016 x 4096 72 -> 47-66    4096 x 11008 42 -> 27-35
 // Error against 64 bits before and now, relative to the root mean square of C (f32 weights; half as many or fewer sums are rounded):
 //     16 rows 11264 x 2048 4.1e-7 -> 1.4e-7    23 rows 2048 x 5632 2.9e-7 -> 1.5e-7    3 rows 1000 x 192 1.3e-7 -> 0.9e-7
+#define SF_SMALL 2
 #define SF_BLOCKS 4  // blocks of 32 k in a chunk, and of W in flight per wavefront
 template <bool WBF16, int MT, int EPI, bool PARTIAL>
 __global__ __launch_bounds__(256, 3) void gemm_f16x2_stream_kernel(GemmArgs a) {
@@ -339,7 +340,7 @@ __global__ __launch_bounds__(256, 3) void gemm_f16x2_stream_kernel(GemmArgs a) {
     constexpr int PIECES = 2 * MT;  // 16-byte pieces of A per thread and chunk
     __shared__ __align__(16) uint16_t As[2][SF_BLOCKS][MT][2][64][8];  // [half][block][tile][part][operand lane]
     __shared__ int ae[2][SF_BLOCKS / EB][MT][16];
-    __shared__ int wide_share[2][4];
+    __shared__ int wide_any[4];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int c = lane & 15, g = lane >> 4;
     const int M = a.M, N = a.N, K = a.K;
@@ -349,7 +350,7 @@ __global__ __launch_bounds__(256, 3) void gemm_f16x2_stream_kernel(GemmArgs a) {
     const int col = bn + c, wrow = min(col, N - 1);
     const int w_code = a.w_exp[wrow], we = code_exponent(w_code);
     const float ws = exp2_int(we);
-    const bool w_wide = __any(is_wide(w_code));
+    int wide = __any(is_wide(w_code));
     const char *wp = (const char *)a.W + ((size_t)wrow * K + (size_t)b0 * 32) * (WBF16 ? 2 : 4) + g * 16;
     // this wavefront's share of a chunk of A: tile share_t, blocks share_b .. share_b + EB - 1; piece p of lane (row c, g): k 4 (4 p + g) of it
     const int share_t = MT == 2 ? wave >> 1 : 0, share_b = MT == 2 ? (wave & 1) * 2 : wave;
@@ -372,29 +373,30 @@ __global__ __launch_bounds__(256, 3) void gemm_f16x2_stream_kernel(GemmArgs a) {
         }
     };
     auto stage_a = [&](int half) {
-        unsigned m = 0;
+        unsigned m = 0, least = ~0u;  // (of magnitudes - 1: a zero is the largest)
 #pragma unroll
-        for (int p = 0; p < PIECES; ++p) m = max(m, magnitude_bits(va[p]));
+        for (int p = 0; p < PIECES; ++p)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const unsigned u = magnitude_bits(va[p][i]);
+                m = max(m, u);
+                least = min(least, u - 1u);
+            }
         m = max(m, (unsigned)__shfl_xor((int)m, 16, 64));
         m = max(m, (unsigned)__shfl_xor((int)m, 32, 64));
         const int e = row_exponent(m);
         const float s = exp2_int(e);
         const unsigned limit = small_limit(m);
-        unsigned least = ~0u;  // (a zero is the largest here)
-#pragma unroll
-        for (int p = 0; p < PIECES; ++p)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) least = min(least, magnitude_bits(va[p][i]) - 1u);
-        int wide = __any(least < limit - 1u);
-        if (wide) {  // uniform
+        if (__any(least < limit - 1u)) {  // uniform
             int small = 0;
 #pragma unroll
             for (int p = 0; p < PIECES; ++p)
 #pragma unroll
                 for (int i = 0; i < 4; ++i) small += is_small(magnitude_bits(va[p][i]), limit);
-            wide = __any(small > 1);
+            small += __shfl_xor(small, 16, 64);
+            small += __shfl_xor(small, 32, 64);
+            wide |= __any(small > SF_SMALL * EB);
         }
-        if (lane == 0) wide_share[half][wave] = wide;
         if (g == 0) ae[half][share_b / EB][share_t][c] = e;
 #pragma unroll
         for (int p = 0; p < PIECES; ++p) {
@@ -416,36 +418,7 @@ __global__ __launch_bounds__(256, 3) void gemm_f16x2_stream_kernel(GemmArgs a) {
     __syncthreads();
     int half = 0;
     for (int d = 0; d < n; d += SF_BLOCKS, half ^= 1) {
-        const int wide = wide_share[half][0] | wide_share[half][1] | wide_share[half][2] | wide_share[half][3];
         fetch_a(d + SF_BLOCKS);
-        if (w_wide || __builtin_amdgcn_readlane(wide, 0)) {
-#pragma unroll
-            for (int j = 0; j < SF_BLOCKS; ++j) {
-                if (d + j >= n) break;
-                // instruction (i, e): element e of this lane's piece i of the block, of both operands
-                v4f ax[MT][2];
-#pragma unroll
-                for (int t = 0; t < MT; ++t) {
-                    const float *row = a.A + (size_t)min(t * 16 + c, M - 1) * K + (size_t)(b0 + d + j) * 32;
-#pragma unroll
-                    for (int i = 0; i < 2; ++i) ax[t][i] = *(const v4f *)(row + (WBF16 ? 8 * g + 4 * i : 16 * i + 4 * g));
-                }
-                float w[8];
-                if (WBF16) {
-                    const unsigned src[4] = {vw[j][0].x, vw[j][0].y, vw[j][0].z, vw[j][0].w};
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) w[e] = __uint_as_float(e & 1 ? src[e >> 1] & 0xffff0000u : src[e >> 1] << 16);
-                } else {
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) w[e] = __uint_as_float(vw[j][WP == 2 ? e >> 2 : 0][e & 3]);
-                }
-                fetch_w(j, d + j + SF_BLOCKS);
-#pragma unroll
-                for (int e = 0; e < 8; ++e)
-#pragma unroll
-                    for (int t = 0; t < MT; ++t) sum[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(ax[t][e >> 2][e & 3], w[e], sum[t], 0, 0, 0);
-            }
-        } else
 #pragma unroll
         for (int e0 = 0; e0 < SF_BLOCKS; e0 += EB) {
             v4f acc[MT];
@@ -495,6 +468,42 @@ __global__ __launch_bounds__(256, 3) void gemm_f16x2_stream_kernel(GemmArgs a) {
         }
         if (d + SF_BLOCKS < n) stage_a(half ^ 1);
         __syncthreads();
+    }
+    if (lane == 0) wide_any[wave] = wide;
+    __syncthreads();
+    if (wide_any[0] | wide_any[1] | wide_any[2] | wide_any[3]) {
+#pragma unroll
+        for (int t = 0; t < MT; ++t) sum[t] = v4f{0.f, 0.f, 0.f, 0.f};
+        const float *arow[MT];
+#pragma unroll
+        for (int t = 0; t < MT; ++t) arow[t] = a.A + (size_t)min(t * 16 + c, M - 1) * K + (size_t)b0 * 32;
+#pragma unroll 1
+        for (int d = 0; d < n; ++d) {
+            // instruction (i, e): element e of this lane's piece i of the block, of both operands
+            v4f ax[MT][2];
+            float w[8];
+#pragma unroll
+            for (int t = 0; t < MT; ++t)
+#pragma unroll
+                for (int i = 0; i < 2; ++i) ax[t][i] = *(const v4f *)(arow[t] + d * 32 + (WBF16 ? 8 * g + 4 * i : 16 * i + 4 * g));
+#pragma unroll
+            for (int i = 0; i < WP; ++i) {
+                const v4u b = *(const v4u *)(wp + (size_t)d * (WBF16 ? 64 : 128) + i * 64);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    if (WBF16) {
+                        w[2 * e] = __uint_as_float(b[e] << 16);
+                        w[2 * e + 1] = __uint_as_float(b[e] & 0xffff0000u);
+                    } else {
+                        w[4 * i + e] = __uint_as_float(b[e]);
+                    }
+                }
+            }
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+#pragma unroll
+                for (int t = 0; t < MT; ++t) sum[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(ax[t][e >> 2][e & 3], w[e], sum[t], 0, 0, 0);
+        }
     }
     float *part = PARTIAL ? a.part + (size_t)blockIdx.z * M * N : nullptr;
 #pragma unroll
