@@ -229,7 +229,10 @@ int lumen_attn_decode_static_f32(lumen_kv_cache *cache, lumen_rope *rope, const 
 /* SelfAttention::forward prefill core, S > 1, self_attention.rs:308-419 with
  * gqa_attention_no_repeat_bshd_view :519-641 and softmax_inplace_view :643-678:
  * q [B, S, H, D], k/v [B, S, H_kv, D] un-rotated; appends S positions to the
- * cache (which may already hold past_len > 0), out [B, S, H, D]. */
+ * cache (which may already hold past_len > 0), out [B, S, H, D].
+ * Many positions of head_dim 64 and 128 are multiplied as pairs of f16 values, 22 to 23 bits at one exponent per query row and per tile of 64
+ * (head_dim 128: 32) keys, and values.  A value 2^18 below the largest of its row or tile keeps an error of 2^-40 of that largest while
+ * fewer than 16 of the tile are that small (of a query row: at most one in 32); with more of them the f32 values are multiplied by f32 instructions. */
 int lumen_attn_prefill_f32(lumen_kv_cache *cache, lumen_rope *rope, const float *q_dev,
                            const float *k_dev, const float *v_dev, float *out_dev,
                            int s, int h, float scale, int causal);
@@ -274,7 +277,9 @@ int lumen_safetensors_find(const char *path, const char *name, int *dtype_out, i
 /* LlamaModel::forward, llama.rs:181-206: ids_host [S] as f32 (main.rs:143-152);
  * S == 1 takes the decode path, S > 1 prefill (appending to the live cache).
  * logits_host receives [S, V] when all_rows != 0 (what the reference computes)
- * or just the last position [V] (what its caller keeps, main.rs:155-163). */
+ * or just the last position [V] (what its caller keeps, main.rs:155-163).
+ * The products of S > 2 run on pairs likewise, one exponent per row of either operand; a row of which more than one value in 32 is 2^18 below its
+ * largest (bf16-stored weights: 2^31; up to 32 positions, a row's share of 32 or 64 values: one in 16) is multiplied by f32 instructions. */
 int lumen_llama_forward(lumen_llama *model, const float *ids_host, int s, float *logits_host, int all_rows);
 /* the generation loop of src/main.rs:340-378 with greedy picks: feeds
  * first_id, then each argmax, for n steps, without leaving the GPU.
