@@ -420,6 +420,8 @@ struct AttnPrefillArgs {
 int launch_attn_prefill(lumen_ctx *ctx, const AttnPrefillArgs &a);
 // the scores / softmax / context part on the matrix cores (q_rot and the cache rows already written)
 bool attn_prefill_mfma_supported(const AttnPrefillArgs &a);
+// does it leave its rows split without a pass of their own, where out_exp is given?
+bool attn_prefill_splits_rows(const lumen_ctx *ctx, const AttnPrefillArgs &a);
 // floats of AttnPrefillArgs::ws for any call of up to s positions over a cache of max_seq rows
 size_t attn_prefill_workspace(const lumen_ctx *ctx, int b, int s, int hq, int hkv, int d, int max_seq);
 int launch_attn_prefill_mfma(lumen_ctx *ctx, const AttnPrefillArgs &a);

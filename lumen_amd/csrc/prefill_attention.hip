@@ -490,21 +490,33 @@ size_t attn_prefill_workspace(const lumen_ctx *ctx, int b, int s, int hq, int hk
     return 2 * (size_t)b * hkv * ((max_seq + trip - 1) / trip) + rows * (d + 2);
 }
 
+// Query heads of a KV group that share a workgroup, the grid of blocks of queries, and how the keys are cut.
+struct FaPlan {
+    int nrep, parts, key_chunk;
+    dim3 grid;
+};
+static FaPlan fa_plan(int num_cus, const AttnPrefillArgs &a) {
+    FaPlan p = {a.hq / a.hkv, 1, 0, dim3(1)};
+    if (!(p.nrep == 1 || p.nrep == 2 || p.nrep == 4 || p.nrep == 8)) p.nrep = 1;  // any other group size: one query head per grid row
+    const int L = a.past_len + a.s, trip = FA_KEYS * (a.d == 64 ? 2 : 1);
+    p.grid = dim3((a.s + FA_ROWS / p.nrep - 1) / (FA_ROWS / p.nrep), a.hq / p.nrep, a.b);
+    p.parts = fa_key_parts(num_cus, (int)(p.grid.x * p.grid.y * p.grid.z), L);
+    if (p.parts > 1) {
+        p.key_chunk = ((L + p.parts - 1) / p.parts + trip - 1) / trip * trip;
+        p.parts = (L + p.key_chunk - 1) / p.key_chunk;
+    }
+    return p;
+}
+static bool merge_splits_rows(const AttnPrefillArgs &a, const FaPlan &p) { return p.parts > 1 && a.hq * a.d / 4 <= 1024; }
+
 template <int D>
 static int launch_fa_d(lumen_ctx *ctx, const AttnPrefillArgs &a_in) {
     AttnPrefillArgs a = a_in;
-    int nrep = a.hq / a.hkv;
-    if (!(nrep == 1 || nrep == 2 || nrep == 4 || nrep == 8)) {  // any other group size: one query head per grid row, its KV head = head / n_rep
-        a.kv_div = nrep;
-        nrep = 1;
-    }
-    const int L = a.past_len + a.s, trip = FA_KEYS * (D == 64 ? 2 : 1);
-    dim3 grid((a.s + FA_ROWS / nrep - 1) / (FA_ROWS / nrep), a.hq / nrep, a.b);
-    int parts = fa_key_parts(ctx->num_cus, (int)(grid.x * grid.y * grid.z), L);
-    if (parts > 1) {
-        a.key_chunk = ((L + parts - 1) / parts + trip - 1) / trip * trip;
-        parts = (L + a.key_chunk - 1) / a.key_chunk;
-    }
+    const FaPlan plan = fa_plan(ctx->num_cus, a);
+    const int nrep = plan.nrep, parts = plan.parts, L = a.past_len + a.s, trip = FA_KEYS * (D == 64 ? 2 : 1);
+    if (nrep != a.hq / a.hkv) a.kv_div = a.hq / a.hkv;  // KV head of a grid row = head / n_rep
+    dim3 grid = plan.grid;
+    a.key_chunk = plan.key_chunk;
     const int tile = trip, tiles = (L + tile - 1) / tile;
     const size_t rows = parts > 1 ? (size_t)a.b * a.s * a.hq * parts : 0, codes = 2 * (size_t)a.b * a.hkv * tiles;
     const size_t need = codes + rows * (D + 2);
@@ -531,7 +543,7 @@ static int launch_fa_d(lumen_ctx *ctx, const AttnPrefillArgs &a_in) {
     const int pieces = a.hq * D / 4;  // of a position's row
     bool split_done = false;
     if (parts > 1) {
-        if (a.out_exp && pieces <= 1024) {
+        if (a.out_exp && merge_splits_rows(a, plan)) {
             hipLaunchKernelGGL(merge_parts_kernel<true>, dim3(a.s, 1, a.b), dim3((pieces + 63) / 64 * 64), 0, ctx->stream, a, parts);
             split_done = true;
         } else {
@@ -550,6 +562,10 @@ static int launch_fa_d(lumen_ctx *ctx, const AttnPrefillArgs &a_in) {
 bool attn_prefill_mfma_supported(const AttnPrefillArgs &a) {
     const long L = (long)a.past_len + a.s;
     return (a.d == 64 || a.d == 128) && (a.s >= 96 || L * a.d >= 64000 || (long)a.b * a.s * a.hq * (a.past_len + a.s / 2) * a.d >= 44000000);
+}
+
+bool attn_prefill_splits_rows(const lumen_ctx *ctx, const AttnPrefillArgs &a) {
+    return attn_prefill_mfma_supported(a) && merge_splits_rows(a, fa_plan(ctx->num_cus, a));
 }
 
 int launch_attn_prefill_mfma(lumen_ctx *ctx, const AttnPrefillArgs &a) {
