@@ -555,13 +555,15 @@ static int launch_fa_d(lumen_ctx *ctx, const AttnPrefillArgs &a_in) {
     return LUMEN_OK;
 }
 
-// Against the row loop (one workgroup per position and head or two: its walk over the keys is a chain, and every position repeats it): from 96
-// positions on, where the cache is long, and where positions times keys are many.  Measured, row loop / this, us: 32 heads of 64, 4 KV heads,
-// 64 positions behind 301: 18.5 / 18.6, 32 behind 600: 18.8 / 18.0, 2 behind 1000: 18.4 / 17.0, 64 behind 2900: 102 / 28; 32 heads of 128, 32
-// KV heads, 64 behind 301: 40 / 25, 2 behind 600: 35 / 23, 2 behind 301: 14 / 20.
+// Against the row loop (one workgroup per position and head or two: its walk over the keys is a chain, and every position repeats it): where the
+// cache is long, and where positions times keys are many.  Measured, row loop / this with its pass over the keys, us: 32 heads of 64, 4 KV heads,
+// 96 first positions 10.3 / 16.4, 160 16.7 / 20.6, 192 20.9 / 21.2, 207 22.9 / 22.1, 64 behind 301 18.5 / 18.6, 32 behind 600 18.8 / 18.0, 2 behind 1000
+// 18.4 / 17.0, 64 behind 2900 102 / 28; 16 heads of 64, 8 KV heads, 192 14.0 / 19.9, 256 21.1 / 20.1; 16 of 128, 8 KV heads, 207 25.7 / 27.7.  A KV
+// head for every head (no rows shared): 32 of 64 160 21.2 / 22.8, 192 26.2 / 23.4, 71 of 64 96 21.7 / 19.8, 128 29.4 / 22.0; 32 of 128 96 19.6 / 22.4,
+// 128 26.8 / 27.1, 64 behind 301 40 / 25, 2 behind 600 35 / 23, 2 behind 301 14 / 20.
 bool attn_prefill_mfma_supported(const AttnPrefillArgs &a) {
-    const long L = (long)a.past_len + a.s;
-    return (a.d == 64 || a.d == 128) && (a.s >= 96 || L * a.d >= 64000 || (long)a.b * a.s * a.hq * (a.past_len + a.s / 2) * a.d >= 44000000);
+    const long L = (long)a.past_len + a.s, work = (long)a.b * a.s * a.hq * (a.past_len + a.s / 2) * a.d;
+    return (a.d == 64 || a.d == 128) && (L * a.d >= 64000 || work >= (a.hq == a.hkv ? 28000000 : 40000000));
 }
 
 bool attn_prefill_splits_rows(const lumen_ctx *ctx, const AttnPrefillArgs &a) {

@@ -487,15 +487,23 @@ static void case_shapes(lumen_ctx *ctx) {
 // A recorded prompt attention of one cache, replayed after another cache's call has needed more scratch than it had.
 static void case_caches(lumen_ctx *ctx) {
     printf("caches: a recorded prompt attention beside a larger one on another cache\n");
-    const int h = 2, d = 64, s = 97;
+    const int h = 2, d = 128, s = 33, past = 512 - s;  // (rows of zeros before: a cache long enough for the matrix-core form)
     lumen_rope *rope = nullptr;
     OK(lumen_rope_create(ctx, d, 1024, 10000.f, &rope));
     std::vector<float> cs((size_t)1024 * d), sn((size_t)1024 * d);
     lo_rope_table(cs.data(), sn.data(), d, 1024, 10000.f);
     lumen_kv_cache *small = nullptr, *large = nullptr;
-    OK(lumen_kv_cache_create(ctx, 1, h, 128, d, &small));
+    OK(lumen_kv_cache_create(ctx, 1, h, 512, d, &small));
     OK(lumen_kv_cache_create(ctx, 1, h, 1024, d, &large));
-    lo_kv_cache *co = lo_kv_cache_new(1, h, 128, d);
+    lo_kv_cache *co = lo_kv_cache_new(1, h, 512, d);
+    co->len = past;
+    const std::vector<float> zeros((size_t)h * 1024 * d);
+    for (lumen_kv_cache *c : {small, large}) {
+        float *k, *v;
+        OK(lumen_kv_cache_ptrs(c, &k, &v));
+        for (float *p : {k, v}) OK(lumen_upload(ctx, p, zeros.data(), (size_t)h * (c == small ? 512 : 1024) * d * 4));
+        OK(lumen_kv_cache_set_len(c, c == small ? past : 1024 - s));
+    }
     const size_t n = (size_t)s * h * d;
     std::vector<float> x[3], got(n), ref(n);
     void *dx[3], *dout, *dother;
@@ -510,13 +518,12 @@ static void case_caches(lumen_ctx *ctx) {
         OK(lumen_attn_prefill_f32(c, rope, (const float *)dx[0], (const float *)dx[1], (const float *)dx[2], (float *)out, s, h, 0.125f, 1));
     };
     prompt(small, dout);  // (the call that allocates)
-    OK(lumen_kv_cache_set_len(small, 0));
+    OK(lumen_kv_cache_set_len(small, past));
     hipGraph_t graph;
     hipGraphExec_t exec;
     if (hipStreamBeginCapture(nullptr, hipStreamCaptureModeThreadLocal) != hipSuccess) exit(2);
     prompt(small, dout);
     if (hipStreamEndCapture(nullptr, &graph) != hipSuccess || hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0) != hipSuccess) exit(2);
-    OK(lumen_kv_cache_set_len(large, 1024 - s));
     prompt(large, dother);
     if (hipGraphLaunch(exec, nullptr) != hipSuccess) exit(2);
     OK(lumen_download(ctx, got.data(), dout, n * 4));

@@ -25,9 +25,10 @@ def attention_rows(d, h, h_kv, past, s, change, causal=True, batch=1):
     q = rng.normal(0, 1, (batch, n, h, d)).astype(np.float32)
     k, v = (rng.normal(0, 1, (batch, n, h_kv, d)).astype(np.float32) for _ in range(2))
     change(q, k, v)
-    rope, scale = RotaryEmbedding(d, 512, 10000.0), d ** -0.5
-    cos, sin = lo.rope_table(d, 512, 10000.0)
-    gpu, ora = KVCacheInner(batch, h_kv, 512, d), lo.KVCache(batch, h_kv, 512, d)
+    size = 512 if n <= 512 else 1152
+    rope, scale = RotaryEmbedding(d, size, 10000.0), d ** -0.5
+    cos, sin = lo.rope_table(d, size, 10000.0)
+    gpu, ora = KVCacheInner(batch, h_kv, size, d), lo.KVCache(batch, h_kv, size, d)
     for at, m in ((0, past), (past, s)):
         if not m:
             continue
@@ -52,7 +53,8 @@ def later(what, first, e):
 
 @pytest.mark.parametrize("e", [12, 16, 18, 20, 24, 30, 40, 100])
 @pytest.mark.parametrize("what", ["k", "v"])
-@pytest.mark.parametrize("d,h,h_kv,past,s", [(64, 4, 1, 0, 96), (128, 2, 2, 0, 97), (64, 8, 1, 301, 99)])
+@pytest.mark.parametrize("d,h,h_kv,past,s", [(64, 4, 1, 0, 96), (128, 2, 2, 0, 97), (64, 8, 1, 301, 99),
+                                              (64, 4, 1, 905, 96), (128, 2, 2, 420, 97), (64, 8, 1, 901, 99)])  # (on pairs: long caches)
 def test_attention_rows_before_a_large_key_or_value(d, h, h_kv, past, s, what, e):
     """The last position only, and all from one inside a tile on."""
     for first in (past + s - 1, past + 37):
@@ -61,7 +63,7 @@ def test_attention_rows_before_a_large_key_or_value(d, h, h_kv, past, s, what, e
 
 
 @pytest.mark.parametrize("e", [-40, -24, -18, 24, 40])
-@pytest.mark.parametrize("d,h,h_kv,past,s", [(64, 4, 2, 0, 130), (128, 4, 1, 400, 20)])
+@pytest.mark.parametrize("d,h,h_kv,past,s", [(64, 4, 2, 0, 130), (128, 4, 1, 400, 20), (64, 4, 2, 871, 130), (128, 4, 1, 490, 20)])
 def test_attention_channels_of_other_magnitudes(d, h, h_kv, past, s, e):
     """Half of the value channels, each held to its own largest output; a rotated pair of channels of the queries, to which the keys are zero;
     one head's values beside the others'."""
@@ -84,7 +86,9 @@ def test_attention_channels_of_other_magnitudes(d, h, h_kv, past, s, e):
     assert row_error(*attention_rows(d, h, h_kv, past, s, head)) <= 2e-5
 
 
-@pytest.mark.parametrize("d,h,h_kv,past,s,batch", [(64, 4, 2, 0, 96, 2), (128, 3, 1, 300, 5, 1), (64, 2, 2, 130, 140, 1), (64, 8, 2, 448, 3, 2)])
+@pytest.mark.parametrize("d,h,h_kv,past,s,batch", [(64, 4, 2, 0, 96, 2), (128, 3, 1, 300, 5, 1), (64, 2, 2, 130, 140, 1), (64, 8, 2, 448, 3, 2),
+                                                    (64, 4, 2, 904, 96, 2), (128, 3, 1, 500, 5, 1), (64, 8, 2, 1000, 3, 2),  # on pairs, keys in parts
+                                                    (64, 32, 4, 0, 290, 4), (128, 32, 32, 0, 258, 4)])  # and in one
 def test_attention_without_a_mask(d, h, h_kv, past, s, batch):
     """All keys for every position, keys in parts and in one, also with tiles that lie far apart in magnitude."""
     for change in (lambda q, k, v: None, later("v", past + s - 20, -30), later("v", past + s - 20, 30)):

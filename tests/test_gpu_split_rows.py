@@ -123,7 +123,8 @@ def test_a_token_that_is_not_finite_stays_in_its_row():
 
 
 @pytest.mark.parametrize("d,h,h_kv,s,past", [(64, 8, 1, 96, 0), (64, 6, 2, 129, 70), (128, 4, 4, 97, 0), (128, 4, 2, 200, 33), (64, 2, 2, 127, 1),
-                                                (128, 4, 2, 40, 461), (64, 8, 1, 97, 300), (128, 3, 1, 2, 510)])  # keys in parts
+                                                (128, 4, 2, 40, 461), (64, 8, 1, 97, 300), (128, 3, 1, 2, 510),  # keys in parts
+                                                (128, 4, 4, 97, 403), (128, 4, 2, 200, 300), (128, 6, 2, 129, 371), (128, 8, 1, 64, 440)])
 @pytest.mark.parametrize("q_exp,k_exp,v_exp", [(0, 0, 0), (-90, 88, -100), (60, -61, 90)])
 def test_prompt_attention_over_magnitudes(d, h, h_kv, s, past, q_exp, k_exp, v_exp):
     """Queries, keys and values far from 1, and keys and values spread over 2^8 within a head (2e-5 of the largest output, the suite's bound for
