@@ -278,7 +278,7 @@ int lumen_safetensors_find(const char *path, const char *name, int *dtype_out, i
  * S == 1 takes the decode path, S > 1 prefill (appending to the live cache).
  * logits_host receives [S, V] when all_rows != 0 (what the reference computes)
  * or just the last position [V] (what its caller keeps, main.rs:155-163).
- * The products of S > 2 run on pairs likewise, one exponent per row of either operand; a row of which more than one value in 32 is 2^18 below its
+ * The products of S > 2 may run on pairs likewise, one exponent per row of either operand; a row of which more than one value in 32 is 2^18 below its
  * largest (bf16-stored weights: 2^31; up to 32 positions, a row's share of 32 or 64 values: one in 16) is multiplied by f32 instructions. */
 int lumen_llama_forward(lumen_llama *model, const float *ids_host, int s, float *logits_host, int all_rows);
 /* the generation loop of src/main.rs:340-378 with greedy picks: feeds

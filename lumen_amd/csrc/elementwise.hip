@@ -764,7 +764,7 @@ extern "C" int lumen_rope_1token_copy_f32(lumen_rope *r, const float *src, float
 // A call of one token is bound by its launches and what lies between them.  A copy of a few bytes costs the host 15-20 us and a
 // synchronisation after it; a kernel that carries the word in its arguments, or writes results into pinned memory, costs a launch.
 // Copies before, these after, ms: TinyLlama shape, prompt of 2 tokens 1.48 -> 1.37, of 9 tokens 1.63 -> 1.52, 16 decoded tokens 14.68 -> 14.53;
-// Qwen3 shape, 16 tokens 12.00 -> 11.86; Pinavik 1024 wide, 20 tokens 1.55 -> 1.47.
+// Qwen3 shape, 16 tokens 11.94 -> 11.89; Pinavik 1024 wide, 20 tokens 1.55 -> 1.47.
 __global__ void put_word_kernel(int *dst, int v) { *dst = v; }
 int launch_put_word(lumen_ctx *ctx, int *dst, int v) {
     hipLaunchKernelGGL(put_word_kernel, dim3(1), dim3(1), 0, ctx->stream, dst, v);

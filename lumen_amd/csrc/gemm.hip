@@ -1004,7 +1004,7 @@ static bool gemm_stream_applies(const GemmArgs &a) {
 // 17 to 32 where W has 5 Mi of them (at 23 rows: 2560 x 2048 12.1 -> 10.3 us, but 2048 x 2048 10.8 -> 11.1 and 1024 x 3072 10.6 -> 14).  Up to 16 rows of
 // f32 weights the f32 instruction needs only one row tile and no splitting (11264 x 2048: 22-23 us against 27-29 on pairs); from 33 rows on the tile
 // kernels win (48 rows of bf16 weights, 12288 x 4096: 40 us there, 49 here).  Prompt passes before and after, ms: Llama-2-7B shape, 8 layers, bf16, 3
-// rows 1.51 -> 1.12, 17 1.55 -> 1.33, 32 1.63 -> 1.48; TinyLlama 17 rows 2.29 -> 2.01, 32 2.30 -> 2.11; Pinavik 2048 wide, bf16, 20 rows 2.22 -> 1.84.
+// rows 1.51 -> 1.12, 17 1.55 -> 1.33, 32 1.63 -> 1.48; TinyLlama 17 rows 2.24 -> 1.89, 32 2.26 -> 2.05; Pinavik 2048 wide, bf16, 20 rows 2.22 -> 1.84.
 static bool stream_pairs_shape(int M, int N, int K, int w_bf16) {
     return M > (w_bf16 ? GEMM_SKINNY_MAX_M : 16) && M <= GEMM_STREAM_MAX_M && K > 0 && K % 64 == 0 && (w_bf16 || (long)N * K >= 5L << 20);
 }
